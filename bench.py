@@ -152,8 +152,10 @@ def roofline_for(key, kernel, ms, b_alg, step_ms=None, n_ops=2):
 # HIP-event-timed launch of that key (a forward is gather + chunk reduction).
 COUNTER_KEYS = {
     "fanarc": {"fanarc_b16:k_pixels<16,0>": ["k_pixels<16, 0, "],
+               "fanarc_b16:k_pixels_walk<16,0>": ["k_pixels_walk<16, 0, "],
                "fanarc_b16:k_bins_split<16,0>": ["k_bins_split<16, 0>", "k_bins_reduce<0>"],
                "fanarc_plain:k_pixels<1,0>": ["k_pixels<1, 0, "],
+               "fanarc_plain:k_pixels_walk<1,0>": ["k_pixels_walk<1, 0, "],
                "fanarc_plain:k_bins_split<1,0>": ["k_bins_split<1, 0>", "k_bins_reduce<0>"],
                "fanarc_plain:k_pixels_prefix<0>": ["k_prefix_sino<true>", "k_prefix_ranges",
                                                    "k_pixels_prefix<0>", "k_sum_chunks"],
@@ -386,9 +388,8 @@ def uneven_c2(torch, dev, steps, warmup, check, tune_grid=True, cpu=False, varia
            "forward_ms": fp_ms / max(fp_n, 1), "adjoint_ms": bp_ms / max(bp_n, 1)}
     var = tune.get("variant", rt.ADJ_QUAD)
     out["forward_kernel"] = "running sums" if var & rt.FWD_PREFIX else "pixel walk"
-    adj_name = {rt.ADJ_QUAD: "k_batch_quads", rt.ADJ_BLOCK_WINDOW: "k_batch_quads_window",
-                rt.ADJ_BLOCK_PREFIX: "k_batch_quads_prefix",
-                rt.ADJ_TILE16: "k_batch_tile"}.get(var & ~rt.FWD_PREFIX, "k_batch_pixels")
+    adj_name = ("k_batch_quads_prefix" if var & ~rt.FWD_PREFIX == rt.ADJ_BLOCK_PREFIX
+                else "k_batch_walk")
     fwd_name = "k_batch_bins_prefix" if var & rt.FWD_PREFIX else "k_batch_bins"
     dom = ((fwd_name, out["forward_ms"]) if out["forward_ms"] >= out["adjoint_ms"]
            else (adj_name, out["adjoint_ms"]))
@@ -879,9 +880,7 @@ def main():
     rt.profile_enable(False)
     fp_ms, bp_ms = fp_ms / max(fp_n, 1), bp_ms / max(bp_n, 1)
     b_alg = 4.0 * V * (N * N + D) * B  # bytes per operator launch over the batch
-    # the adjoint kernel of the chosen variant
-    adj = {rt.ADJ_QUAD: "k_pixels_quad", rt.ADJ_TILE16: "k_pixels_tile",
-           rt.ADJ_TILE8: "k_pixels_tile"}.get(BP.variant, "k_pixels")
+    adj = "k_pixels_walk"
     kernels = {
         "k_bins_split + k_bins_reduce (A, image->sino)":
             {"ms": fp_ms, "effective_GBps": b_alg / (fp_ms * 1e-3) / 1e9},

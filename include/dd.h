@@ -93,10 +93,11 @@ dd_status dd2d_run(int scan, int op, const dd_geom2d* g, const float* input,
  * device memory (code under HIP graph capture, tight serving loops, hosts
  * that forbid allocation).  No counterpart in the reference.  Scratch comes
  * from a fixed buffer inside the library, one per device, resident until the
- * process ends; the call allocates and frees nothing.  A problem whose
- * dd2d_workspace_size() exceeds DD_NOALLOC_SCRATCH_BYTES is rejected with
- * DD_TOO_LARGE (a 512x512 fan-arc slice with 720 views and 736 bins needs
- * 27 MB at batch 1).  Results equal dd2d_run's bit for bit.  Every call on
+ * process ends; the call allocates and frees nothing.  Where the scratch does
+ * not hold the partial images or range table that dd2d_workspace_size()
+ * includes, the op runs without them (slower, the same bits); a problem that
+ * does not fit even so is rejected with DD_TOO_LARGE (a 512x512 fan-arc slice
+ * with 720 views and 736 bins needs 27 MB at batch 1).  Results equal dd2d_run's bit for bit.  Every call on
  * one device shares that device's buffer: calls that overlap on one device
  * (two streams, two host threads) race and must be ordered by the caller. */
 #define DD_NOALLOC_SCRATCH_BYTES (64u << 20)
@@ -141,28 +142,25 @@ dd_status dd2d_sysmatrix_fill(int scan, const dd_geom2d* g,
 size_t dd2d_geometry_size(int scan, const dd_geom2d* g, int views);
 dd_status dd2d_geometry(int scan, const dd_geom2d* g, const float* angles,
                         int views, void* geo, size_t geo_bytes, void* stream);
-/* Kernel variants of the sinogram -> image gathers (all exact and equal):
- * each pixel finds its bins on its own; a 16x16 / 8x8 pixel tile stages its
- * lines' bin-edge positions per view in LDS; or one thread walks the bins of
- * a 2x2 pixel block once for its two lines of two pixels. */
+/* Kernel variants of the sinogram -> image gathers.  The first five name the
+ * walk over each pixel's bins; they are one kernel (a wavefront stages each
+ * view's bins for its pixel tile in LDS; one thread per pixel where the bins
+ * are too fine for that) and give equal results, in every batch size. */
 #define DD_ADJ_PER_PIXEL 0
 #define DD_ADJ_TILE16 1
 #define DD_ADJ_TILE8 2
 #define DD_ADJ_QUAD 3
-/* Uneven batches only: the 4 x 4 pixel blocks, each line's bins read as one
- * window of loads instead of one bin at a time. */
 #define DD_ADJ_BLOCK_WINDOW 4
-/* The 4 x 4 pixel blocks through per-view running integrals of the sinogram
+/* 4 x 4 pixel blocks through per-view running integrals of the sinogram
  * along the detector (FP64 knots at the bin edges): each pixel's value from
  * a view is the difference of the running integral at its two edges, found
  * by one merge walk per 4-pixel run.  PROJ_T and BPROJ only (BPROJ_W, whose
  * weight varies per pixel, keeps a walk).  In uneven batches; and in
  * dd2d_run / planned runs at instance tile 1, where the views are split over
  * workgroups (partial images added in order): a 512^2 x 720-view slice's
- * ProjTrans 0.3 ms instead of the walk's 1.06 ms.  Same operator, different
- * rounding: not bit-equal to the other variants (5e-8 from FP64 against the
- * walks' 2-3e-7), so the automatic choice keeps the walks and this variant
- * is selected explicitly or by the autotuner. */
+ * ProjTrans 0.31 ms, the walk 0.37 ms.  Same operator, different rounding:
+ * not bit-equal to the walk, so the automatic choice keeps the walk and this
+ * variant is selected explicitly or by the autotuner. */
 #define DD_ADJ_BLOCK_PREFIX 5
 /* Flag OR-ed into a variant: the image -> sinogram ops PROJ and BPROJ_T
  * integrate each bin over each line as a difference of the line's running
@@ -204,8 +202,9 @@ typedef struct {
  *   fwd_waves : image -> sinogram: 63-bin wavefronts per workgroup (1, 2, 4);
  *   fwd_views : image -> sinogram: views per workgroup, one after the other
  *               (1 - 8); the lines are one of the 8 per-XCD line chunks;
- *   pix_width : per-pixel sinogram -> image variant: pixels per workgroup
- *               row (16, 32 or 64; 256 threads, so 16, 8 or 4 rows).
+ *   pix_width : per-pixel sinogram -> image gather (bins too fine for the
+ *               staged walk): pixels per workgroup row (16, 32 or 64; 256
+ *               threads, so 16, 8 or 4 rows).
  * The shape never changes a result bit; it is what the autotuner sweeps. */
 typedef struct {
   int fwd_waves;
@@ -255,10 +254,9 @@ size_t dd2d_batch_device_bytes(const dd2d_batch* b);
 /* Grid size in workgroups, each striding over the work items (0 = one
  * workgroup per work item). */
 void dd2d_batch_set_grid(dd2d_batch* b, int workgroups);
-/* Sinogram -> image kernel of the batch: DD_ADJ_PER_PIXEL, DD_ADJ_TILE16,
- * DD_ADJ_QUAD (in a batch: one thread per 4x4 pixel block, four lines of
- * four pixels; the default), DD_ADJ_BLOCK_WINDOW or DD_ADJ_BLOCK_PREFIX,
- * optionally OR-ed with DD_FWD_PREFIX for the image -> sinogram ops. */
+/* Sinogram -> image kernel of the batch: a walk variant (the default) or
+ * DD_ADJ_BLOCK_PREFIX, optionally OR-ed with DD_FWD_PREFIX for the image ->
+ * sinogram ops. */
 void dd2d_batch_set_variant(dd2d_batch* b, int variant);
 dd_status dd2d_batch_setup(dd2d_batch* b, void* device_mem, size_t bytes,
                            void* stream);
@@ -280,12 +278,9 @@ int dd_profile_read(int kernel_class, double* total_ms, long long* launches);
 
 /* Default sinogram -> image kernel variant of dd2d_run and of planned runs
  * given variant -1 (DD_ADJ_PER_PIXEL .. DD_ADJ_QUAD or DD_ADJ_BLOCK_PREFIX,
- * optionally | DD_FWD_PREFIX; -1 = automatic: DD_ADJ_QUAD for up to 4
- * instances per launch when that still gives 4 workgroups per compute unit,
- * DD_ADJ_PER_PIXEL otherwise, walks in both directions).  The running sums
- * apply at instance tile 1 only; above it DD_ADJ_BLOCK_PREFIX falls back to
- * the automatic choice and DD_FWD_PREFIX is ignored.  dd2d_workspace_size
- * follows the current setting. */
+ * optionally | DD_FWD_PREFIX; -1 = automatic: walks in both directions).  The
+ * running sums apply at instance tile 1 only; above it they are ignored.
+ * dd2d_workspace_size follows the current setting. */
 void dd2d_set_adjoint_variant(int variant);
 
 /* Instance tile used per launch (1, 2, 4, 8 or 16 instances share one

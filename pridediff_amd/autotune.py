@@ -2,10 +2,10 @@
 
 Sweeps the launch parameters of a planned operator on the problem it will
 run — the instance tile (how many instances share one geometry evaluation,
-1-16), the sinogram -> image kernel variant (per pixel, 16x16 or 8x8 tiles
-with LDS edge positions, or one thread per 2x2 pixels) and the workgroup
-tiles of both gathers (forward: 63-bin waves x views per workgroup over one
-per-XCD line chunk; per-pixel adjoint: 16x16, 32x8 or 64x4 pixels) of a
+1-16), the sinogram -> image kernel variant (the walk or, at tile 1, the
+running sums) and the workgroup tiles of the gathers (forward: 63-bin waves x
+views per workgroup over one per-XCD line chunk; per-pixel adjoint, where the
+bins are too fine for the staged walk: 16x16, 32x8 or 64x4 pixels) of a
 uniform batch; the grid size and kernel variant of an uneven batch —
 times one forward projection plus one adjoint per candidate with HIP events,
 keeps the fastest, and remembers it in a JSON cache keyed by the device and
@@ -29,7 +29,7 @@ CACHE = os.environ.get("PRIDEDIFF_AMD_TUNE_CACHE",
                        os.path.join(os.path.expanduser("~"), ".cache", "pridediff_amd", "autotune.json"))
 
 
-SWEEP_VERSION = 9  # bumped when the set of swept parameters changes
+SWEEP_VERSION = 10  # bumped when the set of swept parameters changes
 
 _LIB_DIGEST = None
 
@@ -99,12 +99,12 @@ def tune_uniform(projector, angles: torch.Tensor, batch: int, tiles=(1, 2, 4, 8,
     first the instance tile x adjoint kernel variant, then, for the winner,
     the workgroup tile of each gather — forward (63-bin waves x views per
     workgroup; its lines are one of the 8 per-XCD chunks) and per-pixel
-    adjoint (pixels per workgroup row).  The walk variants all give the same
-    bits; ``running_sums`` also sweeps, at tile 1, the running-sum adjoint
-    alone and both directions, which round differently (within 1e-6 of the
-    walks)."""
+    adjoint (pixels per workgroup row).  The walks give the same bits at
+    every tile; ``running_sums`` also sweeps, at tile 1, the running-sum
+    adjoint alone and both directions, which round differently (within 1e-6
+    of the walks)."""
     if variants is None:
-        variants = (rt.ADJ_PER_PIXEL, rt.ADJ_TILE16, rt.ADJ_TILE8, rt.ADJ_QUAD)
+        variants = (rt.ADJ_PER_PIXEL,)  # the walk variants are one kernel
     opts = [round(float(v), 6) for v in projector.host_options().tolist()]
     key = (f"{_device_key()}|uniform|{projector.scan_type}|{opts}|V={angles.numel()}|B={batch}"
            f"|rs{int(running_sums)}")
@@ -175,7 +175,7 @@ def tune_uneven(batch: UnevenBatch2d, grids_per_cu=(0, 2, 8, 32, 128, 512), vari
     round differently from the walks (same operator, errors of the same
     size against FP64)."""
     if variants is None:
-        variants = (rt.ADJ_PER_PIXEL, rt.ADJ_TILE16, rt.ADJ_QUAD, rt.ADJ_BLOCK_WINDOW)
+        variants = (rt.ADJ_QUAD,)  # the walk variants are one kernel
         if prefix:
             variants += (rt.ADJ_BLOCK_PREFIX,)
     cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count

@@ -13,8 +13,10 @@
 //   3. k_bins_split     image -> sinogram ops: one thread per detector bin and
 //                       chunk of image lines gathers along its lines (no
 //                       atomics); k_bins_reduce adds the chunks in order.
-//      k_pixels         sinogram -> image ops: one thread per pixel gathers
-//                       over every view (no atomics).
+//      k_pixels_walk    sinogram -> image ops: one wavefront per 16-wide pixel
+//                       tile and chunk of views gathers over its views, each
+//                       staged in LDS (no atomics); k_sum_chunks adds the
+//                       chunks in order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,6 +24,7 @@
 #include <cmath>
 #include <cstdio>
 #include <mutex>
+#include <type_traits>
 
 #include "dd.h"
 #include "dd2d_body.h"
@@ -35,23 +38,8 @@ using namespace body2d;
 
 std::atomic<int> g_forced_tile{0};
 // sinogram -> image kernel of dd2d_run and of plans without a variant:
-// -1 = automatic: 2 x 2 quads for up to 4 instances per launch when they
-// still give at least 4 workgroups per compute unit, per pixel otherwise.
+// -1 = automatic (the walk).
 std::atomic<int> g_adjoint_variant{-1};
-
-// Compute units of the first device the library runs on (thread-safe static;
-// every device of one process is the same part here).
-int compute_units() {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        n > 0)
-      return n;
-    return 256;
-  }();
-  return cus;
-}
 
 // A variant is a sinogram -> image kernel (DD_ADJ_*), optionally OR-ed with
 // DD_FWD_PREFIX (image -> sinogram through running sums, tile 1).
@@ -63,18 +51,15 @@ bool known_variant(int v) {
 
 // The automatic choice keeps the walks, so a slice run alone gives the bits
 // it gets in any batch; the running-sum adjoint (DD_ADJ_BLOCK_PREFIX, tile 1
-// only) is chosen explicitly or by the autotuner.
+// only) is chosen explicitly or by the autotuner.  The walk variants are one
+// kernel (the staged walk, or per pixel where its bins are too fine).
 int adjoint_variant(int requested, const Geo2& g) {
   if (!known_variant(requested)) requested = g_adjoint_variant;
   // the running sums are per instance: instance tile 1 only
-  int flags = (requested >= 0 && g.BT == 1) ? (requested & DD_FWD_PREFIX) : 0;
-  int adj = requested >= 0 ? (requested & ~DD_FWD_PREFIX) : -1;
-  if (adj == DD_ADJ_BLOCK_PREFIX && g.BT != 1) adj = -1;
-  if (adj < 0) {
-    const long long quad_groups = 1LL * ((g.W + 31) / 32) * ((g.H + 31) / 32) * (g.Bp / g.BT);
-    adj = (g.BT <= 4 && quad_groups >= 4LL * compute_units()) ? DD_ADJ_QUAD : DD_ADJ_PER_PIXEL;
-  }
-  return adj | flags;
+  if (requested < 0 || g.BT != 1) return DD_ADJ_PER_PIXEL;
+  return ((requested & ~DD_FWD_PREFIX) == DD_ADJ_BLOCK_PREFIX ? DD_ADJ_BLOCK_PREFIX
+                                                              : DD_ADJ_PER_PIXEL) |
+         (requested & DD_FWD_PREFIX);
 }
 
 // Whether op runs through the running-sum adjoint (its weights per pixel
@@ -276,8 +261,9 @@ __global__ __launch_bounds__(kThreads) void k_bins_reduce(
   out[o] = epi_value(ep, sum * wk, o);
 }
 
-// sinogram -> image: one thread per pixel, BT instances, all views.
-// Variant DD_ADJ_PER_PIXEL: every pixel finds its bins on its own.
+// sinogram -> image: one thread per pixel, BT instances, all views; every
+// pixel finds its bins on its own.  For detectors so fine that the staged
+// walk's tiles overflow their slots (walk_rows).
 template <int BT, int WM, int TW>
 __global__ __launch_bounds__(kThreads) void k_pixels(
     Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
@@ -291,6 +277,87 @@ __global__ __launch_bounds__(kThreads) void k_pixels(
   const int r = blockIdx.y * TH + ty;
   if (c >= g.W || r >= g.H) return;
   pixels_body<BT, WM>(g, views, edges, lines, pint, sino, out, r, c, blockIdx.z * BT, ep);
+}
+
+// Edge range of every (view, 16 x 8 pixels): ranges[v * tiles + t].
+__global__ __launch_bounds__(kThreads) void k_walk_ranges(
+    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
+    const LineGeo* __restrict__ lines, unsigned* __restrict__ ranges) {
+  const int tx = (g.W + kWalkW - 1) / kWalkW;
+  const int tiles = walk_range_tiles(g);
+  const long long idx = 1LL * blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= 1LL * tiles * g.V) return;
+  const int v = static_cast<int>(idx / tiles), t = static_cast<int>(idx % tiles);
+  const int c0 = (t % tx) * kWalkW, r0 = (t / tx) * kWalkRangeH;
+  ranges[idx] = pack_range(knot_range(
+      g, views[v], edges + static_cast<size_t>(v) * (g.D + 1),
+      lines + static_cast<size_t>(v) * g.Lmax, r0, min(r0 + kWalkRangeH, g.H), c0,
+      min(c0 + kWalkW, g.W)));
+}
+
+// sinogram -> image by the staged walk: one wavefront per pixel tile.  SPLIT:
+// workgroup row y takes view chunk y and writes its partial image to out
+// (k_sum_chunks adds them); otherwise a wavefront takes the chunks one after
+// the other and adds their sums in registers.
+// Wavefronts per SIMD the register budget is held to: 4 (128 registers) where
+// that fits; the distance weight at 4 and more instances spills there (16
+// slices' weighted backprojection 1.00 against 0.87 ms at 3).
+template <int BT, int WM>
+constexpr int walk_waves() {
+  return WM == W_BPW && BT >= 4 ? 3 : 4;
+}
+
+template <int BT, int WM, int NP, bool SPLIT>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(walk_waves<BT, WM>()))) void k_pixels_walk(
+    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
+    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
+    const unsigned* __restrict__ ranges, const float* __restrict__ sino,
+    float* __restrict__ out, Epi ep) {
+  __shared__ WalkLds<BT> lds[kThreads / 64];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
+  const int tx = (g.W + kWalkW - 1) / kWalkW;
+  const int tiles = tx * ((g.H + 4 * NP - 1) / (4 * NP));
+  const int tile = static_cast<int>(blockIdx.x) * (kThreads / 64) + wave;
+  if (tile >= tiles) return;
+  const int c0 = (tile % tx) * kWalkW, r0 = (tile / tx) * 4 * NP;
+  const int b0 = blockIdx.z * BT;
+  const int nc = walk_chunks(g.V);
+  const int ch0 = SPLIT ? static_cast<int>(blockIdx.y) : 0, ch1 = SPLIT ? ch0 + 1 : nc;
+  if (SPLIT) out += static_cast<size_t>(blockIdx.y) * g.B * g.H * g.W;
+  auto put = [&](int r, int c, int b, float v) {
+    if (c < g.W && r < g.H && b0 + b < g.B) {
+      const size_t at = (static_cast<size_t>(b0 + b) * g.H + r) * g.W + c;
+      out[at] = SPLIT ? v : epi_value(ep, v, at);
+    }
+  };
+  float acc[NP][BT];
+  float sum[SPLIT ? 1 : NP][SPLIT ? 1 : BT];
+  for (int ch = ch0; ch < ch1; ++ch) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j)
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc[j][b] = 0.0f;
+    if (!walk_views<BT, WM, NP>(g, views, edges, lines, pint, ranges, sino, r0, c0, b0,
+                                walk_chunk_begin(g.V, ch), walk_chunk_begin(g.V, ch + 1), acc,
+                                lds[wave])) {
+      walk_views_again<BT, WM, NP>(g, views, edges, lines, pint, sino, r0, c0, b0, ch0, ch1, put);
+      return;
+    }
+    if constexpr (!SPLIT) {
+#pragma unroll
+      for (int j = 0; j < NP; ++j)
+#pragma unroll
+        for (int b = 0; b < BT; ++b) sum[j][b] = ch == 0 ? acc[j][b] : sum[j][b] + acc[j][b];
+    }
+  }
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+#pragma unroll
+  for (int j = 0; j < NP; ++j)
+#pragma unroll
+    for (int b = 0; b < BT; ++b)
+      put(r0 + (lane >> 4) + 4 * j, c0 + (lane & 15), b,
+          SPLIT ? acc[j][b] : sum[SPLIT ? 0 : j][SPLIT ? 0 : b]);
 }
 
 // View-resolved sinogram -> image: out[b][v] is view v's contribution
@@ -318,31 +385,6 @@ __global__ __launch_bounds__(kThreads) void k_pixels_views(
     if (b0 + b < g.B)
       out[(static_cast<size_t>(b0 + b) * g.V + v) * plane + static_cast<size_t>(r) * g.W + c] =
           acc[b];
-}
-
-// Variant DD_ADJ_QUAD: one thread per 2 x 2 pixel block, a 32 x 32 pixel
-// tile per workgroup.
-template <int BT, int WM>
-__global__ __launch_bounds__(kThreads) void k_pixels_quad(
-    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
-    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
-    const float* __restrict__ sino, float* __restrict__ out, Epi ep) {
-  const int c0 = blockIdx.x * (2 * kTile) + 2 * (threadIdx.x % kTile);
-  const int r0 = blockIdx.y * (2 * kTile) + 2 * (threadIdx.x / kTile);
-  if (c0 >= g.W || r0 >= g.H) return;
-  quads_body<BT, WM>(g, views, edges, lines, pint, sino, out, r0, c0, blockIdx.z * BT, ep);
-}
-
-// Variants DD_ADJ_TILE16 / DD_ADJ_TILE8: a T x T tile stages its lines' edge
-// positions per view in LDS.
-template <int BT, int WM, int T>
-__global__ __launch_bounds__(T * T) void k_pixels_tile(
-    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
-    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
-    const float* __restrict__ sino, float* __restrict__ out, Epi ep) {
-  __shared__ PixelTileLds<T> lds;
-  pixels_tile_body<BT, WM, T>(g, views, edges, lines, pint, sino, out, blockIdx.x,
-                              blockIdx.y, blockIdx.z * BT, lds, ep);
 }
 
 // ---------------------------------------------------------------------------
@@ -588,10 +630,12 @@ __global__ __launch_bounds__(kThreads) void k_sysmatrix(
 // host side
 // ---------------------------------------------------------------------------
 struct Layout {
-  size_t views, edges, wfp, lines, pint, geo_total;  // geometry tables
+  size_t views, edges, wfp, lines, pint, wranges, geo_total;  // geometry tables
   size_t buf0, buf1, part, data_total;                // data buffers
   size_t psino, krange, ppart;                        // running-sum adjoint
   size_t prow, pcol;                                  // running-sum forward
+  size_t wpart;                                       // staged walk's partial images
+  bool has_ranges, split;
 };
 
 constexpr size_t kAlign = 256;
@@ -612,7 +656,17 @@ bool to_sino(int op) {
 // (16 bytes each), knot ranges [V][tiles] and partial images
 // [chunks][B][H][W]; or the running-sum forward's line tables, rows
 // [B][H][W+1] and columns [B][W][H+1] of 16-byte entries.
-Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone) {
+// Memory of the staged walk a layout holds: range table and partial images,
+// the table alone (a wavefront then takes all view chunks), or neither (the
+// per-pixel kernel).  The bits are the same.
+enum WalkMem { kWalkFull = 0, kWalkNoSplit = 1, kWalkNoTables = 2 };
+
+// Largest partial images that the view chunks are split for: what the
+// Infinity Cache can hand to the sum.  An op with more has wavefronts enough
+// without the split (4096 from 512 x 1024 pixels x 16 on).
+constexpr size_t kWalkPartBytes = size_t{256} << 20;
+
+Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone, int walk = kWalkFull) {
   Layout L{};
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -625,6 +679,8 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone) {
   L.wfp = take(sizeof(float) * g.V * g.D);
   L.lines = take(sizeof(LineGeo) * g.V * g.Lmax);
   L.pint = take(sizeof(float) * g.V * g.Lmax);
+  L.has_ranges = walk != kWalkNoTables;
+  if (L.has_ranges) L.wranges = take(sizeof(unsigned) * g.V * walk_range_tiles(g));
   L.geo_total = off;
   off = 0;
   if (to_sino(op)) {
@@ -638,6 +694,9 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone) {
   } else {
     L.buf0 = take(sizeof(float) * static_cast<size_t>(g.V) * g.D * g.Bp);
     L.buf1 = L.buf0;
+    const size_t part = sizeof(float) * static_cast<size_t>(walk_chunks(g.V)) * g.B * g.H * g.W;
+    L.split = walk == kWalkFull && walk_chunks(g.V) > 1 && part <= kWalkPartBytes;
+    if (L.split) L.wpart = take(part);
     if (prefix & kPrefAdjoint) {
       L.psino = take(16 * static_cast<size_t>(g.B) * g.V * (g.D + 1));
       L.krange = take(8 * static_cast<size_t>(g.V) * prefix_tiles(g));
@@ -646,6 +705,11 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone) {
   }
   L.data_total = off;
   return L;
+}
+
+// Walk memory of a one-call op: none where the staged walk does not run.
+int run_walk_mem(const Geo2& g, int op, int variant) {
+  return to_sino(op) || prefix_path(g, op, variant) ? kWalkNoTables : kWalkFull;
 }
 
 // Planned workspaces hold the running-sum buffers whenever they can be used
@@ -689,6 +753,7 @@ struct GeoPtrs {
   const float* wfp;
   const LineGeo* lines;
   const float* pint;
+  const unsigned* ranges;
 };
 
 GeoPtrs geo_ptrs(const void* geo, const Layout& L) {
@@ -697,11 +762,12 @@ GeoPtrs geo_ptrs(const void* geo, const Layout& L) {
           reinterpret_cast<const double*>(b + L.edges),
           reinterpret_cast<const float*>(b + L.wfp),
           reinterpret_cast<const LineGeo*>(b + L.lines),
-          reinterpret_cast<const float*>(b + L.pint)};
+          reinterpret_cast<const float*>(b + L.pint),
+          L.has_ranges ? reinterpret_cast<const unsigned*>(b + L.wranges) : nullptr};
 }
 
 void launch_setup(const Geo2& g, const float* angles, void* geo,
-                  const Layout& L, hipStream_t st) {
+                  const Layout& L, hipStream_t st, bool ranges) {
   char* b = static_cast<char*>(geo);
   hipLaunchKernelGGL(k_setup2d, dim3(g.V), dim3(kThreads), 0, st, g, angles,
                      reinterpret_cast<ViewGeo*>(b + L.views),
@@ -709,23 +775,50 @@ void launch_setup(const Geo2& g, const float* angles, void* geo,
                      reinterpret_cast<float*>(b + L.wfp),
                      reinterpret_cast<LineGeo*>(b + L.lines),
                      reinterpret_cast<float*>(b + L.pint));
+  if (!ranges || !L.has_ranges) return;
+  const long long n = 1LL * g.V * walk_range_tiles(g);
+  hipLaunchKernelGGL(k_walk_ranges, dim3(static_cast<unsigned>((n + kThreads - 1) / kThreads)),
+                     dim3(kThreads), 0, st, g, reinterpret_cast<const ViewGeo*>(b + L.views),
+                     reinterpret_cast<const double*>(b + L.edges),
+                     reinterpret_cast<const LineGeo*>(b + L.lines),
+                     reinterpret_cast<unsigned*>(b + L.wranges));
 }
 
-// Per-pixel adjoint of one workgroup width (256 threads: TW x 256 / TW pixels).
-template <int BT, int TW>
-void launch_pixels(const Geo2& g, int op, const GeoPtrs& G, const float* buf0, float* output,
-                   hipStream_t st, const Epi& ep) {
-  constexpr int TH = kThreads / TW;
-  dim3 grid((g.W + TW - 1) / TW, (g.H + TH - 1) / TH, g.Bp / BT);
-  if (op == DD_PROJ_T)
-    hipLaunchKernelGGL((k_pixels<BT, W_FP, TW>), grid, dim3(kThreads), 0, st, g, G.views,
-                       G.edges, G.lines, G.pint, buf0, output, ep);
-  else if (op == DD_BPROJ)
-    hipLaunchKernelGGL((k_pixels<BT, W_BP, TW>), grid, dim3(kThreads), 0, st, g, G.views,
-                       G.edges, G.lines, G.pint, buf0, output, ep);
-  else
-    hipLaunchKernelGGL((k_pixels<BT, W_BPW, TW>), grid, dim3(kThreads), 0, st, g, G.views,
-                       G.edges, G.lines, G.pint, buf0, output, ep);
+// Staged walk of the sinogram -> image ops.
+template <int BT, int WM, int NP>
+void launch_walk(const Geo2& g, const GeoPtrs& G, const float* buf0, float* output, char* ws,
+                 const Layout& L, hipStream_t st, const Epi& ep) {
+  constexpr int TH = 4 * NP, kWaves = kThreads / 64;
+  const int tiles = ((g.W + kWalkW - 1) / kWalkW) * ((g.H + TH - 1) / TH);
+  const unsigned groups = (tiles + kWaves - 1) / kWaves;
+  if (L.split) {
+    const int nc = walk_chunks(g.V);
+    auto* part = reinterpret_cast<float*>(ws + L.wpart);
+    hipLaunchKernelGGL((k_pixels_walk<BT, WM, NP, true>), dim3(groups, nc, g.Bp / BT),
+                       dim3(kThreads), 0, st, g, G.views, G.edges, G.lines, G.pint, G.ranges,
+                       buf0, part, Epi{});
+    const size_t npix = static_cast<size_t>(g.B) * g.H * g.W;
+    hipLaunchKernelGGL(k_sum_chunks, dim3(static_cast<unsigned>((npix + kThreads - 1) / kThreads)),
+                       dim3(kThreads), 0, st, g, part, nc, output, ep);
+  } else {
+    hipLaunchKernelGGL((k_pixels_walk<BT, WM, NP, false>), dim3(groups, 1, g.Bp / BT),
+                       dim3(kThreads), 0, st, g, G.views, G.edges, G.lines, G.pint, G.ranges,
+                       buf0, output, ep);
+  }
+}
+
+// Per-pixel gather, workgroups of TW x 256 / TW pixels.
+template <int BT, int WM>
+void launch_pixels(const Geo2& g, const GeoPtrs& G, const float* buf0, float* output,
+                   hipStream_t st, const Epi& ep, int width) {
+  const int tw = width > 0 ? width : pix_tile_w<BT>();
+  const int th = kThreads / tw;
+  const dim3 grid((g.W + tw - 1) / tw, (g.H + th - 1) / th, g.Bp / BT);
+  const auto kernel = tw == 64   ? k_pixels<BT, WM, 64>
+                      : tw == 32 ? k_pixels<BT, WM, 32>
+                                 : k_pixels<BT, WM, 16>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, g, G.views, G.edges, G.lines, G.pint,
+                     buf0, output, ep);
 }
 
 template <int BT>
@@ -735,7 +828,6 @@ dd_status launch_tile(const Geo2& g, int op, int variant, const float* input,
   auto* buf0 = reinterpret_cast<float*>(ws + L.buf0);
   auto* buf1 = reinterpret_cast<float*>(ws + L.buf1);
   const int ntile = g.Bp / BT;
-  const int adj = variant & ~DD_FWD_PREFIX;
   if (BT == 1 && fwd_prefix_path(g, op, variant)) {
     auto* prow = reinterpret_cast<float4*>(ws + L.prow);
     auto* pcol = reinterpret_cast<float4*>(ws + L.pcol);
@@ -821,48 +913,23 @@ dd_status launch_tile(const Geo2& g, int op, int variant, const float* input,
       hipLaunchKernelGGL((k_interleave_sino<BT, false>), sgrid, dim3(kThreads),
                          0, st, g, G.views, G.wfp, input, buf0);
     ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
-    if (adj == DD_ADJ_QUAD) {
-      dim3 grid((g.W + 2 * kTile - 1) / (2 * kTile), (g.H + 2 * kTile - 1) / (2 * kTile), ntile);
-      if (op == DD_PROJ_T)
-        hipLaunchKernelGGL((k_pixels_quad<BT, W_FP>), grid, dim3(kThreads), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-      else if (op == DD_BPROJ)
-        hipLaunchKernelGGL((k_pixels_quad<BT, W_BP>), grid, dim3(kThreads), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
+    constexpr int kMost = BT >= 8 ? 2 : 4;
+    const int rows = L.has_ranges ? walk_rows(g) : 0;
+    auto run = [&](auto wm) {
+      constexpr int WM = decltype(wm)::value;
+      if (rows == kMost)
+        launch_walk<BT, WM, kMost>(g, G, buf0, output, ws, L, st, ep);
+      else if (rows > 0)
+        launch_walk<BT, WM, kMost / 2>(g, G, buf0, output, ws, L, st, ep);
       else
-        hipLaunchKernelGGL((k_pixels_quad<BT, W_BPW>), grid, dim3(kThreads), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-    } else if (adj == DD_ADJ_TILE16) {
-      dim3 grid((g.W + 15) / 16, (g.H + 15) / 16, ntile);
-      if (op == DD_PROJ_T)
-        hipLaunchKernelGGL((k_pixels_tile<BT, W_FP, 16>), grid, dim3(256), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-      else if (op == DD_BPROJ)
-        hipLaunchKernelGGL((k_pixels_tile<BT, W_BP, 16>), grid, dim3(256), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-      else
-        hipLaunchKernelGGL((k_pixels_tile<BT, W_BPW, 16>), grid, dim3(256), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-    } else if (adj == DD_ADJ_TILE8) {
-      dim3 grid((g.W + 7) / 8, (g.H + 7) / 8, ntile);
-      if (op == DD_PROJ_T)
-        hipLaunchKernelGGL((k_pixels_tile<BT, W_FP, 8>), grid, dim3(64), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-      else if (op == DD_BPROJ)
-        hipLaunchKernelGGL((k_pixels_tile<BT, W_BP, 8>), grid, dim3(64), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-      else
-        hipLaunchKernelGGL((k_pixels_tile<BT, W_BPW, 8>), grid, dim3(64), 0, st, g,
-                           G.views, G.edges, G.lines, G.pint, buf0, output, ep);
-    } else {
-      const int tw = sh.pix_width > 0 ? sh.pix_width : pix_tile_w<BT>();
-      if (tw == 64)
-        launch_pixels<BT, 64>(g, op, G, buf0, output, st, ep);
-      else if (tw == 32)
-        launch_pixels<BT, 32>(g, op, G, buf0, output, st, ep);
-      else
-        launch_pixels<BT, 16>(g, op, G, buf0, output, st, ep);
-    }
+        launch_pixels<BT, WM>(g, G, buf0, output, st, ep, sh.pix_width);
+    };
+    if (op == DD_PROJ_T)
+      run(std::integral_constant<int, W_FP>{});
+    else if (op == DD_BPROJ)
+      run(std::integral_constant<int, W_BP>{});
+    else
+      run(std::integral_constant<int, W_BPW>{});
   }
   return hipGetLastError() == hipSuccess ? DD_OK : DD_LAUNCH_FAIL;
 }
@@ -960,7 +1027,8 @@ size_t dd2d_workspace_size(int scan, int op, const dd_geom2d* g, int batch,
                            int views) {
   Geo2 q;
   if (!fill_geo(&q, scan, g, batch, views, pick_tile(batch))) return 0;
-  const Layout L = make_layout(q, op, prefix_regions(q, op, adjoint_variant(-1, q)));
+  const int var = adjoint_variant(-1, q);
+  const Layout L = make_layout(q, op, prefix_regions(q, op, var), run_walk_mem(q, op, var));
   return L.geo_total + L.data_total;
 }
 
@@ -973,11 +1041,11 @@ dd_status dd2d_run(int scan, int op, const dd_geom2d* g, const float* input,
   Geo2 q;
   if (!fill_geo(&q, scan, g, batch, views, pick_tile(batch))) return DD_BAD_ARG;
   const int var = adjoint_variant(-1, q);
-  const Layout L = make_layout(q, op, prefix_regions(q, op, var));
+  const Layout L = make_layout(q, op, prefix_regions(q, op, var), run_walk_mem(q, op, var));
   if (!ws || ws_bytes < L.geo_total + L.data_total) return DD_NO_WORKSPACE;
   auto st = static_cast<hipStream_t>(stream);
   char* w = static_cast<char*>(ws);
-  launch_setup(q, angles, w, L, st);
+  launch_setup(q, angles, w, L, st, !to_sino(op));
   return run_tiles(q, op, var, input, output, geo_ptrs(w, L), w + L.geo_total, L, st);
 }
 
@@ -990,14 +1058,19 @@ dd_status dd2d_run_noalloc(int scan, int op, const dd_geom2d* g, const float* in
   Geo2 q;
   if (!fill_geo(&q, scan, g, batch, views, pick_tile(batch))) return DD_BAD_ARG;
   const int var = adjoint_variant(-1, q);
-  const Layout L = make_layout(q, op, prefix_regions(q, op, var));
+  // the walk's memory as far as the scratch holds it (same bits)
+  Layout L;
+  int mem = run_walk_mem(q, op, var);
+  do {
+    L = make_layout(q, op, prefix_regions(q, op, var), mem);
+  } while (L.geo_total + L.data_total > DD_NOALLOC_SCRATCH_BYTES && mem++ < kWalkNoTables);
   if (L.geo_total + L.data_total > DD_NOALLOC_SCRATCH_BYTES) return DD_TOO_LARGE;
   char* w = static_cast<char*>(scratch_ptr());
   if (!w) return DD_LAUNCH_FAIL;
   // every table and buffer in the scratch is fully written by this call's
   // own launches before it is read, so nothing needs clearing between calls
   auto st = static_cast<hipStream_t>(stream);
-  launch_setup(q, angles, w, L, st);
+  launch_setup(q, angles, w, L, st, !to_sino(op));
   return run_tiles(q, op, var, input, output, geo_ptrs(w, L), w + L.geo_total, L, st);
 }
 
@@ -1012,11 +1085,11 @@ dd_status dd2d_run_views(int scan, int op, const dd_geom2d* g, const float* inpu
   Geo2 q;
   const int tile = std::min(pick_tile(batch), 4);
   if (!fill_geo(&q, scan, g, batch, views, tile)) return DD_BAD_ARG;
-  const Layout L = make_layout(q, op);
+  const Layout L = make_layout(q, op, kPrefNone, kWalkNoTables);
   if (!ws || ws_bytes < L.geo_total + L.data_total) return DD_NO_WORKSPACE;
   auto st = static_cast<hipStream_t>(stream);
   char* w = static_cast<char*>(ws);
-  launch_setup(q, angles, w, L, st);
+  launch_setup(q, angles, w, L, st, false);
   const GeoPtrs G = geo_ptrs(w, L);
   switch (q.BT) {
     case 1: return launch_views<1>(q, op, input, output, G, w + L.geo_total, L, st);
@@ -1030,7 +1103,7 @@ size_t dd2d_views_workspace_size(int scan, int op, const dd_geom2d* g, int batch
   Geo2 q;
   if (check_op(scan, op) != DD_OK) return 0;
   if (!fill_geo(&q, scan, g, batch, views, std::min(pick_tile(batch), 4))) return 0;
-  const Layout L = make_layout(q, op);
+  const Layout L = make_layout(q, op, kPrefNone, kWalkNoTables);
   return L.geo_total + L.data_total;
 }
 
@@ -1048,7 +1121,7 @@ dd_status dd2d_geometry(int scan, const dd_geom2d* g, const float* angles,
   if (!angles || !fill_geo(&q, scan, g, 1, views, 1)) return DD_BAD_ARG;
   const Layout L = make_layout(q, DD_PROJ);
   if (!geo || geo_bytes < L.geo_total) return DD_NO_WORKSPACE;
-  launch_setup(q, angles, geo, L, static_cast<hipStream_t>(stream));
+  launch_setup(q, angles, geo, L, static_cast<hipStream_t>(stream), true);
   return hipGetLastError() == hipSuccess ? DD_OK : DD_LAUNCH_FAIL;
 }
 
@@ -1113,7 +1186,7 @@ bool sys_setup(int scan, const dd_geom2d* g, const float* angles, int views,
                void* ws, size_t ws_bytes, hipStream_t st, Geo2* q, Layout* L) {
   if (scan < DD_PARA || scan > DD_FAN_ARC || !angles) return false;
   if (!fill_geo(q, scan, g, 1, views, 1)) return false;
-  *L = make_layout(*q, DD_PROJ_T);
+  *L = make_layout(*q, DD_PROJ_T, kPrefNone, kWalkNoTables);
   if (!ws || ws_bytes < L->geo_total) return false;
   char* w = static_cast<char*>(ws);
   hipLaunchKernelGGL(k_setup2d, dim3(q->V), dim3(kThreads), 0, st, *q, angles,
@@ -1131,7 +1204,7 @@ extern "C" {
 size_t dd2d_sysmatrix_workspace_size(int scan, const dd_geom2d* g, int views) {
   Geo2 q;
   if (!fill_geo(&q, scan, g, 1, views, 1)) return 0;
-  return make_layout(q, DD_PROJ_T).geo_total;
+  return make_layout(q, DD_PROJ_T, kPrefNone, kWalkNoTables).geo_total;
 }
 
 dd_status dd2d_sysmatrix_count(int scan, const dd_geom2d* g,

@@ -530,8 +530,7 @@ __device__ __forceinline__ float bins_accumulate_prefix(
 // the edge map, closed form per geometry, in FP32 with hardware reciprocals
 // (v_rcp_f32) instead of IEEE divisions.  Only a starting guess; the exact
 // bin is then fixed against the edge table with edge_pos().
-__device__ __forceinline__ int guess_bin_fast(const Geo2& g, const ViewGeo& vg,
-                                              double a) {
+__device__ __forceinline__ float guess_bin_real(const Geo2& g, const ViewGeo& vg, double a) {
   float kf;
   if (g.scan == DD_FAN_ARC) {
     // Fan angle of the ray through a relative to the detector centre,
@@ -559,13 +558,57 @@ __device__ __forceinline__ int guess_bin_fast(const Geo2& g, const ViewGeo& vg,
     const float u = static_cast<float>(vg.xaxis ? a * vg.c : a * vg.s);
     kf = g.D * 0.5f + (vg.flip ? -(u - g.bin) : (u - g.bin)) * __builtin_amdgcn_rcpf(g.det);
   }
-  kf = fminf(fmaxf(kf, -4.0f), g.D + 4.0f);
+  return kf;
+}
+
+__device__ __forceinline__ int guess_bin_fast(const Geo2& g, const ViewGeo& vg, double a) {
+  const float kf = fminf(fmaxf(guess_bin_real(g, vg, a), -4.0f), g.D + 4.0f);
   return static_cast<int>(floorf(kf));
 }
 
+// Where axis points lie relative to pixel i of one line, in pixels from its
+// lower edge: below 0 before the pixel, 1 and up past it.  The one definition
+// used by every sinogram -> image walk, so they agree bit for bit; it is the
+// forward's t - i (edge_pos) up to the FP64 rounding of the products.
+struct PixelFrame {
+  double inv_p, b;
+  __device__ __forceinline__ PixelFrame(double a0, double ip, int i)
+      : inv_p(ip), b(fma(a0, ip, static_cast<double>(i))) {}
+  __device__ __forceinline__ double at(double e) const { return fma(e, inv_p, -b); }
+};
+
+// Fraction of the pixel that lies below such a point.
+__device__ __forceinline__ float pixel_fraction(double u) {
+  return __builtin_amdgcn_fmed3f(static_cast<float>(u), 0.0f, 1.0f);
+}
+
+// Adds the bins from k on that reach the pixel, given the search's state
+// (u1, u2: bin k's edges; k the last bin whose lower edge lies before the
+// pixel, or 0): overlap * weight * sinogram, bins ascending.
+template <int BT>
+__device__ __forceinline__ void pixel_walk(const Geo2& g, const double* __restrict__ ev,
+                                           const PixelFrame& fr, double u1, double u2, int k,
+                                           float gw, const float* __restrict__ sv,
+                                           float (&acc)[BT]) {
+  float p1 = pixel_fraction(u1);
+  while (u1 < 1.0) {
+    const float p2 = pixel_fraction(u2);
+    const float w = (p2 - p1) * gw;
+    float q[BT];
+    load_sino<BT>(g, sv, k, q);
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[b] = fmaf(w, q[b], acc[b]);
+    if (++k >= g.D) break;
+    u1 = u2;
+    p1 = p2;
+    if (u1 >= 1.0) break;
+    u2 = fr.at(ev[k + 1]);
+  }
+}
+
 // Contribution of view v to pixel (r, c): find the bins whose edges bracket
-// the pixel in its line (closed-form guess, fixed exactly with edge_pos),
-// then accumulate overlap * weight * sinogram.
+// the pixel in its line (closed-form guess, fixed exactly against the edge
+// table), then accumulate overlap * weight * sinogram.
 template <int BT, int WM>
 __device__ __forceinline__ void pixel_one_view(
     const Geo2& g, const ViewGeo& vg, int v, const double* __restrict__ edges,
@@ -574,48 +617,35 @@ __device__ __forceinline__ void pixel_one_view(
     float (&acc)[BT]) {
   // line geometry loaded in the branch, so a caller whose row r is
   // wave-uniform gets scalar loads on row-axis views
-  int i, N;
+  int i;
   LineGeo lg;
   float pl;
   if (vg.xaxis) {
     i = c;
-    N = g.W;
     lg = lines[static_cast<size_t>(v) * g.Lmax + r];
     pl = pint[static_cast<size_t>(v) * g.Lmax + r];
   } else {
     i = g.H - 1 - r;
-    N = g.H;
     lg = lines[static_cast<size_t>(v) * g.Lmax + c];
     pl = pint[static_cast<size_t>(v) * g.Lmax + c];
   }
   const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
+  const PixelFrame fr(lg.a0, lg.inv_p, i);
   // k = the last bin whose lower edge lies before pixel i (or 0): unique,
-  // whatever the guess.  The positions of edges k and k + 1 found on the way
-  // start the walk.
+  // whatever the guess
   int k = min(max(guess_bin_fast(g, vg, lg.a0 + (i + 0.5) * static_cast<double>(pl)), 0),
               g.D - 1);
-  EdgePos p1 = edge_pos(ev[k], lg.a0, lg.inv_p, N);
-  while (k > 0 && p1.c >= i) p1 = edge_pos(ev[--k], lg.a0, lg.inv_p, N);
-  EdgePos p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  while (p2.c < i) {
+  double u1 = fr.at(ev[k]);
+  while (k > 0 && u1 >= 0.0) u1 = fr.at(ev[--k]);
+  double u2 = fr.at(ev[k + 1]);
+  while (u2 < 0.0) {
     if (++k >= g.D) return;
-    p1 = p2;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
+    u1 = u2;
+    u2 = fr.at(ev[k + 1]);
   }
   float gw = (WM == W_FP) ? pl : bp_const(g);
   if constexpr (WM == W_BPW) gw *= fbp_weight(g, vg, xcw, ycw);
-  const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
-  while (p1.c <= i) {
-    const float w = overlap_in_pixel(p1, p2, i) * gw;
-    float q[BT];
-    load_sino<BT>(g, sv, k, q);
-#pragma unroll
-    for (int b = 0; b < BT; ++b) acc[b] = fmaf(w, q[b], acc[b]);
-    if (++k >= g.D) break;
-    p1 = p2;
-    if (p1.c > i) break;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  }
+  pixel_walk<BT>(g, ev, fr, u1, u2, k, gw, sino_view<BT>(g, sino, v, b0), acc);
 }
 
 // First-bin guess for the pixel centred at (xc, yc) from the view alone: the
@@ -666,405 +696,31 @@ __device__ __forceinline__ PixViewStart pixel_view_start(
   return s;
 }
 
-// pixel_one_view from a start loaded ahead: the same search (edge k is
-// P(k) = edge_pos(ev[k]); going down, the old lower edge becomes the upper
-// one), the same walk.  Same bins, same order, same values: equal bit for
-// bit.
+// pixel_one_view from a start loaded ahead: the same search (going down, the
+// old lower edge becomes the upper one), the same walk.  Same bins, same
+// order, same values: equal bit for bit.
 template <int BT, int WM>
 __device__ __forceinline__ void pixel_view_from(
     const Geo2& g, const ViewGeo& vg, int v, const double* __restrict__ edges,
     const PixViewStart& s, const float* __restrict__ sino, int r, int c, int b0, float xcw,
     float ycw, float (&acc)[BT]) {
   const int i = vg.xaxis ? c : g.H - 1 - r;
-  const int N = vg.xaxis ? g.W : g.H;
-  const LineGeo lg = s.lg;
   const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
+  const PixelFrame fr(s.lg.a0, s.lg.inv_p, i);
   int k = s.k0;
-  EdgePos p1 = edge_pos(s.ea, lg.a0, lg.inv_p, N);
-  EdgePos p2 = edge_pos(s.eb, lg.a0, lg.inv_p, N);
-  while (k > 0 && p1.c >= i) {
-    p2 = p1;
-    p1 = edge_pos(ev[--k], lg.a0, lg.inv_p, N);
+  double u1 = fr.at(s.ea), u2 = fr.at(s.eb);
+  while (k > 0 && u1 >= 0.0) {
+    u2 = u1;
+    u1 = fr.at(ev[--k]);
   }
-  while (p2.c < i) {
+  while (u2 < 0.0) {
     if (++k >= g.D) return;
-    p1 = p2;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
+    u1 = u2;
+    u2 = fr.at(ev[k + 1]);
   }
   float gw = (WM == W_FP) ? s.pl : bp_const(g);
   if constexpr (WM == W_BPW) gw *= fbp_weight(g, vg, xcw, ycw);
-  const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
-  while (p1.c <= i) {
-    const float w = overlap_in_pixel(p1, p2, i) * gw;
-    float q[BT];
-    load_sino<BT>(g, sv, k, q);
-#pragma unroll
-    for (int b = 0; b < BT; ++b) acc[b] = fmaf(w, q[b], acc[b]);
-    if (++k >= g.D) break;
-    p1 = p2;
-    if (p1.c > i) break;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  }
-}
-
-// Contributions of view v to the two consecutive pixels i0, i0 + 1 of one
-// line (i0 + 1 only when has1): one first-bin search for i0, then one walk
-// over the bins that reach either pixel, each sinogram tile loaded once.  A
-// bin contributes to pixel i exactly when its edge cells bracket i
-// (p1.c <= i <= p2.c), which is the set and order of bins pixel_one_view
-// walks for i, so each pixel's sum is the same bit for bit.
-template <int BT, int WM>
-__device__ __forceinline__ void pixel_pair_view(
-    const Geo2& g, const ViewGeo& vg, int v, const double* __restrict__ edges,
-    const LineGeo& lg, float pl, const float* __restrict__ sino, int i0, bool has1, int N,
-    int b0, float gw0, float gw1, float (&acc0)[BT], float (&acc1)[BT]) {
-  const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
-  const int i1 = i0 + 1, ilast = has1 ? i1 : i0;
-  int k = min(max(guess_bin_fast(g, vg, lg.a0 + (i0 + 0.5) * static_cast<double>(pl)), 0),
-              g.D - 1);
-  EdgePos p1 = edge_pos(ev[k], lg.a0, lg.inv_p, N);
-  while (k > 0 && p1.c >= i0) p1 = edge_pos(ev[--k], lg.a0, lg.inv_p, N);
-  EdgePos p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  while (p2.c < i0) {
-    if (++k >= g.D) return;
-    p1 = p2;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  }
-  const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
-  while (p1.c <= ilast) {
-    float q[BT];
-    load_sino<BT>(g, sv, k, q);
-    if (p1.c <= i0 && i0 <= p2.c) {
-      const float w = overlap_in_pixel(p1, p2, i0) * gw0;
-#pragma unroll
-      for (int b = 0; b < BT; ++b) acc0[b] = fmaf(w, q[b], acc0[b]);
-    }
-    if (has1 && p1.c <= i1 && i1 <= p2.c) {
-      const float w = overlap_in_pixel(p1, p2, i1) * gw1;
-#pragma unroll
-      for (int b = 0; b < BT; ++b) acc1[b] = fmaf(w, q[b], acc1[b]);
-    }
-    if (++k >= g.D) break;
-    p1 = p2;
-    if (p1.c > ilast) break;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  }
-}
-
-// sinogram -> image for the 2 x 2 pixel block at (r0, c0), all views: per
-// view the block is two lines of two consecutive pixels whichever the axis
-// (image rows c0, c0 + 1 on rows r0, r0 + 1; or columns, read bottom-up).
-// Equal bit for bit to pixels_body on each of the four pixels.
-template <int BT, int WM>
-__device__ __forceinline__ void quads_body(
-    const Geo2& g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
-    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
-    const float* __restrict__ sino, float* __restrict__ out, int r0, int c0, int b0,
-    const Epi& ep = Epi{}) {
-  const bool hr = r0 + 1 < g.H, hc = c0 + 1 < g.W;
-  float xc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}}, yc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-  if constexpr (WM == W_BPW) {
-#pragma unroll
-    for (int dr = 0; dr < 2; ++dr)
-#pragma unroll
-      for (int dc = 0; dc < 2; ++dc) pixel_centre(g, 1, r0 + dr, c0 + dc, &xc[dr][dc], &yc[dr][dc]);
-  }
-  float acc[2][2][BT];  // [row offset][column offset][instance]
-#pragma unroll
-  for (int dr = 0; dr < 2; ++dr)
-#pragma unroll
-    for (int dc = 0; dc < 2; ++dc)
-#pragma unroll
-      for (int b = 0; b < BT; ++b) acc[dr][dc][b] = 0.0f;
-  const float kbp = bp_const(g);
-  for (int v = 0; v < g.V; ++v) {
-    const ViewGeo vg = views[v];
-    const LineGeo* __restrict__ lv = lines + static_cast<size_t>(v) * g.Lmax;
-    const float* __restrict__ pv = pint + static_cast<size_t>(v) * g.Lmax;
-    if (vg.xaxis) {
-      // lines = image rows r0, r0 + 1; pixels c0, c0 + 1
-#pragma unroll
-      for (int dr = 0; dr < 2; ++dr) {
-        if (dr == 1 && !hr) break;
-        const int l = r0 + dr;
-        const float pl = pv[l];
-        float gw0 = (WM == W_FP) ? pl : kbp, gw1 = gw0;
-        if constexpr (WM == W_BPW) {
-          gw0 *= fbp_weight(g, vg, xc[dr][0], yc[dr][0]);
-          gw1 *= fbp_weight(g, vg, xc[dr][1], yc[dr][1]);
-        }
-        pixel_pair_view<BT, WM>(g, vg, v, edges, lv[l], pl, sino, c0, hc, g.W, b0, gw0, gw1,
-                                acc[dr][0], acc[dr][1]);
-      }
-    } else {
-      // lines = image columns c0, c0 + 1; pixels i = H - 1 - r: the pair
-      // (i0, i0 + 1) is rows (r0 + 1, r0), or row r0 alone on the last row
-#pragma unroll
-      for (int dc = 0; dc < 2; ++dc) {
-        if (dc == 1 && !hc) break;
-        const int l = c0 + dc;
-        const float pl = pv[l];
-        float gw0 = (WM == W_FP) ? pl : kbp, gw1 = gw0;
-        if (hr) {
-          if constexpr (WM == W_BPW) {
-            gw0 *= fbp_weight(g, vg, xc[1][dc], yc[1][dc]);
-            gw1 *= fbp_weight(g, vg, xc[0][dc], yc[0][dc]);
-          }
-          pixel_pair_view<BT, WM>(g, vg, v, edges, lv[l], pl, sino, g.H - 2 - r0, true, g.H,
-                                  b0, gw0, gw1, acc[1][dc], acc[0][dc]);
-        } else {
-          if constexpr (WM == W_BPW) gw0 *= fbp_weight(g, vg, xc[0][dc], yc[0][dc]);
-          pixel_pair_view<BT, WM>(g, vg, v, edges, lv[l], pl, sino, g.H - 1 - r0, false, g.H,
-                                  b0, gw0, gw1, acc[0][dc], acc[1][dc]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int dr = 0; dr < 2; ++dr)
-#pragma unroll
-    for (int dc = 0; dc < 2; ++dc)
-      if ((dr == 0 || hr) && (dc == 0 || hc))
-#pragma unroll
-        for (int b = 0; b < BT; ++b)
-          if (b0 + b < g.B) {
-            const size_t at = (static_cast<size_t>(b0 + b) * g.H + r0 + dr) * g.W + c0 + dc;
-            out[at] = epi_value(ep, acc[dr][dc][b], at);
-          }
-}
-
-// Contributions of view v to the run of NP consecutive pixels ib .. ib+NP-1
-// of one line, of which positions pf .. pl are real pixels: one first-bin
-// search for pixel ib + pf, then one walk over the bins that reach any of
-// them, each sinogram tile loaded once.  Per pixel the same bins in the same
-// order as pixel_one_view: equal bit for bit.
-template <int BT, int WM, int NP>
-__device__ __forceinline__ void pixel_run_view(
-    const Geo2& g, const ViewGeo& vg, int v, const double* __restrict__ edges,
-    const LineGeo& lg, float pl, const float* __restrict__ sino, int ib, int pf, int plst,
-    int N, int b0, const float (&gw)[NP], float (&acc)[NP][BT]) {
-  const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
-  const int ifirst = ib + pf, ilast = ib + plst;
-  int k = min(max(guess_bin_fast(g, vg, lg.a0 + (ifirst + 0.5) * static_cast<double>(pl)), 0),
-              g.D - 1);
-  EdgePos p1 = edge_pos(ev[k], lg.a0, lg.inv_p, N);
-  while (k > 0 && p1.c >= ifirst) p1 = edge_pos(ev[--k], lg.a0, lg.inv_p, N);
-  EdgePos p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  while (p2.c < ifirst) {
-    if (++k >= g.D) return;
-    p1 = p2;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  }
-  const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
-  while (p1.c <= ilast) {
-    float q[BT];
-    load_sino<BT>(g, sv, k, q);
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int i = ib + p;
-      if (p >= pf && p <= plst && p1.c <= i && i <= p2.c) {
-        const float w = overlap_in_pixel(p1, p2, i) * gw[p];
-#pragma unroll
-        for (int b = 0; b < BT; ++b) acc[p][b] = fmaf(w, q[b], acc[p][b]);
-      }
-    }
-    if (++k >= g.D) break;
-    p1 = p2;
-    if (p1.c > ilast) break;
-    p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-  }
-}
-
-// pixel_run_view with the bins read as one window: the K + 1 edges and K
-// sinogram values from one bin below the first pixel's guess are loaded at
-// once (independent loads, one round trip instead of one per bin), every
-// bin of the window is tested against every pixel of the run, and the walk
-// continues one bin at a time only if the run reaches past the window.  The
-// window is used only when nothing below it can reach the run (its first
-// edge lies before the run, or it starts at bin 0); otherwise the serial
-// search decides.  Per pixel the same bins in the same (ascending) order,
-// with the same overlaps: equal bit for bit.
-template <int BT, int WM, int NP, int K>
-__device__ __forceinline__ void pixel_run_view_win(
-    const Geo2& g, const ViewGeo& vg, int v, const double* __restrict__ edges,
-    const LineGeo& lg, float pl, const float* __restrict__ sino, int ib, int pf, int plst,
-    int N, int b0, const float (&gw)[NP], float (&acc)[NP][BT]) {
-  const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
-  const int ifirst = ib + pf, ilast = ib + plst;
-  if (g.D < K + 1) {
-    pixel_run_view<BT, WM, NP>(g, vg, v, edges, lg, pl, sino, ib, pf, plst, N, b0, gw, acc);
-    return;
-  }
-  static_assert(K % 4 == 0, "window of whole 4-bin groups");
-  const int kg = guess_bin_fast(g, vg, lg.a0 + (ifirst + 0.5) * static_cast<double>(pl));
-  // edges kw .. kw + K + 1 are read in pairs, so the window ends one edge
-  // short of the table's last (index D)
-  const int kw = min(max(kg - 1, 0), g.D - K - 1);
-  double e[K + 2];
-#pragma unroll
-  for (int j = 0; j < K + 2; j += 2) {
-    // 16-byte loads of edge pairs (8-byte aligned)
-    double2 pr;
-    __builtin_memcpy(&pr, ev + kw + j, sizeof(pr));
-    e[j] = pr.x;
-    e[j + 1] = pr.y;
-  }
-  const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
-  float q[K][BT];
-  if constexpr (BT == 1 && !sino_quad_major<BT>()) {
-    if (g.Bp == 1) {
-      // 16-byte loads of four bins (4-byte aligned)
-#pragma unroll
-      for (int j = 0; j < K; j += 4) {
-        float4 t;
-        __builtin_memcpy(&t, sv + kw + j, sizeof(t));
-        q[j][0] = t.x;
-        q[j + 1][0] = t.y;
-        q[j + 2][0] = t.z;
-        q[j + 3][0] = t.w;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < K; ++j) load_sino<BT>(g, sv, kw + j, q[j]);
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < K; ++j) load_sino<BT>(g, sv, kw + j, q[j]);
-  }
-  EdgePos p1 = edge_pos(e[0], lg.a0, lg.inv_p, N);
-  if (kw > 0 && p1.c >= ifirst) {
-    // a bin below the window may reach the run: the serial search decides
-    pixel_run_view<BT, WM, NP>(g, vg, v, edges, lg, pl, sino, ib, pf, plst, N, b0, gw, acc);
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < K; ++j) {
-    const EdgePos p2 = edge_pos(e[j + 1], lg.a0, lg.inv_p, N);
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int i = ib + p;
-      if (p >= pf && p <= plst && p1.c <= i && i <= p2.c) {
-        const float w = overlap_in_pixel(p1, p2, i) * gw[p];
-#pragma unroll
-        for (int b = 0; b < BT; ++b) acc[p][b] = fmaf(w, q[j][b], acc[p][b]);
-      }
-    }
-    p1 = p2;
-  }
-  // past the window, one bin at a time (the walk's own loop)
-  int k = kw + K;
-  if (k >= g.D) return;
-  while (p1.c <= ilast) {
-    const EdgePos p2 = edge_pos(ev[k + 1], lg.a0, lg.inv_p, N);
-    float qk[BT];
-    load_sino<BT>(g, sv, k, qk);
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int i = ib + p;
-      if (p >= pf && p <= plst && p1.c <= i && i <= p2.c) {
-        const float w = overlap_in_pixel(p1, p2, i) * gw[p];
-#pragma unroll
-        for (int b = 0; b < BT; ++b) acc[p][b] = fmaf(w, qk[b], acc[p][b]);
-      }
-    }
-    if (++k >= g.D) break;
-    p1 = p2;
-  }
-}
-
-// sinogram -> image for the Q x Q pixel block at (r0, c0), all views: per
-// view the block is Q lines of Q consecutive pixels whichever the axis (rows
-// over columns c0 .. c0+Q-1, or columns read bottom-up).  Equal bit for bit
-// to pixels_body on each pixel.  KW > 0: each line's bins are read as one
-// window of KW bins (pixel_run_view_win).
-template <int BT, int WM, int Q, int KW = 0>
-__device__ __forceinline__ void blocks_body(
-    const Geo2& g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
-    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
-    const float* __restrict__ sino, float* __restrict__ out, int r0, int c0, int b0) {
-  const int nr = min(Q, g.H - r0), nc = min(Q, g.W - c0);
-  // pixel centres once, before the view loop, as pixels_body takes them
-  float xc[Q][Q], yc[Q][Q];
-  if constexpr (WM == W_BPW) {
-#pragma unroll
-    for (int dr = 0; dr < Q; ++dr)
-#pragma unroll
-      for (int dc = 0; dc < Q; ++dc)
-        pixel_centre(g, 1, min(r0 + dr, g.H - 1), min(c0 + dc, g.W - 1), &xc[dr][dc],
-                     &yc[dr][dc]);
-  }
-  float acc[Q][Q][BT];  // [row offset][column offset][instance]
-#pragma unroll
-  for (int dr = 0; dr < Q; ++dr)
-#pragma unroll
-    for (int dc = 0; dc < Q; ++dc)
-#pragma unroll
-      for (int b = 0; b < BT; ++b) acc[dr][dc][b] = 0.0f;
-  const float kbp = bp_const(g);
-  for (int v = 0; v < g.V; ++v) {
-    const ViewGeo vg = views[v];
-    const LineGeo* __restrict__ lv = lines + static_cast<size_t>(v) * g.Lmax;
-    const float* __restrict__ pv = pint + static_cast<size_t>(v) * g.Lmax;
-    if (vg.xaxis) {
-      // lines = image rows r0 + dr; run position p = column c0 + p
-#pragma unroll
-      for (int dr = 0; dr < Q; ++dr) {
-        if (dr >= nr) break;
-        const int l = r0 + dr;
-        const float pl = pv[l];
-        float gw[Q];
-#pragma unroll
-        for (int p = 0; p < Q; ++p) {
-          gw[p] = (WM == W_FP) ? pl : kbp;
-          if constexpr (WM == W_BPW) gw[p] *= fbp_weight(g, vg, xc[dr][p], yc[dr][p]);
-        }
-        if constexpr (KW > 0)
-          pixel_run_view_win<BT, WM, Q, KW>(g, vg, v, edges, lv[l], pl, sino, c0, 0, nc - 1,
-                                            g.W, b0, gw, acc[dr]);
-        else
-          pixel_run_view<BT, WM, Q>(g, vg, v, edges, lv[l], pl, sino, c0, 0, nc - 1, g.W, b0,
-                                    gw, acc[dr]);
-      }
-    } else {
-      // lines = image columns c0 + dc; pixel i = H - 1 - r, so run position p
-      // (pixel H - r0 - Q + p) is row r0 + Q - 1 - p, real when p >= Q - nr
-      float run[Q][BT];
-#pragma unroll
-      for (int dc = 0; dc < Q; ++dc) {
-        if (dc >= nc) break;
-        const int l = c0 + dc;
-        const float pl = pv[l];
-        float gw[Q];
-#pragma unroll
-        for (int p = 0; p < Q; ++p) {
-          gw[p] = (WM == W_FP) ? pl : kbp;
-          if constexpr (WM == W_BPW)
-            gw[p] *= fbp_weight(g, vg, xc[Q - 1 - p][dc], yc[Q - 1 - p][dc]);
-#pragma unroll
-          for (int b = 0; b < BT; ++b) run[p][b] = acc[Q - 1 - p][dc][b];
-        }
-        if constexpr (KW > 0)
-          pixel_run_view_win<BT, WM, Q, KW>(g, vg, v, edges, lv[l], pl, sino, g.H - r0 - Q,
-                                            Q - nr, Q - 1, g.H, b0, gw, run);
-        else
-          pixel_run_view<BT, WM, Q>(g, vg, v, edges, lv[l], pl, sino, g.H - r0 - Q, Q - nr,
-                                    Q - 1, g.H, b0, gw, run);
-#pragma unroll
-        for (int p = 0; p < Q; ++p)
-#pragma unroll
-          for (int b = 0; b < BT; ++b) acc[Q - 1 - p][dc][b] = run[p][b];
-      }
-    }
-  }
-#pragma unroll
-  for (int dr = 0; dr < Q; ++dr)
-#pragma unroll
-    for (int dc = 0; dc < Q; ++dc)
-      if (dr < nr && dc < nc)
-#pragma unroll
-        for (int b = 0; b < BT; ++b)
-          if (b0 + b < g.B)
-            out[(static_cast<size_t>(b0 + b) * g.H + r0 + dr) * g.W + c0 + dc] = acc[dr][dc][b];
+  pixel_walk<BT>(g, ev, fr, u1, u2, k, gw, sino_view<BT>(g, sino, v, b0), acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1241,20 +897,32 @@ __device__ __forceinline__ int2 knot_range(const Geo2& g, const ViewGeo& vg,
     corner(c0, g.H - r1), corner(c0, g.H - r0), corner(c1 - 1, g.H - r1),
         corner(c1 - 1, g.H - r0);
   }
-  // last knot <= amin, first knot >= amax (edges ascend in walk order)
-  int lo = 0, hi = g.D;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) / 2;
-    if (ev[mid] <= amin) lo = mid; else hi = mid - 1;
-  }
+  // last knot <= amin, first knot >= amax (edges ascend in walk order),
+  // from the closed-form guesses
+  int lo = min(max(guess_bin_fast(g, vg, amin), 0), g.D);
+  while (lo > 0 && ev[lo] > amin) --lo;
+  while (lo < g.D && ev[lo + 1] <= amin) ++lo;
   const int kb = max(lo - 1, 0);
-  lo = 0, hi = g.D;
-  while (lo < hi) {
-    const int mid = (lo + hi) / 2;
-    if (ev[mid] >= amax) hi = mid; else lo = mid + 1;
-  }
-  const int ke = min(lo + 1, g.D);
+  int hi = min(max(guess_bin_fast(g, vg, amax) + 1, 0), g.D);
+  while (hi < g.D && ev[hi] < amax) ++hi;
+  while (hi > 0 && ev[hi - 1] >= amax) --hi;
+  const int ke = min(hi + 1, g.D);
   return make_int2(kb, max(ke, kb + 1));
+}
+
+// Views are summed in chunks, the chunk sums added in order: the same
+// partition and order in every sinogram -> image walk, whether one wavefront
+// takes all chunks or each chunk has its own, so a slice gets the same bits
+// alone and in any batch.  Chunks are what a small image is split over the
+// chip by (a 64 x 64 image is 16 wavefronts); their sums are also shorter, so
+// rounding grows less over the views.
+__host__ __device__ inline int walk_chunks(int views) {
+  const int n = views / 8;
+  return n < 1 ? 1 : n > 8 ? 8 : n;
+}
+
+__host__ __device__ inline int walk_chunk_begin(int views, int ch) {
+  return static_cast<int>(1LL * views * ch / walk_chunks(views));
 }
 
 // sinogram -> image for one pixel, all views.  Each view's search is
@@ -1269,162 +937,404 @@ __device__ __forceinline__ void pixels_body(
     const Epi& ep = Epi{}) {
   float xcw = 0.0f, ycw = 0.0f;
   pixel_centre(g, 1, r, c, &xcw, &ycw);
-  float acc[BT];
-#pragma unroll
-  for (int b = 0; b < BT; ++b) acc[b] = 0.0f;
+  float acc[BT], sum[BT];
   ViewGeo vg = views[0];
   PixViewStart cur = pixel_view_start(g, vg, 0, edges, lines, pint, r, c, xcw, ycw);
-  for (int v = 0; v < g.V; ++v) {
-    const int vn = min(v + 1, g.V - 1);
-    const ViewGeo vgn = views[vn];
-    const PixViewStart nxt = pixel_view_start(g, vgn, vn, edges, lines, pint, r, c, xcw, ycw);
-    pixel_view_from<BT, WM>(g, vg, v, edges, cur, sino, r, c, b0, xcw, ycw, acc);
-    vg = vgn;
-    cur = nxt;
+  const int nc = walk_chunks(g.V);
+  for (int ch = 0, v = 0; ch < nc; ++ch) {
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[b] = 0.0f;
+    for (const int v1 = walk_chunk_begin(g.V, ch + 1); v < v1; ++v) {
+      const int vn = min(v + 1, g.V - 1);
+      const ViewGeo vgn = views[vn];
+      const PixViewStart nxt = pixel_view_start(g, vgn, vn, edges, lines, pint, r, c, xcw, ycw);
+      pixel_view_from<BT, WM>(g, vg, v, edges, cur, sino, r, c, b0, xcw, ycw, acc);
+      vg = vgn;
+      cur = nxt;
+    }
+#pragma unroll
+    for (int b = 0; b < BT; ++b) sum[b] = ch == 0 ? acc[b] : sum[b] + acc[b];
   }
 #pragma unroll
   for (int b = 0; b < BT; ++b)
     if (b0 + b < g.B) {
       const size_t at = (static_cast<size_t>(b0 + b) * g.H + r) * g.W + c;
-      out[at] = epi_value(ep, acc[b], at);
+      out[at] = epi_value(ep, sum[b], at);
     }
 }
 
-// Edge positions staged per (line of a pixel tile, view).
-template <int T>
-struct PixelTileLds {
-  static constexpr int kCap = 4 * T;  // staged edges per line
-  int klo[T];                 // first staged edge of each tile line
-  int n[T];                   // staged edges of each tile line
-  int first[T][T + 1];        // first staged edge with c >= i0 + j
-  int ec[T][kCap];            // edge_pos().c of staged edges
-  float ef[T][kCap];          // edge_pos().f of staged edges
-  int fallback[2];            // per view parity: window did not cover
+// ---------------------------------------------------------------------------
+// 3c. sinogram -> image: the staged walk, one wavefront per pixel tile
+// ---------------------------------------------------------------------------
+constexpr int kWalkW = 16;         // tile width in pixels (height 4 NP)
+constexpr int kWalkRangeH = 8;     // rows of one entry of the range table
+constexpr int kWalkSlots = 64;     // edge slots per view, one per lane
+constexpr int kWalkEdges = 60;     // edges a view may stage; the rest is padding
+constexpr float kWalkEarly = 0.0625f;  // bins a pixel's first bin is guessed early by
+
+__host__ __device__ inline int walk_range_tiles(const Geo2& g) {
+  return ((g.W + kWalkW - 1) / kWalkW) * ((g.H + kWalkRangeH - 1) / kWalkRangeH);
+}
+
+// First edge and edge count of one range entry (16 x 8 pixels of one view),
+// packed; 255: not to be staged.
+__device__ __forceinline__ unsigned pack_range(int2 r) {
+  const int n = r.y - r.x + 1;
+  return (static_cast<unsigned>(r.x) << 8) |
+         static_cast<unsigned>(n > kWalkSlots || r.x >= (1 << 24) ? 255 : n);
+}
+
+// Rows per lane of the staged walk (tiles of 16 x 4 rows pixels), or 0 where
+// the per-pixel kernel takes the op.  A taller tile shares each staged view
+// over more pixels, but its edges have to fit the slots: along its lines a
+// pixel spans at most `per_pixel` bins (pixel over bin at the image corner
+// next to the source), and views at 45 degrees add as many for each of its
+// rows.  From 2.8 bins per pixel on even 16 x 4 pixels do not fit and the
+// walk would fall back view after view.
+inline int walk_rows(const Geo2& g) {
+  const double px = fmax(std::fabs(g.dx), std::fabs(g.dy));
+  const double half = 0.5 * std::hypot(g.W * g.dx, g.H * g.dy) + std::hypot(g.shx, g.shy);
+  double per_pixel;
+  if (g.scan == DD_PARA) {
+    per_pixel = px / std::fabs(g.det);
+  } else {
+    const double near = g.sid - half;
+    if (!(near > 0.0)) return 0;
+    const double det = g.scan == DD_FAN_ARC ? g.sid * std::fabs(g.det)
+                                            : g.sid / g.sdd * std::fabs(g.det);
+    per_pixel = px * g.sid / near / det;
+  }
+  auto fits = [&](int rows) { return (kWalkW + 4 * rows) * per_pixel + 4.0 <= kWalkEdges; };
+  const int most = g.BT >= 8 ? 2 : 4;
+  if (fits(most)) return most;
+  if (fits(most / 2)) return most / 2;
+  return 0;
+}
+
+template <int BT>
+struct WalkLds {
+  double e[kWalkSlots];                    // bin edges from the tile's first on
+  double2 line[kWalkW];                    // {a0, 1 / P} of the tile's lines
+  float4 par[kWalkW];                      // {k0, k1, k2, P}: bin k0 + x (k1 + x k2) at tile pixel x
+  __align__(16) float q[BT * kWalkSlots];  // sinogram values, quad planes [BT / 4][bin][4]
 };
 
-// sinogram -> image for one kTile x kTile pixel tile, all views; every thread
-// of the block must call it (barriers).  Per view, the tile's lines get
-// their bin-edge positions computed once into LDS (instead of once per
-// pixel), a first-edge table is scattered from them, and each pixel reads
-// its bin range and overlaps from LDS.  The overlaps are the same edge_pos
-// values the forward kernel uses, so A^T stays the exact transpose of A.
-// A line whose staged window misses part of the tile takes the per-pixel
-// path for that view (same arithmetic, slower).
-template <int BT, int WM, int kTile>
-__device__ __forceinline__ void pixels_tile_body(
+// What a lane fetches for one view ahead of its turn.
+template <int BT>
+struct WalkFetch {
+  static constexpr int kQ = BT >= 8 ? BT / 2 : BT;  // values per lane
+  double e;
+  float q[kQ];
+  LineGeo lg;
+  float pl;
+};
+
+template <int BT>
+__device__ __forceinline__ void walk_load_q(const float* __restrict__ q, int k, float (&v)[BT]) {
+  if constexpr (BT >= 4) {
+#pragma unroll
+    for (int j = 0; j < BT / 4; ++j) {
+      const float4 t = *reinterpret_cast<const float4*>(q + (j * kWalkSlots + k) * 4);
+      v[4 * j] = t.x;
+      v[4 * j + 1] = t.y;
+      v[4 * j + 2] = t.z;
+      v[4 * j + 3] = t.w;
+    }
+  } else if constexpr (BT == 2) {
+    const float2 t = *reinterpret_cast<const float2*>(q + k * 2);
+    v[0] = t.x;
+    v[1] = t.y;
+  } else {
+    v[0] = q[k];
+  }
+}
+
+// Whether a pixel's window starts at its first bin exactly (one more edge to
+// place), or up to kWalkEarly before it (maybe one more bin to add, dear
+// where a bin holds many values).
+template <int BT>
+constexpr bool walk_shift() {
+  return BT >= 8;
+}
+
+// One staged view's bins for the tile: K bins per pixel from its first one on
+// (K = 0: kd of them), every pixel's independent of the others', so that
+// their LDS reads are in flight together.  Bins beside the pixel, and the
+// padding before and past the detector, have weight or value 0.  Clears `ok`
+// where a window does not hold the whole of a pixel inside the image.
+template <int BT, int WM, int NP, int K>
+__device__ __forceinline__ void walk_window(
+    const Geo2& g, const ViewGeo& vg, const WalkLds<BT>& s, int n, int i0, int px, int py,
+    const float (&xcw)[NP], const float (&ycw)[NP], const bool (&inside)[NP], int kd,
+    float (&acc)[NP][BT], bool& ok) {
+  constexpr int kTH = 4 * NP;
+  asm volatile("; window %0" ::"i"(K) : "memory");  // no code shared between the windows
+  // 16 values a bin: one bin after the other, or the loads that the scheduler
+  // moves ahead spill
+  constexpr bool kOneByOne = BT == 16;
+  const int bins = K > 0 ? K : kd;
+  const float klast = static_cast<float>(n - 2);
+  // row j of the lane: line li + j dli, tile pixel x + j dx
+  const int li = vg.xaxis ? py : px, dli = vg.xaxis ? 4 : 0;
+  const int x0 = vg.xaxis ? px : kTH - 1 - py, dx = vg.xaxis ? 0 : -4;
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const double2 lg = s.line[li + j * dli];
+    const float4 par = s.par[li + j * dli];
+    const PixelFrame fr(lg.x, lg.y, i0 + x0 + j * dx);
+    const float x = static_cast<float>(x0 + j * dx);
+    int k = static_cast<int>(
+        __builtin_amdgcn_fmed3f(fmaf(x, fmaf(x, par.z, par.y), par.x), 0.0f, klast));
+    float gw = (WM == W_FP) ? par.w : bp_const(g);
+    if constexpr (WM == W_BPW) gw *= fbp_weight(g, vg, xcw[j], ycw[j]);
+    float p0 = pixel_fraction(fr.at(s.e[k]));
+    float p1 = pixel_fraction(fr.at(s.e[k + 1]));
+    if constexpr (walk_shift<BT>()) {
+      // leave out a bin that ends before the pixel
+      const bool skip = p1 <= 0.0f;
+      k += skip;
+      p0 = skip ? p1 : p0;
+      p1 = pixel_fraction(fr.at(s.e[k + 1]));
+    }
+    const float first = p0;
+    auto add = [&](int m) {
+      const float w = (p1 - p0) * gw;
+      float q[BT];
+      walk_load_q<BT>(s.q, K > 0 ? k + m : min(k + m, kWalkSlots - 1), q);
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(w, q[b], acc[j][b]);
+      if constexpr (kOneByOne) __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (K > 0) {
+#pragma unroll
+      for (int m = 0; m < K; ++m) {
+        if (m > 0) {
+          p0 = p1;
+          p1 = pixel_fraction(fr.at(s.e[k + m + 1]));
+        }
+        add(m);
+      }
+    } else {
+      add(0);
+      for (int m = 1; m < bins; ++m) {
+        p0 = p1;
+        p1 = pixel_fraction(fr.at(s.e[min(k + m + 1, kWalkSlots - 1)]));
+        add(m);
+      }
+    }
+    ok = ok & ((p1 - first == 1.0f) | !inside[j]);
+    if constexpr (kOneByOne) asm volatile("; row %0" ::"i"(j) : "memory");
+  }
+}
+
+// Adds views [v0, v1) to the zeroed sums of the tile at (r0, c0): lane l owns
+// column c0 + l % 16 and rows r0 + l / 16 + 4 j.  Per view the bin edges and
+// sinogram values the tile can reach (range table) are staged in the
+// wavefront's own LDS (no barrier; the next view's are fetched during this
+// one), and every pixel takes its bins there: the first by a parabola through
+// the bins under three pixel edges of its line, then as many as a pixel can
+// meet at the view's bins per pixel (2 below one bin per pixel, 3 below two).
+// Bins, order, overlaps and products are pixel_one_view's, beside terms of
+// weight zero, so the sums are the same bit for bit.  If a view's range does
+// not fit, a window does not hold its pixel, or a sum is not finite at the
+// end (zero times an infinity is not zero), it returns false and the sums are
+// to be formed by walk_views_again.
+//
+// Bound by VALU issue (about 60 instructions per pixel and view at one
+// instance, two thirds of the cycles) and the LDS reads' latency.  The
+// per-pixel walk it replaces searched and placed three to five edges per
+// pixel in FP64 from global memory, one after the other, at about 200
+// instructions.  ProjTrans of 512 x 512 x 720 views x 736 bins: one slice
+// 1087 -> 372 us, 16 slices 1573 -> 760 us; 256 x 256 x 180 views parallel
+// 206 -> 43 us.
+template <int BT, int WM, int NP>
+__device__ __forceinline__ bool walk_views(
     const Geo2& g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
     const LineGeo* __restrict__ lines, const float* __restrict__ pint,
-    const float* __restrict__ sino, float* __restrict__ out, int tile_c, int tile_r,
-    int b0, PixelTileLds<kTile>& s,
-    const Epi& ep = Epi{}) {
-  constexpr int kEdgeCap = PixelTileLds<kTile>::kCap;
-  const int tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;
-  const int c0 = tile_c * kTile, r0 = tile_r * kTile;
-  const int c = c0 + tx, r = r0 + ty;
-  const bool inside = (c < g.W) && (r < g.H);
-  float xcw = 0.0f, ycw = 0.0f;
-  if constexpr (WM == W_BPW) pixel_centre(g, 1, r, c, &xcw, &ycw);
-  const float kbp = bp_const(g);
-  float acc[BT];
+    const unsigned* __restrict__ ranges, const float* __restrict__ sino, int r0, int c0, int b0,
+    int v0, int v1, float (&acc)[NP][BT], WalkLds<BT>& s) {
+  constexpr int kTH = 4 * NP;  // tile height
+  using F = WalkFetch<BT>;
+  int lane = static_cast<int>(threadIdx.x) & 63;
+  const int c = c0 + (lane & 15);
+  const int rtx = (g.W + kWalkW - 1) / kWalkW;
+  const int rty = (g.H + kWalkRangeH - 1) / kWalkRangeH;
+  const int rtiles = rtx * rty;
+  const size_t plane4 = static_cast<size_t>(g.V) * g.D * 4;
+  float xcw[NP] = {}, ycw[NP] = {};
+  if constexpr (WM == W_BPW) {
 #pragma unroll
-  for (int b = 0; b < BT; ++b) acc[b] = 0.0f;
-  if (threadIdx.x < 2) s.fallback[threadIdx.x] = 0;
-  __syncthreads();
-
-  for (int v = 0; v < g.V; ++v) {
-    const ViewGeo vg = views[v];
-    const int xaxis = vg.xaxis;
-    const int L = xaxis ? g.H : g.W;
-    const int N = xaxis ? g.W : g.H;
-    const int lbase = xaxis ? r0 : c0;
-    const int i0 = xaxis ? c0 : g.H - kTile - r0;
-    const int par = v & 1;
-    const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
-    const LineGeo* __restrict__ lv = lines + static_cast<size_t>(v) * g.Lmax;
-    // A: staged edge window of each tile line
-    if (threadIdx.x == 0) s.fallback[par ^ 1] = 0;
-    if (threadIdx.x < kTile) {
-      const int la = lbase + threadIdx.x;
-      int klo = 0, n = 0;
-      if (la < L) {
-        const LineGeo lg = lv[la];
-        const double p = static_cast<double>(pint[static_cast<size_t>(v) * g.Lmax + la]);
-        const int k0 = guess_bin_fast(g, vg, lg.a0 + i0 * p) - 2;
-        const int k1 = guess_bin_fast(g, vg, lg.a0 + (i0 + kTile) * p) + 3;
-        klo = min(max(k0, 0), g.D);
-        const int khi = min(max(k1, klo), g.D);
-        n = khi - klo + 1;
-        if (n > kEdgeCap) {
-          n = kEdgeCap;
-          s.fallback[par] = 1;
-        }
-      }
-      s.klo[threadIdx.x] = klo;
-      s.n[threadIdx.x] = n;
-#pragma unroll
-      for (int j = 0; j <= kTile; ++j) s.first[threadIdx.x][j] = n;
-    }
-    __syncthreads();
-    // B: edge positions of every staged edge, and the window checks
-    for (int idx = threadIdx.x; idx < kTile * kEdgeCap; idx += blockDim.x) {
-      const int ll = idx / kEdgeCap, e = idx % kEdgeCap;
-      const int n = s.n[ll];
-      if (e >= n) continue;
-      const int klo = s.klo[ll];
-      const LineGeo lg = lv[lbase + ll];
-      const EdgePos ep = edge_pos(ev[klo + e], lg.a0, lg.inv_p, N);
-      s.ec[ll][e] = ep.c;
-      s.ef[ll][e] = ep.f;
-      // the window must start before the tile's first real pixel and end
-      // after its last one, unless it reaches the detector's end
-      if (e == 0 && klo > 0 && ep.c >= max(i0, 0)) s.fallback[par] = 1;
-      if (e == n - 1 && klo + e < g.D && ep.c < min(i0 + kTile, N)) s.fallback[par] = 1;
-    }
-    __syncthreads();
-    // C: first staged edge at or after each pixel edge of the tile
-    for (int idx = threadIdx.x; idx < kTile * kEdgeCap; idx += blockDim.x) {
-      const int ll = idx / kEdgeCap, e = idx % kEdgeCap;
-      if (e >= s.n[ll]) continue;
-      const int ce = s.ec[ll][e];
-      const int cp = (e == 0) ? -(1 << 30) : s.ec[ll][e - 1];
-      const int jlo = max(cp + 1 - i0, 0), jhi = min(ce - i0, kTile);
-      for (int j = jlo; j <= jhi; ++j) s.first[ll][j] = e;
-    }
-    __syncthreads();
-    // D: accumulate
-    if (inside) {
-      if (!s.fallback[par]) {
-        const int ll = xaxis ? ty : tx;
-        const int j = xaxis ? tx : (kTile - 1 - ty);
-        const int i = i0 + j;
-        const int klo = s.klo[ll], n = s.n[ll];
-        const int e0 = max(s.first[ll][j] - 1, 0);
-        const int e1 = min(s.first[ll][j + 1] - 1, n - 2);
-        float gw = (WM == W_FP) ? pint[static_cast<size_t>(v) * g.Lmax + lbase + ll] : kbp;
-        if constexpr (WM == W_BPW) gw *= fbp_weight(g, vg, xcw, ycw);
-        const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
-        for (int e = e0; e <= e1; ++e) {
-          const EdgePos p1{s.ec[ll][e], s.ef[ll][e]};
-          const EdgePos p2{s.ec[ll][e + 1], s.ef[ll][e + 1]};
-          const float w = overlap_in_pixel(p1, p2, i) * gw;
-          float q[BT];
-          load_sino<BT>(g, sv, klo + e, q);
-#pragma unroll
-          for (int b = 0; b < BT; ++b) acc[b] = fmaf(w, q[b], acc[b]);
-        }
-      } else {
-        pixel_one_view<BT, WM>(g, vg, v, edges, lines, pint, sino, r, c, b0, xcw, ycw, acc);
-      }
-    }
-    __syncthreads();
+    for (int j = 0; j < NP; ++j)
+      pixel_centre(g, 1, r0 + (lane >> 4) + 4 * j, c, &xcw[j], &ycw[j]);
   }
-  if (inside) {
+  bool inside[NP];
 #pragma unroll
-    for (int b = 0; b < BT; ++b)
-      if (b0 + b < g.B) {
-        const size_t at = (static_cast<size_t>(b0 + b) * g.H + r) * g.W + c;
-        out[at] = epi_value(ep, acc[b], at);
+  for (int j = 0; j < NP; ++j) inside[j] = c < g.W && r0 + (lane >> 4) + 4 * j < g.H;
+  // first edge and edge count of view v's range over the whole tile; a range
+  // at the detector's start gets a padding edge before it
+  auto range_of = [&](int v, int* kb) {
+    const unsigned* __restrict__ rv =
+        ranges + static_cast<size_t>(v) * rtiles + (r0 / kWalkRangeH) * rtx + c0 / kWalkW;
+    unsigned w = const_load(rv);
+    int lo = static_cast<int>(w >> 8), n = static_cast<int>(w & 255u), hi = lo + n;
+    bool big = n == 255;
+#pragma unroll
+    for (int y = 1; y < (kTH + kWalkRangeH - 1) / kWalkRangeH; ++y) {
+      w = const_load(rv + (r0 / kWalkRangeH + y < rty ? y * rtx : 0));
+      const int l2 = static_cast<int>(w >> 8), n2 = static_cast<int>(w & 255u);
+      big = big || n2 == 255;
+      lo = min(lo, l2);
+      hi = max(hi, l2 + n2);
+    }
+    if (lo == 0) lo = -1;
+    *kb = lo;
+    return big ? 255 : hi - lo;
+  };
+  auto load_quads = [&](const float* sv, int k, float* q) {  // BT >= 8: half the planes
+#pragma unroll
+    for (int m = 0; m < BT / 8; ++m) {
+      const float4 t = *reinterpret_cast<const float4*>(
+          sv + (2 * m + (lane >> 5)) * plane4 + static_cast<size_t>(k) * 4);
+      q[4 * m] = t.x;
+      q[4 * m + 1] = t.y;
+      q[4 * m + 2] = t.z;
+      q[4 * m + 3] = t.w;
+    }
+  };
+  auto store_quads = [&](int slot, const float* q) {
+#pragma unroll
+    for (int m = 0; m < BT / 8; ++m)
+      *reinterpret_cast<float4*>(s.q + ((2 * m + (lane >> 5)) * kWalkSlots + slot) * 4) =
+          make_float4(q[4 * m], q[4 * m + 1], q[4 * m + 2], q[4 * m + 3]);
+  };
+  auto fetch = [&](const ViewGeo& vg, int v, int kb, int n, F& f) {
+    const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
+    const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
+    // padding lies before or past every pixel
+    f.e = kb + lane < 0 ? -1e300 : 1e300;
+    if (kb + lane >= 0 && lane < n) f.e = ev[kb + lane];
+#pragma unroll
+    for (int b = 0; b < F::kQ; ++b) f.q[b] = 0.0f;
+    if constexpr (BT >= 8) {
+      const int bin = lane & 31;
+      if (kb + bin >= 0 && bin < n - 1) load_quads(sv, kb + bin, f.q);
+    } else {
+      if (kb + lane >= 0 && lane < n - 1)
+        load_tile<BT>(sv + static_cast<size_t>(kb + lane) * g.Bp, f.q);
+    }
+    const int l = vg.xaxis ? min(r0 + (lane & 15), g.H - 1) : min(c0 + (lane & 15), g.W - 1);
+    f.lg = lines[static_cast<size_t>(v) * g.Lmax + l];
+    f.pl = pint[static_cast<size_t>(v) * g.Lmax + l];
+  };
+  bool ok = true;
+  int kb = 0;
+  ViewGeo vg = views[v0];
+  int n = range_of(v0, &kb);
+  F f;
+  if (n <= kWalkEdges) fetch(vg, v0, kb, n, f);
+  for (int v = v0; v < v1; ++v) {
+    const int vn = min(v + 1, v1 - 1);
+    const ViewGeo vgn = views[vn];
+    int kbn = 0;
+    const int nn = range_of(vn, &kbn);
+    if (n > kWalkEdges || nn > kWalkEdges) {
+      ok = false;
+      break;
+    }
+    // what follows from the lane alone is cheaper formed again than kept in
+    // registers over the views
+    asm volatile("" : "+v"(lane));
+    const int px = lane & 15, py = lane >> 4;
+    // stage the view
+    const int i0 = vg.xaxis ? c0 : g.H - r0 - kTH;  // the tile's first pixel on its lines
+    s.e[lane] = f.e;
+    if constexpr (BT >= 8) {
+      store_quads(lane & 31, f.q);
+      float q[F::kQ] = {};
+      if (n > 32) {  // bins 32 on, not fetched ahead
+        if (32 + (lane & 31) < n - 1)
+          load_quads(sino_view<BT>(g, sino, v, b0), kb + 32 + (lane & 31), q);
+        store_quads(32 + (lane & 31), q);
+      } else if ((lane & 31) < 4) {
+        store_quads(32 + (lane & 31), q);
       }
+    } else if constexpr (BT == 4) {
+      *reinterpret_cast<float4*>(s.q + lane * 4) = make_float4(f.q[0], f.q[1], f.q[2], f.q[3]);
+    } else {
+#pragma unroll
+      for (int b = 0; b < BT; ++b) s.q[lane * BT + b] = f.q[b];
+    }
+    // the bins under each line's first, middle and last pixel edge in the
+    // tile, and the parabola through them (off by hundredths of a bin)
+    const int span = vg.xaxis ? kWalkW : kTH;
+    const float inv = vg.xaxis ? 1.0f / kWalkW : 1.0f / kTH;
+    const float k0 = guess_bin_real(
+        g, vg, f.lg.a0 + (i0 + py * (span / 2)) * static_cast<double>(f.pl));
+    const float km = __shfl_down(k0, 16), k1 = __shfl_down(k0, 32);
+    const float b1 = (4.0f * km - 3.0f * k0 - k1) * inv;
+    const float b2 = 2.0f * (k0 - 2.0f * km + k1) * inv * inv;
+    float slope = 0.0f;  // most bins per pixel on the line
+    if (lane < 16) {
+      slope = fmaxf(b1, fmaf(2.0f * span, b2, b1));
+      s.line[lane] = make_double2(f.lg.a0, f.lg.inv_p);
+      s.par[lane] = make_float4(k0 - static_cast<float>(kb) - kWalkEarly, b1, b2, f.pl);
+    }
+    if (v + 1 < v1) fetch(vgn, vn, kbn, nn, f);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // bins of a pixel: those its extent (and an early start) can cross
+    constexpr float kSlack = walk_shift<BT>() ? 0.03125f : 2 * kWalkEarly;
+    if (__all(slope < 1.0f - kSlack))
+      walk_window<BT, WM, NP, 2>(g, vg, s, n, i0, px, py, xcw, ycw, inside, 0, acc, ok);
+    else if (__all(slope < 2.0f - kSlack))
+      walk_window<BT, WM, NP, 3>(g, vg, s, n, i0, px, py, xcw, ycw, inside, 0, acc, ok);
+    else {
+      int kd = 4;
+      while (kd < kWalkEdges && !__all(slope < kd - 1 - kSlack)) ++kd;
+      walk_window<BT, WM, NP, 0>(g, vg, s, n, i0, px, py, xcw, ycw, inside, kd, acc, ok);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    vg = vgn;
+    kb = kbn;
+    n = nn;
+  }
+#pragma unroll
+  for (int j = 0; j < NP; ++j)
+#pragma unroll
+    for (int b = 0; b < BT; ++b) ok = ok & (fabsf(acc[j][b]) < __builtin_inff());
+  return __all(ok);
+}
+
+// The tile's sums of views [v0, v1) by pixel_one_view, chunk by chunk, given
+// to put(row, value index, sum): what walk_views could not do.
+template <int BT, int WM, int NP, typename Put>
+__device__ __forceinline__ void walk_views_again(
+    const Geo2& g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
+    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
+    const float* __restrict__ sino, int r0, int c0, int b0, int ch0, int ch1, Put put) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int c = c0 + (lane & 15);
+#pragma unroll 1
+  for (int j = 0; j < NP; ++j) {
+    const int r = r0 + (lane >> 4) + 4 * j;
+    if (c >= g.W || r >= g.H) continue;
+    float xc = 0.0f, yc = 0.0f, sum[BT];
+    if constexpr (WM == W_BPW) pixel_centre(g, 1, r, c, &xc, &yc);
+#pragma unroll 1
+    for (int ch = ch0; ch < ch1; ++ch) {
+      float acc[BT];
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc[b] = 0.0f;
+      const int v1 = walk_chunk_begin(g.V, ch + 1);
+#pragma unroll 1
+      for (int v = walk_chunk_begin(g.V, ch); v < v1; ++v)
+        pixel_one_view<BT, WM>(g, views[v], v, edges, lines, pint, sino, r, c, b0, xc, yc, acc);
+#pragma unroll
+      for (int b = 0; b < BT; ++b) sum[b] = ch == ch0 ? acc[b] : sum[b] + acc[b];
+    }
+#pragma unroll
+    for (int b = 0; b < BT; ++b) put(r, c, b, sum[b]);
   }
 }
 

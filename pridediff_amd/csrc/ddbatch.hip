@@ -42,7 +42,7 @@ using namespace body2d;
 // (pointers read from memory would otherwise be generic: flat loads).
 enum Region {
   kViews, kEdges, kWfp, kLines, kPint, kXrow, kXcol, kSino, kPart, kPrefRow, kPrefCol,
-  kPrefSino, kKnotRange, kRegions
+  kPrefSino, kKnotRange, kWalkRange, kWalkPart, kRegions
 };
 
 enum Phase {
@@ -51,13 +51,16 @@ enum Phase {
   kLayoutSino = 2,
   kGatherPixels = 3,
   kReduceBins = 4,
-  kGatherQuads = 5,   // sinogram -> image with one thread per 4 x 4 pixels
+  kGatherQuads = 5,   // running-sum sinogram -> image, one thread per 4 x 4 pixels
   kLayoutPrefix = 6,  // running sums of every image row and column
-  kPhases = 7
+  kSumPixels = 7,     // staged walk: partial images of the view chunks
+  kPhases = 8
 };
 
 struct BatchDesc {
   Geo2 g;
+  int rows;    // rows per lane of the staged walk, 0: per-pixel gather
+  int chunks;  // workgroups the views of a pixel tile are split over
   unsigned long long off[kRegions];
   long long img_off;   // floats, into the packed image buffer
   long long sino_off;  // floats, into the packed sinogram buffer
@@ -68,6 +71,7 @@ struct BatchDesc {
 // One instance inside a kernel: the descriptor with typed pointers.
 struct BatchInst {
   Geo2 g;
+  int rows, chunks;
   ViewGeo* views;
   double* edges;
   float* wfp;
@@ -80,6 +84,8 @@ struct BatchInst {
   float4* prow;        // running sums of the rows [B][H][W + 1]
   float4* pcol;        // running sums of the columns, bottom-up [B][W][H + 1]
   double2* psino;      // running-sum knots over the bins per view [B][V][D + 1]
+  unsigned* wrange;    // edges each 16 x 8 pixel tile needs, per view
+  float* wpart;        // partial images [chunks][H][W] of the staged walk
   int2* krange;        // knots each 64 x 64 pixel tile needs, per view [V][tiles]
   long long img_off;
   long long sino_off;
@@ -87,12 +93,9 @@ struct BatchInst {
 
 constexpr int kBT = 1;  // one geometry per instance
 
-// Block items of the DD_ADJ_QUAD variant: one thread per kBlockQ x kBlockQ
-// pixel block (one first-bin search and one bin walk per line serve kBlockQ
-// pixels), kQuadSide x kQuadSide threads per item.  Measured on 64 uneven
-// instances: adjoint 17.4 / 16.4 / 14.7 / 17.6 / 21.0 ms for blocks of 2 / 3
-// / 4 / 5 / 6 (register pressure past 4); items of 8 x 8 threads (32 x 32
-// pixels) instead of 16 x 16: 13.9 vs 13.6 ms.
+// Block items of the running-sum adjoint: one thread per kBlockQ x kBlockQ
+// pixel block (one first-bin search and one merge walk per line serve kBlockQ
+// pixels), kQuadSide x kQuadSide threads per item.
 constexpr int kBlockQ = 4;
 constexpr int kQuadSide = 16;
 constexpr int kQuadThreads = kQuadSide * kQuadSide;
@@ -113,6 +116,10 @@ __device__ __forceinline__ BatchInst load_inst(char* __restrict__ mem, int i) {
   const BatchDesc& s = reinterpret_cast<const BatchDesc*>(mem)[i];
   BatchInst d;
   d.g = s.g;
+  d.rows = s.rows;
+  d.chunks = s.chunks;
+  d.wrange = reinterpret_cast<unsigned*>(mem + s.off[kWalkRange]);
+  d.wpart = reinterpret_cast<float*>(mem + s.off[kWalkPart]);
   d.views = reinterpret_cast<ViewGeo*>(mem + s.off[kViews]);
   d.edges = reinterpret_cast<double*>(mem + s.off[kEdges]);
   d.wfp = reinterpret_cast<float*>(mem + s.off[kWfp]);
@@ -155,7 +162,8 @@ __global__ __launch_bounds__(kThreads) void k_batch_setup(
 }
 
 // Per (instance, view): the knot range every 64 x 64 pixel tile of the
-// block items needs (knot_range), for the LDS staging of k_batch_quads_prefix.
+// block items needs (knot_range), for the LDS staging of k_batch_quads_prefix,
+// and the edge range of every 16 x 8 pixels for the staged walk.
 __global__ __launch_bounds__(kThreads) void k_batch_ranges(char* __restrict__ mem, int n_inst,
                                                            int total) {
   const BatchDesc* __restrict__ desc = reinterpret_cast<const BatchDesc*>(mem);
@@ -176,6 +184,14 @@ __global__ __launch_bounds__(kThreads) void k_batch_ranges(char* __restrict__ me
           d.g, vg, d.edges + static_cast<size_t>(v) * (d.g.D + 1),
           d.lines + static_cast<size_t>(v) * d.g.Lmax, r0, min(r0 + kQuadTile, d.g.H), c0,
           min(c0 + kQuadTile, d.g.W));
+    }
+    const int wtx = (d.g.W + kWalkW - 1) / kWalkW, wtiles = walk_range_tiles(d.g);
+    for (int t = threadIdx.x; t < wtiles; t += blockDim.x) {
+      const int c0 = (t % wtx) * kWalkW, r0 = (t / wtx) * kWalkRangeH;
+      d.wrange[static_cast<size_t>(v) * wtiles + t] = pack_range(knot_range(
+          d.g, vg, d.edges + static_cast<size_t>(v) * (d.g.D + 1),
+          d.lines + static_cast<size_t>(v) * d.g.Lmax, r0, min(r0 + kWalkRangeH, d.g.H), c0,
+          min(c0 + kWalkW, d.g.W)));
     }
   }
 }
@@ -306,28 +322,85 @@ __global__ __launch_bounds__(kThreads) void k_batch_reduce(
   }
 }
 
+// One wavefront's share of a gather-pixels item: the staged walk of one pixel
+// tile, over one view chunk (several workgroups per tile) or all of them.
+template <int WM, int NP>
+__device__ __forceinline__ void batch_walk_tile(const BatchInst& d, int tile, int chunk,
+                                                float* __restrict__ out, WalkLds<kBT>& lds) {
+  const int tx = (d.g.W + kWalkW - 1) / kWalkW;
+  const int c0 = (tile % tx) * kWalkW, r0 = (tile / tx) * 4 * NP;
+  const int nc = walk_chunks(d.g.V);
+  const int ch0 = d.chunks > 1 ? chunk : 0, ch1 = d.chunks > 1 ? chunk + 1 : nc;
+  float* __restrict__ o =
+      d.chunks > 1 ? d.wpart + static_cast<size_t>(chunk) * d.g.H * d.g.W : out + d.img_off;
+  auto put = [&](int r, int c, int, float v) {
+    if (c < d.g.W && r < d.g.H) o[static_cast<size_t>(r) * d.g.W + c] = v;
+  };
+  float acc[NP][kBT], sum[NP];
+  for (int ch = ch0; ch < ch1; ++ch) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j) acc[j][0] = 0.0f;
+    if (!walk_views<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.wrange, d.sino, r0,
+                                 c0, 0, walk_chunk_begin(d.g.V, ch),
+                                 walk_chunk_begin(d.g.V, ch + 1), acc, lds)) {
+      walk_views_again<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, r0, c0, 0,
+                                    ch0, ch1, put);
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < NP; ++j) sum[j] = ch == ch0 ? acc[j][0] : sum[j] + acc[j][0];
+  }
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+#pragma unroll
+  for (int j = 0; j < NP; ++j) put(r0 + (lane >> 4) + 4 * j, c0 + (lane & 15), 0, sum[j]);
+}
+
+// Gather-pixels items: (four pixel tiles, view chunk) of the staged walk, or
+// 16 x 16 pixels of the per-pixel gather where an instance's bins are too
+// fine to be staged.
 template <int WM>
-__global__ __launch_bounds__(kThreads) void k_batch_pixels(
-    char* __restrict__ mem, int n_inst, int total, float* __restrict__ out,
-    int per_pixel) {
-  __shared__ PixelTileLds<kTile> lds;
+__global__ __launch_bounds__(kThreads) void k_batch_walk(
+    char* __restrict__ mem, int n_inst, int total, float* __restrict__ out) {
+  __shared__ WalkLds<kBT> lds[kThreads / 64];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
   for (int item = blockIdx.x; item < total; item += gridDim.x) {
     const int i = find_inst(mem, n_inst, kGatherPixels, item);
     const BatchInst d = load_inst(mem, i);
     const int local = item - item0_of(mem, i, kGatherPixels);
-    const int tx = (d.g.W + kTile - 1) / kTile, ty = (d.g.H + kTile - 1) / kTile;
-    const int t = local % (tx * ty);
-    const int b0 = (local / (tx * ty)) * kBT;
-    if (per_pixel) {
-      const int c = (t % tx) * kTile + (threadIdx.x % kTile);
-      const int r = (t / tx) * kTile + (threadIdx.x / kTile);
+    if (d.rows > 0) {
+      const int chunk = local % d.chunks;
+      const int tile = (local / d.chunks) * (kThreads / 64) + wave;
+      const int th = 4 * d.rows;
+      if (tile >= ((d.g.W + kWalkW - 1) / kWalkW) * ((d.g.H + th - 1) / th)) continue;
+      if (d.rows == 4)
+        batch_walk_tile<WM, 4>(d, tile, chunk, out, lds[wave]);
+      else
+        batch_walk_tile<WM, 2>(d, tile, chunk, out, lds[wave]);
+    } else {
+      const int tx = (d.g.W + kTile - 1) / kTile;
+      const int c = (local % tx) * kTile + (threadIdx.x % kTile);
+      const int r = (local / tx) * kTile + (threadIdx.x / kTile);
       if (c < d.g.W && r < d.g.H)
         pixels_body<kBT, WM>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, out + d.img_off,
-                             r, c, b0);
-    } else {
-      pixels_tile_body<kBT, WM, kTile>(d.g, d.views, d.edges, d.lines, d.pint, d.sino,
-                                       out + d.img_off, t % tx, t / tx, b0, lds);
+                             r, c, 0);
     }
+  }
+}
+
+// Sum items: 256 pixels of an instance whose views were split, chunk sums in
+// chunk order.
+__global__ __launch_bounds__(kThreads) void k_batch_sum(
+    char* __restrict__ mem, int n_inst, int total, float* __restrict__ out) {
+  for (int item = blockIdx.x; item < total; item += gridDim.x) {
+    const int i = find_inst(mem, n_inst, kSumPixels, item);
+    const BatchInst d = load_inst(mem, i);
+    const size_t n = static_cast<size_t>(d.g.H) * d.g.W;
+    const size_t at = static_cast<size_t>(item - item0_of(mem, i, kSumPixels)) * kThreads +
+                      threadIdx.x;
+    if (at >= n) continue;
+    float s = d.wpart[at];
+    for (int c = 1; c < d.chunks; ++c) s += d.wpart[c * n + at];
+    out[d.img_off + at] = s;
   }
 }
 
@@ -426,28 +499,6 @@ __attribute__((amdgpu_waves_per_eu(5))) void k_batch_quads_prefix(
   }
 }
 
-// Block items: (instance, 64 x 64 pixel tile), one thread per 4 x 4 pixels;
-// KW > 0 reads each line's bins as one window of KW bins.
-template <int WM, int KW>
-__global__ __launch_bounds__(kQuadThreads)
-__attribute__((amdgpu_waves_per_eu(KW > 0 ? 4 : 1))) void k_batch_quads(
-    char* __restrict__ mem, int n_inst, int total, float* __restrict__ out) {
-  for (int item = blockIdx.x; item < total; item += gridDim.x) {
-    const int i = find_inst(mem, n_inst, kGatherQuads, item);
-    const BatchInst d = load_inst(mem, i);
-    const int local = item - item0_of(mem, i, kGatherQuads);
-    const int tx = (d.g.W + kQuadTile - 1) / kQuadTile;
-    const int ty = (d.g.H + kQuadTile - 1) / kQuadTile;
-    const int t = local % (tx * ty);
-    const int b0 = (local / (tx * ty)) * kBT;
-    const int c0 = (t % tx) * kQuadTile + kBlockQ * (threadIdx.x % kQuadSide);
-    const int r0 = (t / tx) * kQuadTile + kBlockQ * (threadIdx.x / kQuadSide);
-    if (c0 < d.g.W && r0 < d.g.H)
-      blocks_body<kBT, WM, kBlockQ, KW>(d.g, d.views, d.edges, d.lines, d.pint, d.sino,
-                                        out + d.img_off, r0, c0, b0);
-  }
-}
-
 }  // namespace
 }  // namespace dd
 
@@ -461,7 +512,7 @@ struct dd2d_batch {
   size_t total_views = 0;
   int total[kPhases] = {};
   int grid = 0;                  // workgroups per launch (0 = one per work item)
-  int variant = DD_ADJ_QUAD;     // sinogram -> image kernel (per pixel, 16x16 tiles, 4x4 blocks)
+  bool prefix = false;           // sinogram -> image through running sums (DD_ADJ_BLOCK_PREFIX)
   bool fwd_prefix = false;       // image -> sinogram through running sums (DD_FWD_PREFIX)
   char* dev = nullptr;           // device memory given to setup()
 };
@@ -483,23 +534,9 @@ int grid_for(const dd2d_batch* b, int total) {
   return std::max(1, std::min(g, total));
 }
 
-// Bins per window of DD_ADJ_BLOCK_WINDOW: a 4-pixel run meets up to ~6 bins
-// of these geometries, so 8 rarely leaves a bin to the serial tail.
-constexpr int kBlockWindow = 8;
-
-template <int KW>
-void launch_quads(const dd2d_batch* b, int op, char* inst, int n, int qt, float* output,
-                  hipStream_t st) {
-  if (op == DD_PROJ_T)
-    hipLaunchKernelGGL((k_batch_quads<W_FP, KW>), dim3(grid_for(b, qt)), dim3(kQuadThreads), 0,
-                       st, inst, n, qt, output);
-  else if (op == DD_BPROJ)
-    hipLaunchKernelGGL((k_batch_quads<W_BP, KW>), dim3(grid_for(b, qt)), dim3(kQuadThreads), 0,
-                       st, inst, n, qt, output);
-  else
-    hipLaunchKernelGGL((k_batch_quads<W_BPW, KW>), dim3(grid_for(b, qt)), dim3(kQuadThreads), 0,
-                       st, inst, n, qt, output);
-}
+// Largest partial images of a whole batch that its pixel tiles are split over
+// their view chunks for (as in one-call ops: what the Infinity Cache holds).
+constexpr unsigned long long kWalkPartBytes = 256ull << 20;
 
 }  // namespace
 
@@ -532,6 +569,11 @@ dd2d_batch* dd2d_batch_create(const dd2d_batch_item* items, int n) {
   b->desc_off = take(&off, sizeof(BatchDesc) * n);  // 0: kernels find it at the block base
   b->angles_off = take(&off, sizeof(float*) * n);
   b->inst.resize(n);
+  // staged walk: partial images of the whole batch
+  unsigned long long parts = 0;
+  for (int j = 0; j < n; ++j)
+    parts += sizeof(float) * 1ull * walk_chunks(items[j].views) * items[j].geom.width *
+             items[j].geom.height * items[j].batch;
   int acc[kPhases] = {};
   for (int j = 0; j < n; ++j) {
     const auto& it = items[b->order[j]];
@@ -575,6 +617,11 @@ dd2d_batch* dd2d_batch_create(const dd2d_batch_item* items, int n) {
     d.off[kKnotRange] = take(&off, sizeof(int2) * static_cast<size_t>(g.V) *
                                        ((g.W + kQuadTile - 1) / kQuadTile) *
                                        ((g.H + kQuadTile - 1) / kQuadTile));
+    d.rows = walk_rows(g);
+    d.chunks = d.rows > 0 && parts <= kWalkPartBytes ? walk_chunks(g.V) : 1;
+    d.off[kWalkRange] = take(&off, sizeof(unsigned) * g.V * walk_range_tiles(g));
+    d.off[kWalkPart] =
+        d.chunks > 1 ? take(&off, sizeof(float) * static_cast<size_t>(d.chunks) * img) : 0;
     d.img_off = it.image_offset;
     d.sino_off = it.sino_offset;
     const int tiles = it.batch;  // kBT == 1
@@ -584,7 +631,13 @@ dd2d_batch* dd2d_batch_create(const dd2d_batch_item* items, int n) {
     d.nitems[kGatherQuads] =
         ((g.W + kQuadTile - 1) / kQuadTile) * ((g.H + kQuadTile - 1) / kQuadTile) * tiles;
     d.nitems[kLayoutSino] = g.V * tiles;
-    d.nitems[kGatherPixels] = ((g.W + kTile - 1) / kTile) * ((g.H + kTile - 1) / kTile) * tiles;
+    if (d.rows > 0) {
+      const int wt = ((g.W + kWalkW - 1) / kWalkW) * ((g.H + 4 * d.rows - 1) / (4 * d.rows));
+      d.nitems[kGatherPixels] = (wt + 3) / 4 * d.chunks * tiles;
+    } else {
+      d.nitems[kGatherPixels] = ((g.W + kTile - 1) / kTile) * ((g.H + kTile - 1) / kTile) * tiles;
+    }
+    d.nitems[kSumPixels] = d.chunks > 1 ? (g.W * g.H + kThreads - 1) / kThreads * tiles : 0;
     d.nitems[kLayoutPrefix] = (g.H + g.W) * tiles;
     for (int ph = 0; ph < kPhases; ++ph) {
       d.item0[ph] = acc[ph];
@@ -606,11 +659,7 @@ void dd2d_batch_set_grid(dd2d_batch* b, int workgroups) {
 
 void dd2d_batch_set_variant(dd2d_batch* b, int variant) {
   if (!b) return;
-  const int adj = variant & ~DD_FWD_PREFIX;
-  b->variant = (adj == DD_ADJ_TILE16 || adj == DD_ADJ_QUAD || adj == DD_ADJ_BLOCK_WINDOW ||
-                adj == DD_ADJ_BLOCK_PREFIX)
-                   ? adj
-                   : DD_ADJ_PER_PIXEL;
+  b->prefix = (variant & ~DD_FWD_PREFIX) == DD_ADJ_BLOCK_PREFIX;
   b->fwd_prefix = (variant & DD_FWD_PREFIX) != 0;
 }
 
@@ -691,7 +740,7 @@ dd_status dd2d_batch_run(const dd2d_batch* b, int op, const float* input, float*
                          st, inst, n, rtot, output);
     }
   } else {
-    if (b->variant == DD_ADJ_BLOCK_PREFIX && op != DD_BPROJ_W) {
+    if (b->prefix && op != DD_BPROJ_W) {
       // running sums of every view, then one merge walk per 4-pixel run
       ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
       const int lt = b->total[kLayoutSino], qt = b->total[kGatherQuads];
@@ -718,25 +767,19 @@ dd_status dd2d_batch_run(const dd2d_batch* b, int op, const float* input, float*
                          dim3(kThreads), 0, st, inst, n, static_cast<int>(kLayoutSino),
                          b->total[kLayoutSino], input);
     ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
-    if (b->variant == DD_ADJ_QUAD || b->variant == DD_ADJ_BLOCK_WINDOW ||
-        b->variant == DD_ADJ_BLOCK_PREFIX) {
-      const int qt = b->total[kGatherQuads];
-      if (b->variant == DD_ADJ_QUAD)
-        launch_quads<0>(b, op, inst, n, qt, output, st);
-      else  // DD_ADJ_BLOCK_WINDOW, and BPROJ_W of DD_ADJ_BLOCK_PREFIX
-        launch_quads<kBlockWindow>(b, op, inst, n, qt, output, st);
-      return hipGetLastError() == hipSuccess ? DD_OK : DD_LAUNCH_FAIL;
-    }
-    const int tot = b->total[kGatherPixels];
+    const int tot = b->total[kGatherPixels], stot = b->total[kSumPixels];
     if (op == DD_PROJ_T)
-      hipLaunchKernelGGL((k_batch_pixels<W_FP>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
-                         inst, n, tot, output, b->variant != DD_ADJ_TILE16);
+      hipLaunchKernelGGL((k_batch_walk<W_FP>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
+                         inst, n, tot, output);
     else if (op == DD_BPROJ)
-      hipLaunchKernelGGL((k_batch_pixels<W_BP>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
-                         inst, n, tot, output, b->variant != DD_ADJ_TILE16);
+      hipLaunchKernelGGL((k_batch_walk<W_BP>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
+                         inst, n, tot, output);
     else
-      hipLaunchKernelGGL((k_batch_pixels<W_BPW>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
-                         inst, n, tot, output, b->variant != DD_ADJ_TILE16);
+      hipLaunchKernelGGL((k_batch_walk<W_BPW>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
+                         inst, n, tot, output);
+    if (stot > 0)
+      hipLaunchKernelGGL(k_batch_sum, dim3(grid_for(b, stot)), dim3(kThreads), 0, st, inst, n,
+                         stot, output);
   }
   return hipGetLastError() == hipSuccess ? DD_OK : DD_LAUNCH_FAIL;
 }
