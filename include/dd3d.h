@@ -62,25 +62,28 @@ dd_status dd3d_run(int scan, int op, const dd_geom3d* g, const float* input,
                    int batch, int views, void* ws, size_t ws_bytes,
                    void* stream);
 
-/* Running sums over detector rows of the sinogram -> volume ops:
- *   1: compensated FP32 pairs (hi + lo, plus each row's own value), so every
- *      slice's sum is rounded relative to the slice;
- *   0: rounded to FP32 (a third of the workspace; error relative to the
- *      whole running sum, i.e. growing with the number of detector rows);
- *   2 (default, and any other value): compensated when the instance tile is
- *      1 or 2 (no extra load per evaluation), rounded at tile 4 (batches of
- *      3 or more), where the compensated gather needs a third 16-byte load.
+/* How the sinogram -> volume ops sum detector rows:
+ *   2 (default, and any other value): row by row, each weighted by its
+ *      overlap with the slice, where a slice is at most 3 rows thick and the
+ *      detector's columns are not much finer than the pixels; otherwise by
+ *      running sums, compensated when the instance tile is 1 or 2 (no extra
+ *      load per evaluation), rounded at tile 4 (batches of 3 or more);
+ *   1: compensated running sums, FP32 pairs (hi + lo, plus each row's own
+ *      value), so every slice's sum is rounded relative to the slice;
+ *   0: running sums rounded to FP32 (a third of the workspace; error relative
+ *      to the whole running sum, i.e. growing with the number of rows).
  * Process-wide; affects calls issued afterwards and the workspace they need.
  * No counterpart in the reference, whose adjoint walks rows and slices with
  * atomics (ConeFlatDisCUDA3d.cu:284-536). */
 void dd3d_set_compensated(int mode);
-/* Whether the sinogram -> volume gather stages each view's row running sums
- * for its 16 x 16 pixel tile in LDS: 0 never, 1 always, 2 (default)
- * automatic — with compensated sums or batches of 1-2 (cone-flat 256^3 x 2:
- * adjoint 20.0 -> 15.6 ms), not for rounded sums at batches of 3+ (helical
- * 512x512x64 x 4: 94 ms unstaged, 105 ms staged).  The same bits either
- * way; a view whose block exceeds 32 KB of LDS is read from global memory.
- * No counterpart in the reference. */
+/* Whether the sinogram -> volume gather stages each view's rows (or row
+ * running sums) for its 16 x 16 pixel tile in LDS: 0 never, 1 always, 2
+ * (default) automatic: rows always; compensated sums, and rounded sums at
+ * batches of 1-2 (at batches of 3+ 94 ms unstaged, 105 ms staged, helical
+ * 512x512x64 x 4 x 3456 views).  The same values either way; a view whose
+ * block exceeds the LDS buffer is read from global memory (with rows: after
+ * the others, so such a sum is rounded in another order).  No counterpart in
+ * the reference. */
 void dd3d_set_adjoint_staging(int mode);
 /* Dispatch order of the volume -> sinogram gather: 0 views first (two
  * detector-row chunks per workgroup), 1 detector columns first (one chunk),

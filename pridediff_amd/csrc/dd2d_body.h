@@ -566,22 +566,6 @@ __device__ __forceinline__ int guess_bin_fast(const Geo2& g, const ViewGeo& vg, 
   return static_cast<int>(floorf(kf));
 }
 
-// Where axis points lie relative to pixel i of one line, in pixels from its
-// lower edge: below 0 before the pixel, 1 and up past it.  The one definition
-// used by every sinogram -> image walk, so they agree bit for bit; it is the
-// forward's t - i (edge_pos) up to the FP64 rounding of the products.
-struct PixelFrame {
-  double inv_p, b;
-  __device__ __forceinline__ PixelFrame(double a0, double ip, int i)
-      : inv_p(ip), b(fma(a0, ip, static_cast<double>(i))) {}
-  __device__ __forceinline__ double at(double e) const { return fma(e, inv_p, -b); }
-};
-
-// Fraction of the pixel that lies below such a point.
-__device__ __forceinline__ float pixel_fraction(double u) {
-  return __builtin_amdgcn_fmed3f(static_cast<float>(u), 0.0f, 1.0f);
-}
-
 // Adds the bins from k on that reach the pixel, given the search's state
 // (u1, u2: bin k's edges; k the last bin whose lower edge lies before the
 // pixel, or 0): overlap * weight * sinogram, bins ascending.
@@ -986,25 +970,22 @@ __device__ __forceinline__ unsigned pack_range(int2 r) {
 
 // Rows per lane of the staged walk (tiles of 16 x 4 rows pixels), or 0 where
 // the per-pixel kernel takes the op.  A taller tile shares each staged view
-// over more pixels, but its edges have to fit the slots: along its lines a
-// pixel spans at most `per_pixel` bins (pixel over bin at the image corner
-// next to the source), and views at 45 degrees add as many for each of its
-// rows.  From 2.8 bins per pixel on even 16 x 4 pixels do not fit and the
-// walk would fall back view after view.
+// over more pixels, but its edges have to fit the slots: a tile's diagonal
+// spans at most its length over the bin's width at the image corner next to
+// the source (beam divergence and a flat detector's slant included).  Where
+// even 16 x 4 (8 rows of 16 below 8 instances) pixels do not fit, the walk
+// would go back to single views' bins in memory all the time.
 inline int walk_rows(const Geo2& g) {
-  const double px = fmax(std::fabs(g.dx), std::fabs(g.dy));
   const double half = 0.5 * std::hypot(g.W * g.dx, g.H * g.dy) + std::hypot(g.shx, g.shy);
-  double per_pixel;
-  if (g.scan == DD_PARA) {
-    per_pixel = px / std::fabs(g.det);
-  } else {
+  double bin = std::fabs(g.det);  // smallest bin across the rays
+  if (g.scan != DD_PARA) {
     const double near = g.sid - half;
     if (!(near > 0.0)) return 0;
-    const double det = g.scan == DD_FAN_ARC ? g.sid * std::fabs(g.det)
-                                            : g.sid / g.sdd * std::fabs(g.det);
-    per_pixel = px * g.sid / near / det;
+    bin *= g.scan == DD_FAN_ARC ? near : near / g.sdd / std::hypot(1.0, half / near);
   }
-  auto fits = [&](int rows) { return (kWalkW + 4 * rows) * per_pixel + 4.0 <= kWalkEdges; };
+  auto fits = [&](int rows) {
+    return std::hypot(kWalkW * g.dx, 4.0 * rows * g.dy) / bin + 5.0 <= kWalkEdges;
+  };
   const int most = g.BT >= 8 ? 2 : 4;
   if (fits(most)) return most;
   if (fits(most / 2)) return most / 2;

@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 
 #include "dd3d.h"
 #include "dd_common.h"
@@ -99,6 +100,7 @@ struct ViewGeo3 {
   double theta_ref;    // arc: detector angle base + column shift
   double colp, cshp;   // column pitch and shift (radians, or virtual mm)
   double zdet0, rowp;  // detector row edge r at zdet0 + r * rowp
+  double row0;         // row coordinate of the source's plane: (sz - zdet0) / rowp
   double sid_eff;      // source-isocentre distance of this view
   float sxf, syf, kbp; // float copies; BackProj constant
   float zlo, zhi;      // world z range the view's rays can reach in the volume
@@ -165,8 +167,10 @@ __device__ __forceinline__ float fbp_weight3(const Geo3& g, const ViewGeo3& vg,
 __global__ __launch_bounds__(kThreads3) void k_setup3d(
     Geo3 g, const float* __restrict__ angles, const float* __restrict__ spos,
     ViewGeo3* __restrict__ views, double* __restrict__ cedge,
-    double* __restrict__ mag, LineGeo3* __restrict__ lines) {
+    double* __restrict__ mag, double2* __restrict__ colz, LineGeo3* __restrict__ lines,
+    int* __restrict__ misfits) {
   const int v = blockIdx.x;
+  if (v == 0 && threadIdx.x == 0) *misfits = 0;
   const int C = g.C;
   double sid = g.sid, sdd = g.sdd, colp = g.col, csh = g.csh, sz = 0.0, zoff = 0.0;
   float th_src_f = angles[v];
@@ -205,6 +209,7 @@ __global__ __launch_bounds__(kThreads3) void k_setup3d(
     const double rs = flat ? static_cast<double>(g.sid) / g.sdd : 1.0;
     vg.zdet0 = flat ? (-g.R / 2.0 * g.row + g.rsh) * rs : (-g.R / 2.0 * g.row + g.rsh + zoff);
     vg.rowp = g.row * rs;
+    vg.row0 = (sz - vg.zdet0) / vg.rowp;
     vg.sid_eff = sid;
     vg.sxf = static_cast<float>(sx);
     vg.syf = static_cast<float>(sy);
@@ -242,6 +247,8 @@ __global__ __launch_bounds__(kThreads3) void k_setup3d(
     }
     const double mk = xaxis ? sy / (sy - dcy) : sx / (sx - dcx);
     mag[static_cast<size_t>(v) * C + k] = mk;
+    const double mr = mk * vg.rowp;  // detector row height on the axis plane
+    colz[static_cast<size_t>(v) * C + k] = make_double2(1.0 / mr, mr);
     mag_lo = fmin(mag_lo, mk);
     mag_hi = fmax(mag_hi, mk);
   }
@@ -437,6 +444,36 @@ __global__ __launch_bounds__(kThreads3) void k_prefix_sino3d(
     }
     store_tile<2 * BT>(q2v + 2 * static_cast<size_t>(g.R) * rstride, pair);
     store_tile<2 * BT>(q2v + 2 * static_cast<size_t>(g.R + 1) * rstride, pair);
+  }
+}
+
+// p [B][V][R][C] -> s [V][R][C][Bp], columns in walk order, optionally times
+// the FP weight of each cell: what k_voxel_rows gathers from.
+template <int BT, bool FOLD_W>
+__global__ __launch_bounds__(kThreads3) void k_interleave_sino3d(
+    Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
+    const double* __restrict__ mag, const float* __restrict__ p, float* __restrict__ s) {
+  const int nkc = (g.C + kThreads3 - 1) / kThreads3;
+  const int k = (blockIdx.x % nkc) * kThreads3 + threadIdx.x;
+  const int v = blockIdx.x / nkc;
+  const int b0 = blockIdx.z * BT;
+  if (k >= g.C) return;
+  const ViewGeo3 vg = views[v];
+  const int kk = vg.flip ? g.C - 1 - k : k;
+  for (int r = blockIdx.y; r < g.R; r += gridDim.y) {
+    float w = 1.0f;
+    if (FOLD_W) {
+      const double* ce = cedge + static_cast<size_t>(v) * (g.C + 1);
+      const double m = mag[static_cast<size_t>(v) * g.C + k];
+      w = fp_weight3(g, vg, ce[k], ce[k + 1], row_z(vg, m, r), row_z(vg, m, r + 1));
+    }
+    float val[BT];
+#pragma unroll
+    for (int b = 0; b < BT; ++b)
+      val[b] = (b0 + b < g.B)
+                   ? p[((static_cast<size_t>(b0 + b) * g.V + v) * g.R + r) * g.C + kk] * w
+                   : 0.0f;
+    store_tile<BT>(s + ((static_cast<size_t>(v) * g.R + r) * g.C + k) * g.Bp + b0, val);
   }
 }
 
@@ -1040,14 +1077,511 @@ __attribute__((amdgpu_waves_per_eu(adj_waves3<BT>()))) void k_voxels3d(
 }
 
 // ---------------------------------------------------------------------------
+// sinogram -> image by detector rows: slices no thicker than a few rows
+// ---------------------------------------------------------------------------
+// The same for any d (a source that comes nearer than the geometry's own
+// radius, which the host does not see): every row of a slice read for itself.
+template <int BT, int S, typename Row>
+__device__ __forceinline__ void column_slices_any(float du, float d, float wx, Row row,
+                                                  float (&acc)[S][BT]) {
+  asm volatile("; any rows" : "+v"(du));
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+    const float u = fmaf(static_cast<float>(j), d, du);
+    const float fl = floorf(u);
+    float t[BT], w = fminf(d, 1.0f - (u - fl)), rest = d;
+#pragma unroll
+    for (int b = 0; b < BT; ++b) t[b] = 0.0f;
+    for (int m = 0; rest > 0.0f; ++m) {
+      float x[BT];
+      row(fl, m, x);
+#pragma unroll
+      for (int b = 0; b < BT; ++b) t[b] = fmaf(w, x[b], t[b]);
+      rest -= w;
+      w = fminf(rest, 1.0f);
+    }
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(wx, t[b], acc[j][b]);
+  }
+}
+
+// Floats of LDS that hold one view's rows x columns (kRowPitch entries a row,
+// odd: neighbouring rows fall in different banks), and columns of it: with
+// the tables four workgroups share a compute unit (BT = 1: six).
+template <int BT>
+constexpr int row_floats3() {
+  return BT == 1 ? 5600 : 9600;
+}
+constexpr int kRowCols = 64;
+constexpr int kRowPitch = kRowCols + 1;
+
+template <int BT>
+constexpr int row_slices3() {
+  return BT >= 4 ? 8 : 16;
+}
+
+// What k_voxel_rows stages of one view for one 16 x 16 pixel tile: columns
+// [kb, ke), which hold every pixel edge of the tile, and, to bound the rows
+// from the slices, the slice edges z - sz on the tile's first and last line
+// (z0 + s pz) and the rows per z at its columns' extreme magnifications.
+// FP32: the rows of margin cover the rounding.
+struct RowRange {
+  float z0[2], pz[2], rows[2];
+  int kb, ke;  // ke = kb: the block does not fit the LDS buffer
+
+  // First row and row count of the block of slices [s0, s1).  A row
+  // coordinate (z - sz) / (m rowp) + row0 is monotone in z and in the
+  // magnification m, so the corners bound it (and one row before and two
+  // after).
+  __device__ __forceinline__ void block(float s0, float s1, float row0, float* first,
+                                        float* count) const {
+    const float zmin = fminf(fmaf(s0, pz[0], z0[0]), fmaf(s0, pz[1], z0[1]));
+    const float zmax = fmaxf(fmaf(s1, pz[0], z0[0]), fmaf(s1, pz[1], z0[1]));
+    const float ra = fminf(zmin * rows[0], zmin * rows[1]) + row0;
+    const float rb = fmaxf(zmax * rows[0], zmax * rows[1]) + row0;
+    *first = floorf(fmaxf(ra, -1e6f)) - 1.0f;
+    *count = floorf(fminf(rb, 1e6f)) + 3.0f - *first;
+  }
+};
+
+// One thread per (view, pixel tile).  The tile's axis extent is spanned by
+// its corners (a pixel edge's axis point is monotone along and across the
+// lines), widened by one column edge each side against rounding.
+template <int BT>
+__global__ __launch_bounds__(kThreads3) void k_row_ranges(
+    Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
+    const double2* __restrict__ colz, const LineGeo3* __restrict__ lines,
+    RowRange* __restrict__ out, int* __restrict__ misfits) {
+  const int ntx = (g.W + kTile3 - 1) / kTile3;
+  const int tiles = ntx * ((g.H + kTile3 - 1) / kTile3);
+  const long long idx = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (idx >= static_cast<long long>(tiles) * g.V) return;
+  const int v = static_cast<int>(idx / tiles), t = static_cast<int>(idx % tiles);
+  const int c0 = (t % ntx) * kTile3, r0 = (t / ntx) * kTile3;
+  const int c1 = min(c0 + kTile3, g.W), r1 = min(r0 + kTile3, g.H);
+  const ViewGeo3 vg = views[v];
+  const LineGeo3* __restrict__ lv = lines + static_cast<size_t>(v) * g.Lmax;
+  double amin = 1e300, amax = -1e300;
+  auto corner = [&](int l, int i) {
+    const double a = lv[l].a0 + i / lv[l].inv_p;
+    amin = fmin(amin, a);
+    amax = fmax(amax, a);
+  };
+  if (vg.xaxis) {  // lines = rows, pixel edges = columns
+    corner(r0, c0), corner(r0, c1), corner(r1 - 1, c0), corner(r1 - 1, c1);
+  } else {  // lines = columns, pixel edges from the bottom
+    corner(c0, g.H - r1), corner(c0, g.H - r0), corner(c1 - 1, g.H - r1),
+        corner(c1 - 1, g.H - r0);
+  }
+  const double* __restrict__ ce = cedge + static_cast<size_t>(v) * (g.C + 1);
+  int lo = guess_col_fast(g, vg, amin);  // last edge <= amin
+  while (lo > 0 && ce[lo] > amin) --lo;
+  while (lo < g.C && ce[lo + 1] <= amin) ++lo;
+  RowRange r;
+  r.kb = min(max(lo - 1, 0), g.C - 1);
+  int hi = guess_col_fast(g, vg, amax) + 1;  // first edge >= amax
+  while (hi < g.C && ce[hi] < amax) ++hi;
+  while (hi > 0 && ce[hi - 1] >= amax) --hi;
+  r.ke = max(min(hi + 1, g.C), r.kb + 1);
+  float rmin = 3e38f, rmax = -3e38f;
+  for (int k = r.kb; k < r.ke; ++k) {
+    const float m = static_cast<float>(colz[static_cast<size_t>(v) * g.C + k].x);
+    rmin = fminf(rmin, m);
+    rmax = fmaxf(rmax, m);
+  }
+  r.rows[0] = rmin;
+  r.rows[1] = rmax;
+  const int la = vg.xaxis ? r0 : c0, lb = (vg.xaxis ? r1 : c1) - 1;
+  r.z0[0] = static_cast<float>(lv[la].z0 - vg.sz);
+  r.z0[1] = static_cast<float>(lv[lb].z0 - vg.sz);
+  r.pz[0] = static_cast<float>(lv[la].pz);
+  r.pz[1] = static_cast<float>(lv[lb].pz);
+  // the block's rows over all chunks: their span is largest at one end of
+  // the slices, up to the rounding of both bounds to rows
+  constexpr int S = row_slices3<BT>();
+  const int last = (g.Dz - 1) / S * S;
+  float first, n0, n1;
+  r.block(0.0f, S, static_cast<float>(vg.row0), &first, &n0);
+  r.block(static_cast<float>(last), static_cast<float>(last + S), static_cast<float>(vg.row0),
+          &first, &n1);
+  const int ncols = r.ke - r.kb;
+  if (ncols > kRowCols || (fmaxf(n0, n1) + 2.0f) * (kRowPitch * BT) > row_floats3<BT>()) {
+    r.ke = r.kb;
+    *misfits = 1;
+  }
+  out[idx] = r;
+}
+
+// Adds one detector column's rows to S consecutive slices.  Slice edge j lies
+// at row coordinate u_j = du + j d (relative to a base row), so slice j holds
+// d rows from u_j on: w_0 = min(d, 1 - fraction) of row floor(u_j), then
+// whole rows, then the rest, K rows in all (d <= K - 1); each weight times
+// its row, times wx.  The last of them is row floor(u_{j+1}), the first of
+// the next slice, so it is read once: one row per slice at K = 2, two at 3.
+// row(fl, m, x) gives row fl + m.
+template <int BT, int S, int K, typename Row>
+__device__ __forceinline__ void column_slices(float du, float d, float wx, Row row,
+                                              float (&acc)[S][BT]) {
+  asm volatile("; %1 rows" : "+v"(du) : "i"(K));  // no code shared between the K
+  float fl = floorf(du), f = du - fl;
+  float x[K][BT];
+  row(fl, 0, x[0]);
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+#pragma unroll
+    for (int m = 1; m < K - 1; ++m) row(fl, m, x[m]);
+    const float u = fmaf(static_cast<float>(j + 1), d, du);
+    fl = floorf(u);
+    row(fl, 0, x[K - 1]);
+    float w[K];
+    w[0] = fminf(d, 1.0f - f);
+    float rest = d - w[0];
+#pragma unroll
+    for (int m = 1; m < K; ++m) {
+      w[m] = m < K - 1 ? fminf(rest, 1.0f) : rest;
+      rest -= w[m];
+    }
+    f = u - fl;
+    if constexpr (BT >= 4) {
+#pragma unroll
+      for (int m = 0; m < K; ++m) {
+        const float wm = w[m] * wx;
+#pragma unroll
+        for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(wm, x[m][b], acc[j][b]);
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < BT; ++b) {
+        float t = w[0] * x[0][b];
+#pragma unroll
+        for (int m = 1; m < K; ++m) t = fmaf(w[m], x[m][b], t);
+        acc[j][b] = fmaf(wx, t, acc[j][b]);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < BT; ++b) x[0][b] = x[K - 1][b];
+    if (j % 2) __builtin_amdgcn_sched_barrier(0);  // loads further ahead spill
+  }
+}
+
+// One view's rows into the pixel (row, col)'s slices s0 .. s0 + S - 1,
+// columns [kmin, kend) (column k of the detector being k + koff), through the
+// given accessors: edge k, z law of column k, and one column's rows.
+template <int BT, int WM, int S, typename Edge, typename ZLaw, typename Rows>
+__device__ __forceinline__ void gather_rows(const Geo3& g, const ViewGeo3& vg,
+                                            const LineGeo3& lg, int row, int col, int s0,
+                                            int kmin, int kend, Edge edge, ZLaw zlaw, Rows rows,
+                                            float (&acc)[S][BT], int koff) {
+  const int i = vg.xaxis ? col : g.H - 1 - row;
+  const PixelFrame fr(lg.a0, lg.inv_p, i);
+  // first column: the last whose lower edge lies before pixel i (or kmin);
+  // the edge positions found on the way start the walk
+  int k = guess_col_fast(g, vg, lg.a0 + (i + 0.5) * static_cast<double>(lg.p)) - koff;
+  k = min(max(k, kmin), kend - 1);
+  double u1 = fr.at(edge(k));
+  while (k > kmin && u1 >= 0.0) u1 = fr.at(edge(--k));
+  double u2 = fr.at(edge(k + 1));
+  while (u2 < 0.0 && k < kend - 1) {
+    ++k;
+    u1 = u2;
+    u2 = fr.at(edge(k + 1));
+  }
+  float gw = (WM == W3_FP) ? lg.p * lg.pzf : vg.kbp;
+  if constexpr (WM == W3_BPW) {
+    float xc, yc;
+    pixel_centre3(g, 1, row, col, &xc, &yc);
+    gw *= fbp_weight3(g, vg, xc, yc);
+  }
+  // z - sz of the chunk's first slice edge on this line
+  const double zs = fma(static_cast<double>(s0), lg.pz, lg.z0) - vg.sz;
+  float p1 = pixel_fraction(u1);
+  while (u1 < 1.0) {
+    const float p2 = pixel_fraction(u2);
+    // Rows: slice edge z lies at row u = (z - sz) / (m rowp) + row0, kept
+    // relative to the chunk's first row so that float holds it; d rows per
+    // slice, each row 1 / d of a slice.
+    const double2 z = zlaw(k);
+    const double u0 = fma(zs, z.x, vg.row0);
+    const double rb = floor(u0);
+    const int rbase = static_cast<int>(fmin(fmax(rb, -1.0e6), 1.0e6));
+    const float du = static_cast<float>(u0 - rb);
+    const float d = static_cast<float>(lg.pz * z.x);
+    const float wx = (p2 - p1) * gw * static_cast<float>(z.y * lg.inv_pz);
+    const auto row_at = rows(k, rbase);
+    if (__all(d <= 1.0f))
+      column_slices<BT, S, 2>(du, d, wx, row_at, acc);
+    else if (__all(d <= 2.0f))
+      column_slices<BT, S, 3>(du, d, wx, row_at, acc);
+    else if (__all(d <= 3.0f))
+      column_slices<BT, S, 4>(du, d, wx, row_at, acc);
+    else
+      column_slices_any<BT, S>(du, d, wx, row_at, acc);
+    if (++k >= kend) break;
+    u1 = u2;
+    p1 = p2;
+    if (u1 >= 1.0) break;
+    u2 = fr.at(edge(k + 1));
+  }
+}
+
+template <int BT, int S, bool ADD>
+__device__ __forceinline__ void store_slices(const Geo3& g, float* __restrict__ out, int row,
+                                             int col, int s0, int b0,
+                                             const float (&acc)[S][BT]) {
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+    const int sl = s0 + j;
+    if (sl < g.Dz) {
+#pragma unroll
+      for (int b = 0; b < BT; ++b)
+        if (b0 + b < g.B) {
+          float* o = out + ((static_cast<size_t>(b0 + b) * g.Dz + sl) * g.H + row) * g.W + col;
+          *o = ADD ? *o + acc[j][b] : acc[j][b];
+        }
+    }
+  }
+}
+
+template <int BT>
+struct RowLds {
+  __align__(16) float q[row_floats3<BT>()];
+  double2 colz[kRowCols];
+  double edge[kRowCols + 1];
+  __align__(16) LineGeo3 line[kTile3];
+};
+
+template <int BT>
+constexpr int row_waves3() {  // per SIMD: what the LDS block allows
+  return BT == 1 ? 5 : 4;
+}
+// One thread per pixel and chunk of S slices, all views.  Per view the
+// workgroup's 16 x 16 pixels first stage in LDS the block of rows and columns
+// that their slices can meet (zeros where it leaves the detector), the
+// columns' edges and z laws and the lines' maps (two barriers a view); each
+// pixel then finds its columns as in 2D and adds their rows to its slices
+// (column_slices).  Views whose block does not fit are left to
+// k_voxel_rows_global.
+//
+// Bound by VALU issue (saturated): 18-19 instructions per column, slice and
+// pair of instances.  It replaces differences of running row sums, which need
+// a serial scan over the rows, three LDS reads of sums and values per slice
+// edge where this reads one or two rows, and 23 instructions.  ProjTrans of
+// cone-flat 256^3 x 360 views x 512 x 384 x 2 16.4 -> 11.0 ms with its
+// prologue, helical 512 x 512 x 64 x 1152 views x 4 56.1 -> 40.3 ms; a
+// 96 x 81 x 50 volume x 100 views 0.51 -> 0.11 ms with its views split.
+//
+// Workgroup z takes instance tile z / nsplit and the views' part z % nsplit
+// (nsplit > 1: partial volumes, added by k_sum_volumes).
+template <int BT, int WM>
+__global__ __launch_bounds__(kThreads3)
+__attribute__((amdgpu_waves_per_eu(row_waves3<BT>()))) void k_voxel_rows(
+    Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
+    const double2* __restrict__ colz, const LineGeo3* __restrict__ lines,
+    const float* __restrict__ sino, float* __restrict__ out,
+    const RowRange* __restrict__ ranges, int nsplit) {
+  constexpr int S = row_slices3<BT>();
+  __shared__ RowLds<BT> lds;
+  const int ntx = (g.W + kTile3 - 1) / kTile3;
+  const int tile = blockIdx.x;
+  const int tiles = ntx * ((g.H + kTile3 - 1) / kTile3);
+  int tx = static_cast<int>(threadIdx.x) % kTile3;
+  int ty = static_cast<int>(threadIdx.x) / kTile3;
+  const int tc = (tile % ntx) * kTile3, tr = (tile / ntx) * kTile3;
+  const int s0 = blockIdx.y * S;
+  const int b0 = (blockIdx.z / nsplit) * BT, part = blockIdx.z % nsplit;
+  const int v0 = static_cast<int>(1LL * g.V * part / nsplit);
+  const int v1 = static_cast<int>(1LL * g.V * (part + 1) / nsplit);
+  float acc[S][BT];
+#pragma unroll
+  for (int j = 0; j < S; ++j)
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[j][b] = 0.0f;
+  // world z extent of this thread's slices (block-uniform)
+  const float z0w = -g.Dz * 0.5f * g.dz + (g.scan == DD_SPIRAL ? 0.0f : g.shz);
+  const float zc_lo = z0w + s0 * g.dz, zc_hi = z0w + min(s0 + S, g.Dz) * g.dz;
+  for (int v = v0; v < v1; ++v) {
+    const ViewGeo3 vg = views[v];
+    if (zc_hi < vg.zlo || zc_lo > vg.zhi) continue;  // the view's cone misses the chunk
+    const RowRange vr = ranges[static_cast<size_t>(v) * tiles + tile];
+    float first, count;
+    vr.block(static_cast<float>(s0), static_cast<float>(s0 + S), static_cast<float>(vg.row0),
+             &first, &count);
+    // past the detector, or too large
+    if (first + count < 0.0f || first > static_cast<float>(g.R) || vr.ke == vr.kb) continue;
+    const int srb = __builtin_amdgcn_readfirstlane(static_cast<int>(first));
+    const int nrow = __builtin_amdgcn_readfirstlane(static_cast<int>(count));
+    const int skb = vr.kb, ncols = vr.ke - vr.kb;
+    // what follows from the lane alone is cheaper formed again than kept in
+    // registers over the views
+    asm volatile("" : "+v"(tx), "+v"(ty));
+    __syncthreads();  // the previous view's walks are done with the block
+    {
+      const char* __restrict__ sv = reinterpret_cast<const char*>(
+          sino + static_cast<size_t>(v) * g.R * g.C * g.Bp + b0);
+      // 16 columns x 16 rows of threads per step
+      for (int c = tx; c < ncols; c += kTile3)
+        for (int r = ty; r < nrow; r += kTile3) {
+          const int rr = srb + r;
+          float x[BT];
+#pragma unroll
+          for (int b = 0; b < BT; ++b) x[b] = 0.0f;
+          if (static_cast<unsigned>(rr) < static_cast<unsigned>(g.R))
+            load_tile<BT>(reinterpret_cast<const float*>(
+                              sv + 4u * static_cast<unsigned>((rr * g.C + skb + c) * g.Bp)),
+                          x);
+          store_tile<BT>(lds.q + (r * kRowPitch + c) * BT, x);
+        }
+      const int t = static_cast<int>(threadIdx.x);
+      if (t <= ncols) lds.edge[t] = cedge[static_cast<size_t>(v) * (g.C + 1) + skb + t];
+      if (t < ncols) lds.colz[t] = colz[static_cast<size_t>(v) * g.C + skb + t];
+      // the tile's lines, dword by dword
+      constexpr int kWords = sizeof(LineGeo3) / 4;
+      const int l0 = vg.xaxis ? tr : tc, nl = min(kTile3, (vg.xaxis ? g.H : g.W) - l0);
+      if (t < nl * kWords)
+        reinterpret_cast<int*>(lds.line)[t] =
+            reinterpret_cast<const int*>(lines + static_cast<size_t>(v) * g.Lmax + l0)[t];
+    }
+    __syncthreads();
+    const int col = tc + tx, row = tr + ty;
+    if (col >= g.W || row >= g.H) continue;
+    gather_rows<BT, WM, S>(
+        g, vg, lds.line[vg.xaxis ? ty : tx], row, col, s0, 0, ncols,
+        [&](int k) { return lds.edge[k]; }, [&](int k) { return lds.colz[k]; },
+        [&](int k, int rbase) {
+          // row rbase + fl + m of column k at byte lb + (fl + m) kStep of the
+          // block, formed in float (below 2^24: exact)
+          constexpr int kStep = kRowPitch * BT * 4;
+          const float lb = static_cast<float>((rbase - srb) * kStep + k * BT * 4);
+          const char* lq = reinterpret_cast<const char*>(lds.q);
+          return [=](float fl, int m, float(&x)[BT]) {
+            const int at = static_cast<int>(fmaf(fl, static_cast<float>(kStep), lb));
+            load_tile<BT>(reinterpret_cast<const float*>(lq + at) + m * (kStep / 4), x);
+          };
+        },
+        acc, skb);
+  }
+  const int col = tc + tx, row = tr + ty;
+  if (col >= g.W || row >= g.H) return;
+  if (nsplit > 1) out += static_cast<size_t>(part) * g.B * g.Dz * g.H * g.W;
+  store_slices<BT, S, false>(g, out, row, col, s0, b0, acc);
+}
+
+// The same from global memory: all views (ranges null), or, added to the
+// result, those whose block does not fit the LDS buffer (nothing to do
+// unless *misfits).
+template <int BT, int WM>
+__global__ __launch_bounds__(kThreads3) void k_voxel_rows_global(
+    Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
+    const double2* __restrict__ colz, const LineGeo3* __restrict__ lines,
+    const float* __restrict__ sino, float* __restrict__ out,
+    const RowRange* __restrict__ ranges, const int* __restrict__ misfits) {
+  constexpr int S = row_slices3<BT>();
+  if (ranges && *misfits == 0) return;
+  const int ntx = (g.W + kTile3 - 1) / kTile3;
+  const int tiles = ntx * ((g.H + kTile3 - 1) / kTile3);
+  const int chunks = (g.Dz + S - 1) / S;
+  const long long items = 1LL * tiles * chunks * (g.Bp / BT);
+  for (long long item = blockIdx.x; item < items; item += gridDim.x) {
+    const int tile = static_cast<int>(item % tiles);
+    const int s0 = static_cast<int>(item / tiles % chunks) * S;
+    const int b0 = static_cast<int>(item / tiles / chunks) * BT;
+    const int col = (tile % ntx) * kTile3 + static_cast<int>(threadIdx.x) % kTile3;
+    const int row = (tile / ntx) * kTile3 + static_cast<int>(threadIdx.x) / kTile3;
+    if (col >= g.W || row >= g.H) continue;
+    float acc[S][BT];
+#pragma unroll
+    for (int j = 0; j < S; ++j)
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc[j][b] = 0.0f;
+    const float z0w = -g.Dz * 0.5f * g.dz + (g.scan == DD_SPIRAL ? 0.0f : g.shz);
+    const float zc_lo = z0w + s0 * g.dz, zc_hi = z0w + min(s0 + S, g.Dz) * g.dz;
+    bool any = !ranges;
+    for (int v = 0; v < g.V; ++v) {
+      if (ranges) {
+        const RowRange& vr = ranges[static_cast<size_t>(v) * tiles + tile];
+        if (vr.ke > vr.kb) continue;
+        any = true;
+      }
+      const ViewGeo3 vg = views[v];
+      if (zc_hi < vg.zlo || zc_lo > vg.zhi) continue;
+      const double* __restrict__ ce = cedge + static_cast<size_t>(v) * (g.C + 1);
+      const double2* __restrict__ cz = colz + static_cast<size_t>(v) * g.C;
+      const char* __restrict__ sv = reinterpret_cast<const char*>(
+          sino + static_cast<size_t>(v) * g.R * g.C * g.Bp + b0);
+      gather_rows<BT, WM, S>(
+          g, vg, lines[static_cast<size_t>(v) * g.Lmax + (vg.xaxis ? row : col)], row, col, s0,
+          0, g.C, [&](int k) { return ce[k]; }, [&](int k) { return cz[k]; },
+          [&](int k, int rbase) {
+            return [=, &g](float fl, int m, float(&x)[BT]) {
+              const int r = rbase + static_cast<int>(fl) + m;
+              const bool in = static_cast<unsigned>(r) < static_cast<unsigned>(g.R);
+              load_tile<BT>(
+                  reinterpret_cast<const float*>(
+                      sv + 4u * static_cast<unsigned>(((in ? r : 0) * g.C + k) * g.Bp)),
+                  x);
+#pragma unroll
+              for (int b = 0; b < BT; ++b) x[b] = in ? x[b] : 0.0f;
+            };
+          },
+          acc, 0);
+    }
+    if (!any) continue;
+    if (ranges)
+      store_slices<BT, S, true>(g, out, row, col, s0, b0, acc);
+    else
+      store_slices<BT, S, false>(g, out, row, col, s0, b0, acc);
+  }
+}
+
+// out = sum of the parts' partial volumes, in order.
+__global__ __launch_bounds__(kThreads3) void k_sum_volumes(const float* __restrict__ part,
+                                                           size_t n, int parts,
+                                                           float* __restrict__ out) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  float s = part[i];
+  for (int p = 1; p < parts; ++p) s += part[static_cast<size_t>(p) * n + i];
+  out[i] = s;
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 constexpr size_t kAlign3 = 256;
 
 struct Layout3 {
-  size_t views, cedge, mag, lines, geo_total;
-  size_t buf0, buf1, ranges, data_total;
+  size_t views, cedge, mag, colz, lines, misfits, geo_total;
+  size_t buf0, buf1, ranges, parts, data_total;
+  bool rows;    // sinogram -> volume by detector rows (k_voxel_rows)
+  int nsplit;   // its view parts
 };
+
+// Whether the sinogram -> volume ops add detector rows directly: where a
+// slice meets at most 4 rows (is at most 3 rows thick at the volume's corner
+// next to the source) and a 16 x 16 pixel tile's columns fit the LDS tables
+// there.  Thicker slices take the running sums, whose cost does not depend on
+// the rows per slice; so does dd3d_set_compensated(0 / 1).
+bool use_rows3(const Geo3& g) {
+  if (g_compensated.load() != 2) return false;
+  const double half = 0.5 * std::hypot(g.W * g.dx, g.H * g.dy) + std::hypot(g.shx, g.shy);
+  const double near = g.sid - half;
+  if (!(near > 0.0) || !(g.row > 0.0f) || !(g.dz > 0.0f) || !(g.col > 0.0f)) return false;
+  const bool flat = g.scan == DD_CONE_FLAT;
+  const double across = std::hypot(kTile3 * g.dx, kTile3 * g.dy) *
+                        (flat ? std::hypot(1.0, half / near) * g.sdd : 1.0) / near / g.col;
+  return g.dz * g.sdd / near / g.row <= 3.0 && across + 4.0 <= kRowCols;
+}
+
+// Parts the views of such an op are split over, so that a small volume fills
+// the chip: about 2048 workgroups of 16 x 16 pixels x 16 slices, at least 8
+// views each.  It depends on the volume and the views alone, so a volume gets
+// the same partition in any batch.
+int view_split3(const Geo3& g) {
+  const long long groups = 1LL * ((g.W + kTile3 - 1) / kTile3) * ((g.H + kTile3 - 1) / kTile3) *
+                           ((g.Dz + 15) / 16);
+  const long long n = std::min<long long>(2048 / groups, g.V / 8);
+  return static_cast<int>(std::max<long long>(1, std::min<long long>(n, 16)));
+}
 
 bool to_sino3(int op) {
   return op == DD_PROJ || op == DD_BPROJ_T || op == DD_BPROJ_TW;
@@ -1070,7 +1604,9 @@ Layout3 make_layout3(const Geo3& g, int op) {
   L.views = take(sizeof(ViewGeo3) * g.V);
   L.cedge = take(sizeof(double) * g.V * (g.C + 1));
   L.mag = take(sizeof(double) * g.V * g.C);
+  L.colz = take(sizeof(double2) * g.V * g.C);
   L.lines = take(sizeof(LineGeo3) * g.V * g.Lmax);
+  L.misfits = take(sizeof(int));
   L.geo_total = off;
   off = 0;
   const size_t vox = static_cast<size_t>(g.W) * g.H * g.Dz * g.Bp;
@@ -1078,6 +1614,14 @@ Layout3 make_layout3(const Geo3& g, int op) {
     // one pixel of padding: k_bins3d loads pixels in pairs
     L.buf0 = take(sizeof(float) * (vox + g.BT));
     L.buf1 = take(sizeof(float) * (vox + g.BT));
+  } else if (use_rows3(g)) {
+    L.rows = true;
+    L.buf0 = take(sizeof(float) * static_cast<size_t>(g.V) * g.R * g.C * g.Bp);
+    L.ranges = take(sizeof(RowRange) * g.V * ((g.W + kTile3 - 1) / kTile3) *
+                    ((g.H + kTile3 - 1) / kTile3));
+    L.nsplit = view_split3(g);
+    if (L.nsplit > 1)
+      L.parts = take(sizeof(float) * L.nsplit * static_cast<size_t>(g.B) * g.Dz * g.H * g.W);
   } else {
     const size_t q = sizeof(float) * static_cast<size_t>(g.V) * (g.R + 2) * g.C * g.Bp;
     L.buf0 = take(q);
@@ -1171,6 +1715,61 @@ void launch_adjoint3(const Geo3& g, int op, const float* input, float* output,
   }
 }
 
+// sinogram -> volume by detector rows
+template <int BT>
+void launch_rows3(const Geo3& g, int op, const float* input, float* output,
+                  const ViewGeo3* views, const double* cedge, const double* mag,
+                  const double2* colz, const LineGeo3* lines, int* misfits, char* ws,
+                  const Layout3& L, hipStream_t st) {
+  auto* q = reinterpret_cast<float*>(ws + L.buf0);
+  auto* ranges = reinterpret_cast<RowRange*>(ws + L.ranges);
+  const dim3 sgrid((g.C + kThreads3 - 1) / kThreads3 * g.V, std::min(g.R, 65535), g.Bp / BT);
+  if (op == DD_PROJ_T)
+    hipLaunchKernelGGL((k_interleave_sino3d<BT, true>), sgrid, dim3(kThreads3), 0, st, g, views,
+                       cedge, mag, input, q);
+  else
+    hipLaunchKernelGGL((k_interleave_sino3d<BT, false>), sgrid, dim3(kThreads3), 0, st, g, views,
+                       cedge, mag, input, q);
+  constexpr int S = row_slices3<BT>();
+  const int ntx = (g.W + kTile3 - 1) / kTile3, nty = (g.H + kTile3 - 1) / kTile3;
+  const int chunks = (g.Dz + S - 1) / S;
+  const long long items = 1LL * ntx * nty * chunks * (g.Bp / BT);
+  ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
+  auto run = [&](auto wm) {
+    constexpr int WM = decltype(wm)::value;
+    if (g_stage3.load() == 0) {
+      hipLaunchKernelGGL((k_voxel_rows_global<BT, WM>), dim3(static_cast<unsigned>(items)),
+                         dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, output,
+                         static_cast<const RowRange*>(nullptr), misfits);
+      return;
+    }
+    const long long n = 1LL * ntx * nty * g.V;
+    hipLaunchKernelGGL((k_row_ranges<BT>),
+                       dim3(static_cast<unsigned>((n + kThreads3 - 1) / kThreads3)),
+                       dim3(kThreads3), 0, st, g, views, cedge, colz, lines, ranges, misfits);
+    auto* dst = L.nsplit > 1 ? reinterpret_cast<float*>(ws + L.parts) : output;
+    hipLaunchKernelGGL((k_voxel_rows<BT, WM>), dim3(ntx * nty, chunks, g.Bp / BT * L.nsplit),
+                       dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, dst, ranges,
+                       L.nsplit);
+    if (L.nsplit > 1) {
+      const size_t m = static_cast<size_t>(g.B) * g.Dz * g.H * g.W;
+      hipLaunchKernelGGL(k_sum_volumes,
+                         dim3(static_cast<unsigned>((m + kThreads3 - 1) / kThreads3)),
+                         dim3(kThreads3), 0, st, dst, m, L.nsplit, output);
+    }
+    hipLaunchKernelGGL((k_voxel_rows_global<BT, WM>),
+                       dim3(static_cast<unsigned>(std::min<long long>(items, 1024))),
+                       dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, output, ranges,
+                       misfits);
+  };
+  if (op == DD_PROJ_T)
+    run(std::integral_constant<int, W3_FP>{});
+  else if (op == DD_BPROJ)
+    run(std::integral_constant<int, W3_BP>{});
+  else
+    run(std::integral_constant<int, W3_BPW>{});
+}
+
 bool use_cols_first(const Geo3& g, int bt) {
   const int m = g_fwd_order.load();
   if (g.V > 65535) return false;  // the views are grid dimension y
@@ -1223,6 +1822,10 @@ dd_status launch3(const Geo3& g, int op, const float* input, float* output,
       launch_bins3<BT, false>(g, op, dim3(g.V, ncolb, ncb * ntile), kChunksViewsFirst, views,
                               cedge, mag, lines, buf0, buf1, output, st);
     }
+  } else if (L.rows) {
+    launch_rows3<BT>(g, op, input, output, views, cedge, mag,
+                     reinterpret_cast<const double2*>(geo + L.colz), lines,
+                     reinterpret_cast<int*>(geo + L.misfits), ws, L, st);
   } else {
     auto* ranges = reinterpret_cast<VoxRange*>(ws + L.ranges);
     if (buf1 != buf0)
@@ -1277,7 +1880,9 @@ dd_status dd3d_run(int scan, int op, const dd_geom3d* g, const float* input,
                      source_pos, reinterpret_cast<ViewGeo3*>(w + L.views),
                      reinterpret_cast<double*>(w + L.cedge),
                      reinterpret_cast<double*>(w + L.mag),
-                     reinterpret_cast<LineGeo3*>(w + L.lines));
+                     reinterpret_cast<double2*>(w + L.colz),
+                     reinterpret_cast<LineGeo3*>(w + L.lines),
+                     reinterpret_cast<int*>(w + L.misfits));
   char* data = w + L.geo_total;
   switch (q.BT) {
     case 1: return launch3<1>(q, op, input, output, w, data, L, st);

@@ -72,6 +72,22 @@ __device__ __forceinline__ float overlap_in_pixel(EdgePos p1, EdgePos p2,
   return hi - lo;
 }
 
+// Where axis points lie relative to pixel i of one line, in pixels from its
+// lower edge: below 0 before the pixel, 1 and up past it.  The one definition
+// used by every sinogram -> image walk, so they agree bit for bit; it is the
+// forward's t - i (edge_pos) up to the FP64 rounding of the products.
+struct PixelFrame {
+  double inv_p, b;
+  __device__ __forceinline__ PixelFrame(double a0, double ip, int i)
+      : inv_p(ip), b(fma(a0, ip, static_cast<double>(i))) {}
+  __device__ __forceinline__ double at(double e) const { return fma(e, inv_p, -b); }
+};
+
+// Fraction of the pixel that lies below such a point.
+__device__ __forceinline__ float pixel_fraction(double u) {
+  return __builtin_amdgcn_fmed3f(static_cast<float>(u), 0.0f, 1.0f);
+}
+
 // Axis choice exactly as the reference takes it: FP32 cosine squared in FP32
 // (`cosVal * cosVal > 0.5`, FanArcDisCPU2d.cpp:76; flips :78-84, :148-154).
 __device__ __forceinline__ void choose_axis(float theta, int* xaxis,
