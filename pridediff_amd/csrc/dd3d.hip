@@ -313,12 +313,13 @@ __global__ __launch_bounds__(kThreads3) void k_setup3d(
 // ---------------------------------------------------------------------------
 // layout prologues
 // ---------------------------------------------------------------------------
-// x [B][Dz][H][W] -> xrow [tile][H][Dz][W][BT], xcol [tile][W][Dz][H][BT]
+// x [B][Dz][H][W] -> xrow [tile][H][Dz + 2][W][BT], xcol [tile][W][Dz + 2][H][BT]
 // (bottom-up), tile = BT consecutive instances: a pixel's BT values and its
-// neighbour's are contiguous, whatever the padded batch.  One workgroup per
-// 16 x 16 pixels of one slice: the column copy runs down the image's
-// columns, so the tile passes through LDS and is written transposed, and a
-// wave's lanes write contiguous pixels of both copies.
+// neighbour's are contiguous, whatever the padded batch; a slice of zeros
+// before and after each line's, so that rows reaching past the volume need no
+// masks.  One workgroup per 16 x 16 pixels of one slice: the column copy runs
+// down the image's columns, so the tile passes through LDS and is written
+// transposed, and a wave's lanes write contiguous pixels of both copies.
 constexpr int kItile3 = 16;
 
 template <int BT>
@@ -333,18 +334,19 @@ __global__ __launch_bounds__(kItile3 * kItile3) void k_interleave_volume(
   const int tx = static_cast<int>(threadIdx.x) % kItile3;
   const int ty = static_cast<int>(threadIdx.x) / kItile3;
   const int w0 = (blockIdx.x % ntw) * kItile3, h0 = (blockIdx.x / ntw) * kItile3;
-  const int s = blockIdx.y;
+  const int s = blockIdx.y;  // slice s - 1 of the volume
+  const bool zero = s == 0 || s > g.Dz;
   const int b0 = blockIdx.z * BT;
-  const size_t tile = static_cast<size_t>(blockIdx.z) * g.W * g.H * g.Dz * BT;
+  const size_t tile = static_cast<size_t>(blockIdx.z) * g.W * g.H * (g.Dz + 2) * BT;
   if (h0 + ty < g.H && w0 + tx < g.W) {
     const int h = h0 + ty, w = w0 + tx;
     float v[BT];
 #pragma unroll
     for (int b = 0; b < BT; ++b)
-      v[b] = (b0 + b < g.B)
-                 ? x[((static_cast<size_t>(b0 + b) * g.Dz + s) * g.H + h) * g.W + w]
+      v[b] = (b0 + b < g.B && !zero)
+                 ? x[((static_cast<size_t>(b0 + b) * g.Dz + s - 1) * g.H + h) * g.W + w]
                  : 0.0f;
-    store_tile<BT>(xrow + tile + ((static_cast<size_t>(h) * g.Dz + s) * g.W + w) * BT, v);
+    store_tile<BT>(xrow + tile + ((static_cast<size_t>(h) * (g.Dz + 2) + s) * g.W + w) * BT, v);
 #pragma unroll
     for (int b = 0; b < BT; ++b) t[ty * kRowPitch + tx * (BT + 1) + b] = v[b];
   }
@@ -355,8 +357,8 @@ __global__ __launch_bounds__(kItile3 * kItile3) void k_interleave_volume(
     float v[BT];
 #pragma unroll
     for (int b = 0; b < BT; ++b) v[b] = t[tx * kRowPitch + ty * (BT + 1) + b];
-    store_tile<BT>(xcol + tile + ((static_cast<size_t>(w) * g.Dz + s) * g.H + (g.H - 1 - h)) * BT,
-                   v);
+    store_tile<BT>(
+        xcol + tile + ((static_cast<size_t>(w) * (g.Dz + 2) + s) * g.H + (g.H - 1 - h)) * BT, v);
   }
 }
 
@@ -573,14 +575,242 @@ constexpr int adj_waves3() {
   return DD3D_ADJ_WAVES;
 }
 
+// Rows per thread of k_bins3d, wavefronts per SIMD its registers are held to,
+// and rows between scheduling barriers (0: none).  More rows share a line's
+// geometry and the slice at a chunk's end; how many loads the scheduler may
+// move ahead decides the rest, and differs with the load's width.  Forward of
+// 256^3 x 120 views x 512 x 384, ms: one instance, 16 rows 3.4 (barrier every
+// 3 rows, 5 wavefronts), 4.4 (every 2, 4), 7.4 (none); 8 rows 4.4.  Two: 16
+// rows 4.2 (none, 3), 4.7 (every 4); 8 rows 4.8.  Four: 8 rows 7.9 (every 4,
+// 3), 8.8 (every 2), 13.6 (none).  A small op takes 8 rows, for twice the
+// wavefronts (96 x 81 x 50, 131 x 75 x 100 views: 0.19 against 0.26 ms).
+template <int BT>
+constexpr int line_rows3(bool small) {
+  return BT >= 4 || small ? 8 : 16;
+}
+template <int BT, int S>
+constexpr int line_waves3() {
+  return BT >= 2 ? 3 : S == 8 ? 6 : 5;
+}
+template <int BT, int S>
+constexpr int line_batch3() {
+  return BT >= 4 ? 4 : BT == 2 ? 0 : S == 8 ? 2 : 3;
+}
+
+// One line's share of a detector column's S rows, by rows: n <= NX pixels from
+// px on (weights wx), summed over x slice by slice as the rows meet them.  Row
+// edge j lies at slice coordinate t_j = dt + j d relative to slice `base`,
+// so row j holds d slices from t_j on: min(d, 1 - fraction) of slice
+// floor(t_j), then whole slices, then the rest, K slices in all
+// (d <= K - 1); the last of them is the first of the next row, so it is read
+// once.  K = 0: any d, every slice of a row read for itself (a source that
+// comes nearer than the geometry's own radius, which the host does not see).
+// Slices outside the volume are its zero slices.
+template <int BT, int S, int K, int NX>
+__device__ __forceinline__ void line_rows(const float* __restrict__ px, int sstride, int base,
+                                          int Dz, float dt, float d, const float (&wx)[NX],
+                                          int n, float (&acc)[S][BT]) {
+  asm volatile("; %1 slices" : "+v"(dt) : "i"(K * 10 + NX));  // no code shared between the K
+  const float lo = static_cast<float>(-1 - base), hi = static_cast<float>(Dz - base);
+  const char* __restrict__ pb = reinterpret_cast<const char*>(px);
+  const unsigned at0 = static_cast<unsigned>(base) * static_cast<unsigned>(sstride);
+  auto slice = [&](float fl, float (&x)[BT]) {
+    const int s = static_cast<int>(__builtin_amdgcn_fmed3f(fl, lo, hi));
+    const float* q = reinterpret_cast<const float*>(
+        pb + static_cast<int>(at0 + static_cast<unsigned>(__mul24(s, sstride))));
+    float x0[BT], x1[BT];
+    load_pair<BT>(q, BT, x0, x1);
+#pragma unroll
+    for (int b = 0; b < BT; ++b) {
+      x[b] = wx[0] * x0[b];
+      const float y = fmaf(wx[1], x1[b], x[b]);
+      x[b] = n > 1 ? y : x[b];
+    }
+    if constexpr (NX > 2) {
+      load_tile<BT>(q + 2 * BT, x0);
+#pragma unroll
+      for (int b = 0; b < BT; ++b) {
+        const float y = fmaf(wx[2], x0[b], x[b]);
+        x[b] = n > 2 ? y : x[b];
+      }
+    }
+  };
+  float fl = floorf(dt), f = dt - fl;
+  if constexpr (K == 0) {
+#pragma unroll
+    for (int j = 0; j < S; ++j) {
+      const float t = fmaf(static_cast<float>(j), d, dt);
+      fl = floorf(t);
+      float w = fminf(d, 1.0f - (t - fl)), rest = d;
+      for (float s = fl; rest > 0.0f; s += 1.0f) {
+        float x[BT];
+        slice(s, x);
+#pragma unroll
+        for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(w, x[b], acc[j][b]);
+        rest -= w;
+        w = fminf(rest, 1.0f);
+      }
+    }
+    return;
+  }
+  float x[K > 0 ? K : 1][BT];
+  slice(fl, x[0]);
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+#pragma unroll
+    for (int m = 1; m < K - 1; ++m) slice(fl + static_cast<float>(m), x[m]);
+    const float t = fmaf(static_cast<float>(j + 1), d, dt);
+    fl = floorf(t);
+    slice(fl, x[K - 1]);
+    float w[K > 0 ? K : 1];
+    w[0] = fminf(d, 1.0f - f);
+    float rest = d - w[0];
+#pragma unroll
+    for (int m = 1; m < K; ++m) {
+      w[m] = m < K - 1 ? fminf(rest, 1.0f) : rest;
+      rest -= w[m];
+    }
+    f = t - fl;
+#pragma unroll
+    for (int m = 0; m < K; ++m)
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(w[m], x[m][b], acc[j][b]);
+#pragma unroll
+    for (int b = 0; b < BT; ++b) x[0][b] = x[K - 1][b];
+    if constexpr (line_batch3<BT, S>() > 0)
+      if (j % line_batch3<BT, S>() == line_batch3<BT, S>() - 1) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // image -> sinogram: one thread per (view, column, chunk of S rows).  Per
+// line the column's x footprint and the z law are evaluated once and shared
+// by the S rows (line_rows).
+//
+// Bound by the vector-memory path's latency and return rate; the slice-major
+// form it replaces spread each slice over all the chunk's rows, two thirds of
+// them with weight zero, at twice the VALU instructions (saturated).  Forward
+// of cone-flat 256^3 x 360 views x 512 x 384 x 2 17.7 -> 12.2 ms, helical
+// 512 x 512 x 64 x 1152 views x 4 49.7 -> 43 ms.
+template <int BT, int WM, int S, bool COLS_FIRST>
+__global__ __launch_bounds__(kFwdThreads)
+__attribute__((amdgpu_waves_per_eu(line_waves3<BT, S>()))) void k_bins3d(
+    Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
+    const double* __restrict__ mag, const LineGeo3* __restrict__ lines,
+    const float* __restrict__ xrow, const float* __restrict__ xcol,
+    float* __restrict__ out) {
+  constexpr int CH = COLS_FIRST ? kChunksColsFirst : kChunksViewsFirst;
+  const int v = COLS_FIRST ? blockIdx.y : blockIdx.x;
+  const int k = (COLS_FIRST ? blockIdx.x : blockIdx.y) * kColsPerBlock +
+                (threadIdx.x % kColsPerBlock);
+  const int nch = (g.R + S - 1) / S;
+  const int ncb = (nch + CH - 1) / CH;
+  const int ch = (blockIdx.z % ncb) * CH + threadIdx.x / kColsPerBlock;
+  const int b0 = (blockIdx.z / ncb) * BT;
+  const int r0 = ch * S;
+  if (k >= g.C || r0 >= g.R) return;
+  const int nr = min(S, g.R - r0);
+  const ViewGeo3 vg = views[v];
+  const int xaxis = vg.xaxis;
+  const int L = xaxis ? g.H : g.W;
+  const int N = xaxis ? g.W : g.H;
+  const float* __restrict__ src =
+      (xaxis ? xrow : xcol) + static_cast<size_t>(b0) * g.W * g.H * (g.Dz + 2);  // tile b0 / BT
+  const double* ce = cedge + static_cast<size_t>(v) * (g.C + 1);
+  const double e1 = ce[k], e2 = ce[k + 1];
+  const double m = mag[static_cast<size_t>(v) * g.C + k];
+  const LineGeo3* __restrict__ lv = lines + static_cast<size_t>(v) * g.Lmax;
+  // row edge r0 and the row height on the axis plane
+  const double z0 = row_z(vg, m, r0), dz = m * vg.rowp;
+  float acc[S][BT];
+#pragma unroll
+  for (int j = 0; j < S; ++j)
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[j][b] = 0.0f;
+  int lfirst, llast;
+  line_range(lv, L, g.Dz, z0, row_z(vg, m, r0 + nr), &lfirst, &llast);
+  // one line of margin: the range test and the row walk round differently
+  lfirst = max(lfirst - 1, 0);
+  llast = min(llast + 1, L - 1);
+  const int sstride = N * BT * 4;  // bytes from slice to slice
+  // the next line's geometry is loaded while this line is worked on
+  LineGeo3 lg_next = lv[min(lfirst, L - 1)];
+  for (int l = lfirst; l <= llast; ++l) {
+    const LineGeo3 lg = lg_next;
+    lg_next = lv[min(l + 1, llast)];
+    const EdgePos p1 = edge_pos(e1, lg.a0, lg.inv_p, N);
+    const EdgePos p2 = edge_pos(e2, lg.a0, lg.inv_p, N);
+    const int cs = max(p1.c, 0), cl = min(p2.c, N - 1);
+    if (cs > cl) continue;
+    // the chunk's row edges in slices: t_j = base + dt + j d
+    const double t0 = fmin(fmax((z0 - lg.z0) * lg.inv_pz, -1.0e6), 1.0e6);
+    const double tb = floor(t0);
+    const int base = static_cast<int>(tb);
+    const float dt = static_cast<float>(t0 - tb), d = static_cast<float>(dz * lg.inv_pz);
+    const float end = fmaf(static_cast<float>(S), d, dt);
+    // the chunk's rows miss the slab
+    if (base >= g.Dz || static_cast<float>(base) + end < 0.0f) continue;
+    const float wl = (WM == W3_FP) ? lg.p * lg.pzf : vg.kbp;
+    const float* __restrict__ line = src + (static_cast<size_t>(l) * (g.Dz + 2) + 1) * N * BT;
+    auto weight = [&](int c) {
+      float w = overlap_in_pixel(p1, p2, c) * wl;
+      if constexpr (WM == W3_BPW) {
+        float xc, yc;
+        pixel_centre3(g, xaxis, l, c, &xc, &yc);
+        w *= fbp_weight3(g, vg, xc, yc);
+      }
+      return w;
+    };
+    // pixels by twos, or threes where some column of the wavefront meets a
+    // third (the padding keeps the loads past a line's end in the buffer)
+    auto rows = [&](auto kk) {
+      constexpr int K = decltype(kk)::value;
+      if (__all(cl - cs <= 1)) {
+        const float w[2] = {weight(cs), weight(cs + 1)};
+        line_rows<BT, S, K, 2>(line + static_cast<size_t>(cs) * BT, sstride, base, g.Dz, dt, d,
+                               w, cl - cs + 1, acc);
+      } else if (__all(cl - cs <= 2)) {
+        const float w[3] = {weight(cs), weight(cs + 1), weight(cs + 2)};
+        line_rows<BT, S, K, 3>(line + static_cast<size_t>(cs) * BT, sstride, base, g.Dz, dt, d,
+                               w, cl - cs + 1, acc);
+      } else {
+        for (int c = cs; c <= cl; c += 2) {
+          const float w[2] = {weight(c), weight(c + 1)};
+          line_rows<BT, S, K, 2>(line + static_cast<size_t>(c) * BT, sstride, base, g.Dz, dt, d,
+                                 w, cl - c + 1, acc);
+        }
+      }
+    };
+    if (__all(d <= 1.0f))
+      rows(std::integral_constant<int, 2>{});
+    else if (__all(d <= 2.0f))
+      rows(std::integral_constant<int, 3>{});
+    else
+      rows(std::integral_constant<int, 0>{});
+  }
+  const int kk = vg.flip ? g.C - 1 - k : k;
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+    if (j < nr) {
+      const int r = r0 + j;
+      const float wk = (WM == W3_FP)
+                           ? fp_weight3(g, vg, e1, e2, row_z(vg, m, r), row_z(vg, m, r + 1))
+                           : 1.0f;
+#pragma unroll
+      for (int b = 0; b < BT; ++b)
+        if (b0 + b < g.B)
+          out[((static_cast<size_t>(b0 + b) * g.V + v) * g.R + r) * g.C + kk] = acc[j][b] * wk;
+    }
+  }
+}
+
+// The same for rows thicker than two slices, slice by slice: per
 // line the column's x footprint and the z law are evaluated once and shared
 // by the S rows; the slices the chunk reaches are then visited once each,
 // every slice's voxels loaded once and spread over the S rows by their z
 // overlaps (slice-major: a row-by-row walk reloads each slice for every
 // row that overlaps it).
 template <int BT, int WM, bool COLS_FIRST>
-__global__ __launch_bounds__(kFwdThreads) void k_bins3d(
+__global__ __launch_bounds__(kFwdThreads) void k_bins3d_slices(
     Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
     const double* __restrict__ mag, const LineGeo3* __restrict__ lines,
     const float* __restrict__ xrow, const float* __restrict__ xcol,
@@ -602,7 +832,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_bins3d(
   const int L = xaxis ? g.H : g.W;
   const int N = xaxis ? g.W : g.H;
   const float* __restrict__ src =
-      (xaxis ? xrow : xcol) + static_cast<size_t>(b0) * g.W * g.H * g.Dz;  // tile b0 / BT
+      (xaxis ? xrow : xcol) + static_cast<size_t>(b0) * g.W * g.H * (g.Dz + 2);  // tile b0 / BT
   const double* ce = cedge + static_cast<size_t>(v) * (g.C + 1);
   const double e1 = ce[k], e2 = ce[k + 1];
   const double m = mag[static_cast<size_t>(v) * g.C + k];
@@ -636,7 +866,8 @@ __global__ __launch_bounds__(kFwdThreads) void k_bins3d(
     const int s_hi = min(re.base + static_cast<int>(floorf(t[S])), g.Dz - 1);
     if (s_lo > s_hi) continue;  // the chunk's rows miss the slab
     const float wl = (WM == W3_FP) ? lg.p * lg.pzf : vg.kbp;
-    const float* __restrict__ line = src + static_cast<size_t>(l) * g.Dz * N * BT;
+    const float* __restrict__ line =
+        src + (static_cast<size_t>(l) * (g.Dz + 2) + 1) * N * BT;  // slice 0
     // Columns in pairs: each slice's pair is loaded once and its x-weighted
     // sum spread over the chunk's rows by their z overlaps.  The second
     // column of a pair past cl is masked (its load stays inside the
@@ -1609,11 +1840,11 @@ Layout3 make_layout3(const Geo3& g, int op) {
   L.misfits = take(sizeof(int));
   L.geo_total = off;
   off = 0;
-  const size_t vox = static_cast<size_t>(g.W) * g.H * g.Dz * g.Bp;
+  const size_t vox = static_cast<size_t>(g.W) * g.H * (g.Dz + 2) * g.Bp;
   if (to_sino3(op)) {
-    // one pixel of padding: k_bins3d loads pixels in pairs
-    L.buf0 = take(sizeof(float) * (vox + g.BT));
-    L.buf1 = take(sizeof(float) * (vox + g.BT));
+    // two pixels of padding: the gathers load pixels in pairs and threes
+    L.buf0 = take(sizeof(float) * (vox + 2 * g.BT));
+    L.buf1 = take(sizeof(float) * (vox + 2 * g.BT));
   } else if (use_rows3(g)) {
     L.rows = true;
     L.buf0 = take(sizeof(float) * static_cast<size_t>(g.V) * g.R * g.C * g.Bp);
@@ -1778,20 +2009,40 @@ bool use_cols_first(const Geo3& g, int bt) {
   return tile_bytes > 192.0 * (1 << 20);
 }
 
+// Whether the volume -> sinogram ops go row by row: rows at most two slices
+// thick at the volume's far corner.  Thicker rows go slice by slice.
+bool use_line_rows3(const Geo3& g) {
+  const double half = 0.5 * std::hypot(g.W * g.dx, g.H * g.dy) + std::hypot(g.shx, g.shy);
+  return g.row > 0.0f && g.dz > 0.0f && g.sdd > 0.0f &&
+         g.row / g.sdd * (g.sid + half) / g.dz <= 2.0;
+}
+
 template <int BT, bool COLS_FIRST>
-void launch_bins3(const Geo3& g, int op, dim3 grid, int chunks, const ViewGeo3* views,
-                  const double* cedge, const double* mag, const LineGeo3* lines,
-                  const float* buf0, const float* buf1, float* output, hipStream_t st) {
-  const dim3 block(kColsPerBlock * chunks);
+void launch_bins3(const Geo3& g, int op, const ViewGeo3* views, const double* cedge,
+                  const double* mag, const LineGeo3* lines, const float* buf0, const float* buf1,
+                  float* output, hipStream_t st) {
+  constexpr int CH = COLS_FIRST ? kChunksColsFirst : kChunksViewsFirst;
+  const unsigned ncolb = (g.C + kColsPerBlock - 1) / kColsPerBlock;
+  const bool by_rows = use_line_rows3(g);
+  // small: fewer than 4 wavefronts per SIMD at the most rows
+  const bool small = 1LL * g.V * ncolb * ((g.R + 15) / 16) * (g.Bp / BT) < 4096;
+  const int S = by_rows ? line_rows3<BT>(small) : rows3<BT>();
+  const unsigned z = ((g.R + S - 1) / S + CH - 1) / CH * (g.Bp / BT);
+  const dim3 grid = COLS_FIRST ? dim3(ncolb, g.V, z) : dim3(g.V, ncolb, z);
+  auto run = [&](auto wm) {
+    constexpr int WM = decltype(wm)::value;
+    const auto kernel = !by_rows ? k_bins3d_slices<BT, WM, COLS_FIRST>
+                        : small  ? k_bins3d<BT, WM, line_rows3<BT>(true), COLS_FIRST>
+                                 : k_bins3d<BT, WM, line_rows3<BT>(false), COLS_FIRST>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kColsPerBlock * CH), 0, st, g, views, cedge, mag,
+                       lines, buf0, buf1, output);
+  };
   if (op == DD_PROJ)
-    hipLaunchKernelGGL((k_bins3d<BT, W3_FP, COLS_FIRST>), grid, block, 0, st, g, views, cedge,
-                       mag, lines, buf0, buf1, output);
+    run(std::integral_constant<int, W3_FP>{});
   else if (op == DD_BPROJ_T)
-    hipLaunchKernelGGL((k_bins3d<BT, W3_BP, COLS_FIRST>), grid, block, 0, st, g, views, cedge,
-                       mag, lines, buf0, buf1, output);
+    run(std::integral_constant<int, W3_BP>{});
   else
-    hipLaunchKernelGGL((k_bins3d<BT, W3_BPW, COLS_FIRST>), grid, block, 0, st, g, views, cedge,
-                       mag, lines, buf0, buf1, output);
+    run(std::integral_constant<int, W3_BPW>{});
 }
 
 template <int BT>
@@ -1807,21 +2058,13 @@ dd_status launch3(const Geo3& g, int op, const float* input, float* output,
   if (to_sino3(op)) {
     hipLaunchKernelGGL(k_interleave_volume<BT>,
                        dim3(((g.W + kItile3 - 1) / kItile3) * ((g.H + kItile3 - 1) / kItile3),
-                            g.Dz, ntile),
+                            g.Dz + 2, ntile),
                        dim3(kItile3 * kItile3), 0, st, g, input, buf0, buf1);
-    constexpr int S = rows3<BT>();
-    const int nch = (g.R + S - 1) / S;
-    const unsigned ncolb = (g.C + kColsPerBlock - 1) / kColsPerBlock;
     ProfileScope prof(DD_KERNEL_IMAGE_TO_SINO, st);
-    if (use_cols_first(g, BT)) {
-      const int ncb = (nch + kChunksColsFirst - 1) / kChunksColsFirst;
-      launch_bins3<BT, true>(g, op, dim3(ncolb, g.V, ncb * ntile), kChunksColsFirst, views,
-                             cedge, mag, lines, buf0, buf1, output, st);
-    } else {
-      const int ncb = (nch + kChunksViewsFirst - 1) / kChunksViewsFirst;
-      launch_bins3<BT, false>(g, op, dim3(g.V, ncolb, ncb * ntile), kChunksViewsFirst, views,
-                              cedge, mag, lines, buf0, buf1, output, st);
-    }
+    if (use_cols_first(g, BT))
+      launch_bins3<BT, true>(g, op, views, cedge, mag, lines, buf0, buf1, output, st);
+    else
+      launch_bins3<BT, false>(g, op, views, cedge, mag, lines, buf0, buf1, output, st);
   } else if (L.rows) {
     launch_rows3<BT>(g, op, input, output, views, cedge, mag,
                      reinterpret_cast<const double2*>(geo + L.colz), lines,
