@@ -325,14 +325,14 @@ __global__ __launch_bounds__(kThreads) void k_batch_reduce(
 // One wavefront's share of a gather-pixels item: the staged walk of one pixel
 // tile, over one view chunk (several workgroups per tile) or all of them.
 template <int WM, int NP>
-__device__ __forceinline__ void batch_walk_tile(const BatchInst& d, int tile, int chunk,
+__device__ __forceinline__ void batch_walk_tile(const BatchInst& d, int tile, int chunk, int b0,
                                                 float* __restrict__ out, WalkLds<kBT>& lds) {
   const int tx = (d.g.W + kWalkW - 1) / kWalkW;
   const int c0 = (tile % tx) * kWalkW, r0 = (tile / tx) * 4 * NP;
   const int nc = walk_chunks(d.g.V);
   const int ch0 = d.chunks > 1 ? chunk : 0, ch1 = d.chunks > 1 ? chunk + 1 : nc;
-  float* __restrict__ o =
-      d.chunks > 1 ? d.wpart + static_cast<size_t>(chunk) * d.g.H * d.g.W : out + d.img_off;
+  const size_t n = static_cast<size_t>(d.g.H) * d.g.W;
+  float* __restrict__ o = (d.chunks > 1 ? d.wpart + n * d.g.Bp * chunk : out + d.img_off) + n * b0;
   auto put = [&](int r, int c, int, float v) {
     if (c < d.g.W && r < d.g.H) o[static_cast<size_t>(r) * d.g.W + c] = v;
   };
@@ -341,9 +341,9 @@ __device__ __forceinline__ void batch_walk_tile(const BatchInst& d, int tile, in
 #pragma unroll
     for (int j = 0; j < NP; ++j) acc[j][0] = 0.0f;
     if (!walk_views<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.wrange, d.sino, r0,
-                                 c0, 0, walk_chunk_begin(d.g.V, ch),
+                                 c0, b0, walk_chunk_begin(d.g.V, ch),
                                  walk_chunk_begin(d.g.V, ch + 1), acc, lds)) {
-      walk_views_again<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, r0, c0, 0,
+      walk_views_again<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, r0, c0, b0,
                                     ch0, ch1, put);
       return;
     }
@@ -369,20 +369,24 @@ __global__ __launch_bounds__(kThreads) void k_batch_walk(
     const int local = item - item0_of(mem, i, kGatherPixels);
     if (d.rows > 0) {
       const int chunk = local % d.chunks;
-      const int tile = (local / d.chunks) * (kThreads / 64) + wave;
       const int th = 4 * d.rows;
-      if (tile >= ((d.g.W + kWalkW - 1) / kWalkW) * ((d.g.H + th - 1) / th)) continue;
+      const int tiles = ((d.g.W + kWalkW - 1) / kWalkW) * ((d.g.H + th - 1) / th);
+      const int groups = (tiles + kThreads / 64 - 1) / (kThreads / 64);
+      const int tile = (local / d.chunks) % groups * (kThreads / 64) + wave;
+      const int b0 = local / d.chunks / groups * kBT;
+      if (tile >= tiles) continue;
       if (d.rows == 4)
-        batch_walk_tile<WM, 4>(d, tile, chunk, out, lds[wave]);
+        batch_walk_tile<WM, 4>(d, tile, chunk, b0, out, lds[wave]);
       else
-        batch_walk_tile<WM, 2>(d, tile, chunk, out, lds[wave]);
+        batch_walk_tile<WM, 2>(d, tile, chunk, b0, out, lds[wave]);
     } else {
-      const int tx = (d.g.W + kTile - 1) / kTile;
-      const int c = (local % tx) * kTile + (threadIdx.x % kTile);
-      const int r = (local / tx) * kTile + (threadIdx.x / kTile);
+      const int tx = (d.g.W + kTile - 1) / kTile, ty = (d.g.H + kTile - 1) / kTile;
+      const int t = local % (tx * ty);
+      const int c = (t % tx) * kTile + (threadIdx.x % kTile);
+      const int r = (t / tx) * kTile + (threadIdx.x / kTile);
       if (c < d.g.W && r < d.g.H)
         pixels_body<kBT, WM>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, out + d.img_off,
-                             r, c, 0);
+                             r, c, local / (tx * ty) * kBT);
     }
   }
 }
@@ -394,7 +398,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_sum(
   for (int item = blockIdx.x; item < total; item += gridDim.x) {
     const int i = find_inst(mem, n_inst, kSumPixels, item);
     const BatchInst d = load_inst(mem, i);
-    const size_t n = static_cast<size_t>(d.g.H) * d.g.W;
+    const size_t n = static_cast<size_t>(d.g.H) * d.g.W * d.g.Bp;
     const size_t at = static_cast<size_t>(item - item0_of(mem, i, kSumPixels)) * kThreads +
                       threadIdx.x;
     if (at >= n) continue;
@@ -637,7 +641,7 @@ dd2d_batch* dd2d_batch_create(const dd2d_batch_item* items, int n) {
     } else {
       d.nitems[kGatherPixels] = ((g.W + kTile - 1) / kTile) * ((g.H + kTile - 1) / kTile) * tiles;
     }
-    d.nitems[kSumPixels] = d.chunks > 1 ? (g.W * g.H + kThreads - 1) / kThreads * tiles : 0;
+    d.nitems[kSumPixels] = d.chunks > 1 ? static_cast<int>((img + kThreads - 1) / kThreads) : 0;
     d.nitems[kLayoutPrefix] = (g.H + g.W) * tiles;
     for (int ph = 0; ph < kPhases; ++ph) {
       d.item0[ph] = acc[ph];
