@@ -155,12 +155,15 @@ dd_status dd2d_geometry(int scan, const dd_geom2d* g, const float* angles,
  * along the detector (FP64 knots at the bin edges): each pixel's value from
  * a view is the difference of the running integral at its two edges, found
  * by one merge walk per 4-pixel run.  PROJ_T and BPROJ only (BPROJ_W, whose
- * weight varies per pixel, keeps a walk).  In uneven batches; and in
- * dd2d_run / planned runs at instance tile 1, where the views are split over
- * workgroups (partial images added in order): a 512^2 x 720-view slice's
- * ProjTrans 0.31 ms, the walk 0.37 ms.  Same operator, different rounding:
- * not bit-equal to the walk, so the automatic choice keeps the walk and this
- * variant is selected explicitly or by the autotuner. */
+ * weight varies per pixel, keeps a walk).  In dd2d_run / planned runs at
+ * instance tile 1, where the views are split over workgroups (partial images
+ * added in order): a 512^2 slice of 360 views in 155 us, the walk 165 us; one
+ * of 64^2 in 92 and 22 us.  In uneven batches for the instances whose bins
+ * are too fine for the staged walk; the others keep the walk, which is the
+ * faster there (64 slices of 256^2 to 512^2: 5.6 ms, running sums 7.1 ms).
+ * Same operator, different rounding: not bit-equal to the walk, so the
+ * automatic choice keeps the walk and this variant is selected explicitly or
+ * by the autotuner. */
 #define DD_ADJ_BLOCK_PREFIX 5
 /* Flag OR-ed into a variant: the image -> sinogram ops PROJ and BPROJ_T
  * integrate each bin over each line as a difference of the line's running
@@ -255,7 +258,7 @@ size_t dd2d_batch_device_bytes(const dd2d_batch* b);
  * workgroup per work item). */
 void dd2d_batch_set_grid(dd2d_batch* b, int workgroups);
 /* Sinogram -> image kernel of the batch: a walk variant (the default) or
- * DD_ADJ_BLOCK_PREFIX, optionally OR-ed with DD_FWD_PREFIX for the image ->
+ * DD_ADJ_BLOCK_PREFIX (instances of fine bins), optionally OR-ed with DD_FWD_PREFIX for the image ->
  * sinogram ops. */
 void dd2d_batch_set_variant(dd2d_batch* b, int variant);
 dd_status dd2d_batch_setup(dd2d_batch* b, void* device_mem, size_t bytes,

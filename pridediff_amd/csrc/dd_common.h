@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace dd {
 
 // Per-view geometry shared by all kernels of one call.
@@ -37,7 +39,17 @@ struct LineGeo {
 // device block).
 template <typename T>
 __device__ __forceinline__ T const_load(const T* p) {
-  return *(const __attribute__((address_space(4))) T*)(p);
+  if constexpr (std::is_class_v<T>) {  // as words: a class has no copy from that space
+    struct Words {
+      unsigned w[sizeof(T) / 4];
+    } a;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i)
+      a.w[i] = ((const __attribute__((address_space(4))) unsigned*)(p))[i];
+    return __builtin_bit_cast(T, a);
+  } else {
+    return *(const __attribute__((address_space(4))) T*)(p);
+  }
 }
 
 // Integer pixel + fractional position of an axis point on one line.

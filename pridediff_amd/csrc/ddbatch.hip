@@ -5,13 +5,14 @@
 // detector, view count and angles) and its own slot in one packed image
 // buffer and one packed sinogram buffer.  setup() builds every instance's
 // FP64 geometry tables once and uploads a device descriptor table; run() is
-// then two or three launches per op for the whole batch — a layout phase, a
-// gather phase and, for image -> sinogram ops, the chunk reduction — each a
-// grid over a static list of work items (instance, view, bin block, line
-// chunk), (instance, view, bin block) or (instance, pixel tile), heaviest
-// instances first: by default one workgroup per item, or a set number of
-// workgroups that stride over the list.  No counters, no atomics, no host work: a run is capturable and
-// replays bit-identically.
+// then a few launches per op for the whole batch — a layout phase, a gather
+// phase (sinogram -> image: one launch per tile height of the staged walk and
+// one for instances whose bins are too fine for it) and the sum over chunks —
+// each a grid over a static list of work items (instance, view, bin block,
+// line chunk), (instance, view, bin block) or (instance, pixel tile, view
+// chunk), heaviest instances first: by default one workgroup per item, or a
+// set number of workgroups that stride over the list.  No counters, no
+// atomics, no host work: a run is capturable and replays bit-identically.
 //
 // The per-item arithmetic is the one of the one-call kernels
 // (dd2d_body.h), so a batched result equals the per-instance call exactly.
@@ -49,12 +50,15 @@ enum Phase {
   kLayoutImage = 0,
   kGatherBins = 1,
   kLayoutSino = 2,
-  kGatherPixels = 3,
+  kGatherPixels = 3,  // sinogram -> image by the staged walk, tiles of 16 rows
   kReduceBins = 4,
-  kGatherQuads = 5,   // running-sum sinogram -> image, one thread per 4 x 4 pixels
+  kGatherQuads = 5,   // running-sum sinogram -> image: 4 x 4 pixels a thread, same instances
   kLayoutPrefix = 6,  // running sums of every image row and column
   kSumPixels = 7,     // staged walk: partial images of the view chunks
-  kPhases = 8
+  kGatherShort = 8,   // sinogram -> image by the staged walk, tiles of 8 rows
+  kGatherFine = 9,    // sinogram -> image per pixel: bins too fine to stage
+  kLayoutKnots = 10,  // running sums of the views of those instances
+  kPhases = 11
 };
 
 struct BatchDesc {
@@ -107,7 +111,7 @@ __device__ __forceinline__ int find_inst(const char* __restrict__ mem, int n, in
   int lo = 0, hi = n - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) / 2;
-    if (desc[mid].item0[phase] <= item) lo = mid; else hi = mid - 1;
+    if (const_load(&desc[mid].item0[phase]) <= item) lo = mid; else hi = mid - 1;
   }
   return lo;
 }
@@ -115,33 +119,33 @@ __device__ __forceinline__ int find_inst(const char* __restrict__ mem, int n, in
 __device__ __forceinline__ BatchInst load_inst(char* __restrict__ mem, int i) {
   const BatchDesc& s = reinterpret_cast<const BatchDesc*>(mem)[i];
   BatchInst d;
-  d.g = s.g;
-  d.rows = s.rows;
-  d.chunks = s.chunks;
-  d.wrange = reinterpret_cast<unsigned*>(mem + s.off[kWalkRange]);
-  d.wpart = reinterpret_cast<float*>(mem + s.off[kWalkPart]);
-  d.views = reinterpret_cast<ViewGeo*>(mem + s.off[kViews]);
-  d.edges = reinterpret_cast<double*>(mem + s.off[kEdges]);
-  d.wfp = reinterpret_cast<float*>(mem + s.off[kWfp]);
-  d.lines = reinterpret_cast<LineGeo*>(mem + s.off[kLines]);
-  d.pint = reinterpret_cast<float*>(mem + s.off[kPint]);
-  d.xrow = reinterpret_cast<float*>(mem + s.off[kXrow]);
-  d.xcol = reinterpret_cast<float*>(mem + s.off[kXcol]);
-  d.sino = reinterpret_cast<float*>(mem + s.off[kSino]);
-  d.part = reinterpret_cast<float*>(mem + s.off[kPart]);
-  d.prow = reinterpret_cast<float4*>(mem + s.off[kPrefRow]);
-  d.pcol = reinterpret_cast<float4*>(mem + s.off[kPrefCol]);
-  d.psino = reinterpret_cast<double2*>(mem + s.off[kPrefSino]);
-  d.krange = reinterpret_cast<int2*>(mem + s.off[kKnotRange]);
-  d.img_off = s.img_off;
-  d.sino_off = s.sino_off;
+  d.g = const_load(&s.g);
+  d.rows = const_load(&s.rows);
+  d.chunks = const_load(&s.chunks);
+  d.wrange = reinterpret_cast<unsigned*>(mem + const_load(&s.off[kWalkRange]));
+  d.wpart = reinterpret_cast<float*>(mem + const_load(&s.off[kWalkPart]));
+  d.views = reinterpret_cast<ViewGeo*>(mem + const_load(&s.off[kViews]));
+  d.edges = reinterpret_cast<double*>(mem + const_load(&s.off[kEdges]));
+  d.wfp = reinterpret_cast<float*>(mem + const_load(&s.off[kWfp]));
+  d.lines = reinterpret_cast<LineGeo*>(mem + const_load(&s.off[kLines]));
+  d.pint = reinterpret_cast<float*>(mem + const_load(&s.off[kPint]));
+  d.xrow = reinterpret_cast<float*>(mem + const_load(&s.off[kXrow]));
+  d.xcol = reinterpret_cast<float*>(mem + const_load(&s.off[kXcol]));
+  d.sino = reinterpret_cast<float*>(mem + const_load(&s.off[kSino]));
+  d.part = reinterpret_cast<float*>(mem + const_load(&s.off[kPart]));
+  d.prow = reinterpret_cast<float4*>(mem + const_load(&s.off[kPrefRow]));
+  d.pcol = reinterpret_cast<float4*>(mem + const_load(&s.off[kPrefCol]));
+  d.psino = reinterpret_cast<double2*>(mem + const_load(&s.off[kPrefSino]));
+  d.krange = reinterpret_cast<int2*>(mem + const_load(&s.off[kKnotRange]));
+  d.img_off = const_load(&s.img_off);
+  d.sino_off = const_load(&s.sino_off);
   return d;
 }
 
 // First work item of instance i in a phase (read from the table, not the
 // copy, so a runtime phase index does not put the copy in scratch memory).
 __device__ __forceinline__ int item0_of(const char* __restrict__ mem, int i, int phase) {
-  return reinterpret_cast<const BatchDesc*>(mem)[i].item0[phase];
+  return const_load(&reinterpret_cast<const BatchDesc*>(mem)[i].item0[phase]);
 }
 
 __global__ __launch_bounds__(kThreads) void k_batch_setup(
@@ -161,9 +165,9 @@ __global__ __launch_bounds__(kThreads) void k_batch_setup(
   }
 }
 
-// Per (instance, view): the knot range every 64 x 64 pixel tile of the
-// block items needs (knot_range), for the LDS staging of k_batch_quads_prefix,
-// and the edge range of every 16 x 8 pixels for the staged walk.
+// Per (instance, view): the edge range of every 16 x 8 pixels for the staged
+// walk; where the bins are too fine for it, the knot range of every 64 x 64
+// pixel tile for the LDS staging of k_batch_quads_prefix.
 __global__ __launch_bounds__(kThreads) void k_batch_ranges(char* __restrict__ mem, int n_inst,
                                                            int total) {
   const BatchDesc* __restrict__ desc = reinterpret_cast<const BatchDesc*>(mem);
@@ -175,23 +179,26 @@ __global__ __launch_bounds__(kThreads) void k_batch_ranges(char* __restrict__ me
     }
     const BatchInst d = load_inst(mem, i);
     const int v = item - base;
-    const int tx = (d.g.W + kQuadTile - 1) / kQuadTile;
-    const int tiles = tx * ((d.g.H + kQuadTile - 1) / kQuadTile);
-    const ViewGeo vg = d.views[v];
-    for (int t = threadIdx.x; t < tiles; t += blockDim.x) {
-      const int c0 = (t % tx) * kQuadTile, r0 = (t / tx) * kQuadTile;
-      d.krange[static_cast<size_t>(v) * tiles + t] = knot_range(
-          d.g, vg, d.edges + static_cast<size_t>(v) * (d.g.D + 1),
-          d.lines + static_cast<size_t>(v) * d.g.Lmax, r0, min(r0 + kQuadTile, d.g.H), c0,
-          min(c0 + kQuadTile, d.g.W));
-    }
-    const int wtx = (d.g.W + kWalkW - 1) / kWalkW, wtiles = walk_range_tiles(d.g);
-    for (int t = threadIdx.x; t < wtiles; t += blockDim.x) {
-      const int c0 = (t % wtx) * kWalkW, r0 = (t / wtx) * kWalkRangeH;
-      d.wrange[static_cast<size_t>(v) * wtiles + t] = pack_range(knot_range(
-          d.g, vg, d.edges + static_cast<size_t>(v) * (d.g.D + 1),
-          d.lines + static_cast<size_t>(v) * d.g.Lmax, r0, min(r0 + kWalkRangeH, d.g.H), c0,
-          min(c0 + kWalkW, d.g.W)));
+    const ViewGeo vg = const_load(d.views + v);
+    const double* __restrict__ ev = d.edges + static_cast<size_t>(v) * (d.g.D + 1);
+    const LineGeo* __restrict__ lv = d.lines + static_cast<size_t>(v) * d.g.Lmax;
+    if (d.rows > 0) {
+      const int tx = (d.g.W + kWalkW - 1) / kWalkW, tiles = walk_range_tiles(d.g);
+      for (int t = threadIdx.x; t < tiles; t += blockDim.x) {
+        const int c0 = (t % tx) * kWalkW, r0 = (t / tx) * kWalkRangeH;
+        d.wrange[static_cast<size_t>(v) * tiles + t] =
+            pack_range(knot_range(d.g, vg, ev, lv, r0, min(r0 + kWalkRangeH, d.g.H), c0,
+                                  min(c0 + kWalkW, d.g.W)));
+      }
+    } else {
+      const int tx = (d.g.W + kQuadTile - 1) / kQuadTile;
+      const int tiles = tx * ((d.g.H + kQuadTile - 1) / kQuadTile);
+      for (int t = threadIdx.x; t < tiles; t += blockDim.x) {
+        const int c0 = (t % tx) * kQuadTile, r0 = (t / tx) * kQuadTile;
+        d.krange[static_cast<size_t>(v) * tiles + t] =
+            knot_range(d.g, vg, ev, lv, r0, min(r0 + kQuadTile, d.g.H), c0,
+                       min(c0 + kQuadTile, d.g.W));
+      }
     }
   }
 }
@@ -269,7 +276,7 @@ __global__ __launch_bounds__(kBinsWave) void k_batch_bins(
     const int b0 = (rest / d.g.V) * kBT;
     // the whole wave works every item (the edge exchange needs it); lanes
     // past the last bin use clamped edges and write nothing
-    const ViewGeo vg = d.views[v];
+    const ViewGeo vg = const_load(d.views + v);
     const int L = vg.xaxis ? d.g.H : d.g.W;
     const int N = vg.xaxis ? d.g.W : d.g.H;
     const double e1 = d.edges[static_cast<size_t>(v) * (d.g.D + 1) + min(k, d.g.D)];
@@ -315,7 +322,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_reduce(
     float sum = d.part[at];
 #pragma unroll
     for (int c = 1; c < kSplit; ++c) sum += d.part[c * plane + at];
-    const ViewGeo vg = d.views[v];
+    const ViewGeo vg = const_load(d.views + v);
     const int kk = vg.flip ? d.g.D - 1 - k : k;
     const float wk = (WM == W_FP) ? d.wfp[static_cast<size_t>(v) * d.g.D + k] : 1.0f;
     out[d.sino_off + (static_cast<size_t>(b) * d.g.V + v) * d.g.D + kk] = sum * wk;
@@ -340,9 +347,9 @@ __device__ __forceinline__ void batch_walk_tile(const BatchInst& d, int tile, in
   for (int ch = ch0; ch < ch1; ++ch) {
 #pragma unroll
     for (int j = 0; j < NP; ++j) acc[j][0] = 0.0f;
-    if (!walk_views<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.wrange, d.sino, r0,
-                                 c0, b0, walk_chunk_begin(d.g.V, ch),
-                                 walk_chunk_begin(d.g.V, ch + 1), acc, lds)) {
+    if (!walk_views<kBT, WM, NP, true>(d.g, d.views, d.edges, d.lines, d.pint, d.wrange, d.sino,
+                                       r0, c0, b0, walk_chunk_begin(d.g.V, ch),
+                                       walk_chunk_begin(d.g.V, ch + 1), acc, lds)) {
       walk_views_again<kBT, WM, NP>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, r0, c0, b0,
                                     ch0, ch1, put);
       return;
@@ -355,39 +362,48 @@ __device__ __forceinline__ void batch_walk_tile(const BatchInst& d, int tile, in
   for (int j = 0; j < NP; ++j) put(r0 + (lane >> 4) + 4 * j, c0 + (lane & 15), 0, sum[j]);
 }
 
-// Gather-pixels items: (four pixel tiles, view chunk) of the staged walk, or
-// 16 x 16 pixels of the per-pixel gather where an instance's bins are too
-// fine to be staged.
-template <int WM>
-__global__ __launch_bounds__(kThreads) void k_batch_walk(
+// Gather items of the staged walk: (four pixel tiles, view chunk) of the
+// instances with NP rows per lane.  Bound by VALU issue and LDS latency, so
+// waves count: one kernel for both heights, with views and descriptors in
+// vector registers, had 155 of them (3 waves per SIMD), 8.25 ms for ProjTrans
+// of 64 slices of 256^2 to 512^2; a kernel per height 7.95 (104 registers),
+// views and descriptors through scalar loads (const_load) 5.6 (80).
+template <int WM, int NP>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(WM == W_FP ? 6 : 4))) void k_batch_walk(
     char* __restrict__ mem, int n_inst, int total, float* __restrict__ out) {
+  constexpr int kPhase = NP == 4 ? kGatherPixels : kGatherShort;
   __shared__ WalkLds<kBT> lds[kThreads / 64];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
   for (int item = blockIdx.x; item < total; item += gridDim.x) {
-    const int i = find_inst(mem, n_inst, kGatherPixels, item);
+    const int i = find_inst(mem, n_inst, kPhase, item);
     const BatchInst d = load_inst(mem, i);
-    const int local = item - item0_of(mem, i, kGatherPixels);
-    if (d.rows > 0) {
-      const int chunk = local % d.chunks;
-      const int th = 4 * d.rows;
-      const int tiles = ((d.g.W + kWalkW - 1) / kWalkW) * ((d.g.H + th - 1) / th);
-      const int groups = (tiles + kThreads / 64 - 1) / (kThreads / 64);
-      const int tile = (local / d.chunks) % groups * (kThreads / 64) + wave;
-      const int b0 = local / d.chunks / groups * kBT;
-      if (tile >= tiles) continue;
-      if (d.rows == 4)
-        batch_walk_tile<WM, 4>(d, tile, chunk, b0, out, lds[wave]);
-      else
-        batch_walk_tile<WM, 2>(d, tile, chunk, b0, out, lds[wave]);
-    } else {
-      const int tx = (d.g.W + kTile - 1) / kTile, ty = (d.g.H + kTile - 1) / kTile;
-      const int t = local % (tx * ty);
-      const int c = (t % tx) * kTile + (threadIdx.x % kTile);
-      const int r = (t / tx) * kTile + (threadIdx.x / kTile);
-      if (c < d.g.W && r < d.g.H)
-        pixels_body<kBT, WM>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, out + d.img_off,
-                             r, c, local / (tx * ty) * kBT);
-    }
+    const int local = item - item0_of(mem, i, kPhase);
+    const int tiles = ((d.g.W + kWalkW - 1) / kWalkW) * ((d.g.H + 4 * NP - 1) / (4 * NP));
+    const int groups = (tiles + kThreads / 64 - 1) / (kThreads / 64);
+    const int tile = (local / d.chunks) % groups * (kThreads / 64) + wave;
+    if (tile < tiles)
+      batch_walk_tile<WM, NP>(d, tile, local % d.chunks, local / d.chunks / groups * kBT, out,
+                              lds[wave]);
+  }
+}
+
+// Gather items of the instances whose bins are too fine to be staged: 16 x 16
+// pixels.
+template <int WM>
+__global__ __launch_bounds__(kThreads) void k_batch_pixels(
+    char* __restrict__ mem, int n_inst, int total, float* __restrict__ out) {
+  for (int item = blockIdx.x; item < total; item += gridDim.x) {
+    const int i = find_inst(mem, n_inst, kGatherFine, item);
+    const BatchInst d = load_inst(mem, i);
+    const int local = item - item0_of(mem, i, kGatherFine);
+    const int tx = (d.g.W + kTile - 1) / kTile, ty = (d.g.H + kTile - 1) / kTile;
+    const int t = local % (tx * ty);
+    const int c = (t % tx) * kTile + (threadIdx.x % kTile);
+    const int r = (t / tx) * kTile + (threadIdx.x / kTile);
+    if (c < d.g.W && r < d.g.H)
+      pixels_body<kBT, WM>(d.g, d.views, d.edges, d.lines, d.pint, d.sino, out + d.img_off, r, c,
+                           local / (tx * ty) * kBT);
   }
 }
 
@@ -408,16 +424,16 @@ __global__ __launch_bounds__(kThreads) void k_batch_sum(
   }
 }
 
-// Sinogram running-sum items: the layout items (view, instance), one
-// workgroup per view.
+// Sinogram running-sum items: (view, instance) of the instances whose bins are
+// too fine to be staged, one workgroup per view.
 template <bool FOLD_W>
 __global__ __launch_bounds__(kThreads) void k_batch_prefix_sino(
     char* __restrict__ mem, int n_inst, int total, const float* __restrict__ in) {
   __shared__ double lds[kThreads];
   for (int item = blockIdx.x; item < total; item += gridDim.x) {
-    const int i = find_inst(mem, n_inst, kLayoutSino, item);
+    const int i = find_inst(mem, n_inst, kLayoutKnots, item);
     const BatchInst d = load_inst(mem, i);
-    const int local = item - item0_of(mem, i, kLayoutSino);
+    const int local = item - item0_of(mem, i, kLayoutKnots);
     const int v = local % d.g.V, b = local / d.g.V;
     prefix_sino_view<FOLD_W>(
         d.g, d.views, d.edges, d.wfp, in + d.sino_off + static_cast<size_t>(b) * d.g.V * d.g.D,
@@ -474,7 +490,7 @@ __attribute__((amdgpu_waves_per_eu(5))) void k_batch_quads_prefix(
       const bool mine = v + 1 < d.g.V && staged_n && tid <= rn.y - rn.x;
       if (mine) kn = tab[static_cast<size_t>(vn) * (d.g.D + 1) + rn.x + tid];
       if (active) {
-        const ViewGeo vg = d.views[v];
+        const ViewGeo vg = const_load(d.views + v);
         const LineGeo* __restrict__ lv = d.lines + static_cast<size_t>(v) * d.g.Lmax;
         const float* __restrict__ pv = d.pint + static_cast<size_t>(v) * d.g.Lmax;
         if (staged)
@@ -516,7 +532,7 @@ struct dd2d_batch {
   size_t total_views = 0;
   int total[kPhases] = {};
   int grid = 0;                  // workgroups per launch (0 = one per work item)
-  bool prefix = false;           // sinogram -> image through running sums (DD_ADJ_BLOCK_PREFIX)
+  bool prefix = false;           // fine bins through running sums (DD_ADJ_BLOCK_PREFIX)
   bool fwd_prefix = false;       // image -> sinogram through running sums (DD_FWD_PREFIX)
   char* dev = nullptr;           // device memory given to setup()
 };
@@ -616,31 +632,30 @@ dd2d_batch* dd2d_batch_create(const dd2d_batch_item* items, int n) {
                                      prefix_entries(g.W));
     d.off[kPrefCol] = take(&off, sizeof(float4) * static_cast<size_t>(g.Bp) * g.W *
                                      prefix_entries(g.H));
-    d.off[kPrefSino] =
-        take(&off, sizeof(double2) * static_cast<size_t>(g.Bp) * g.V * (g.D + 1));
-    d.off[kKnotRange] = take(&off, sizeof(int2) * static_cast<size_t>(g.V) *
-                                       ((g.W + kQuadTile - 1) / kQuadTile) *
-                                       ((g.H + kQuadTile - 1) / kQuadTile));
     d.rows = walk_rows(g);
     d.chunks = d.rows > 0 && parts <= kWalkPartBytes ? walk_chunks(g.V) : 1;
-    d.off[kWalkRange] = take(&off, sizeof(unsigned) * g.V * walk_range_tiles(g));
-    d.off[kWalkPart] =
-        d.chunks > 1 ? take(&off, sizeof(float) * static_cast<size_t>(d.chunks) * img) : 0;
+    const int tiles = it.batch;  // kBT == 1
+    const int quads = ((g.W + kQuadTile - 1) / kQuadTile) * ((g.H + kQuadTile - 1) / kQuadTile);
+    d.nitems[kLayoutSino] = g.V * tiles;
+    if (d.rows > 0) {
+      d.off[kWalkRange] = take(&off, sizeof(unsigned) * g.V * walk_range_tiles(g));
+      if (d.chunks > 1)
+        d.off[kWalkPart] = take(&off, sizeof(float) * static_cast<size_t>(d.chunks) * img);
+      const int wt = ((g.W + kWalkW - 1) / kWalkW) * ((g.H + 4 * d.rows - 1) / (4 * d.rows));
+      d.nitems[d.rows == 4 ? kGatherPixels : kGatherShort] = (wt + 3) / 4 * d.chunks * tiles;
+    } else {
+      d.off[kPrefSino] =
+          take(&off, sizeof(double2) * static_cast<size_t>(g.Bp) * g.V * (g.D + 1));
+      d.off[kKnotRange] = take(&off, sizeof(int2) * static_cast<size_t>(g.V) * quads);
+      d.nitems[kGatherFine] = ((g.W + kTile - 1) / kTile) * ((g.H + kTile - 1) / kTile) * tiles;
+      d.nitems[kLayoutKnots] = g.V * tiles;
+      d.nitems[kGatherQuads] = quads * tiles;
+    }
     d.img_off = it.image_offset;
     d.sino_off = it.sino_offset;
-    const int tiles = it.batch;  // kBT == 1
     d.nitems[kLayoutImage] = g.H * tiles;
     d.nitems[kGatherBins] = kSplit * g.V * ((g.D + kBinsPerWave - 1) / kBinsPerWave) * tiles;
     d.nitems[kReduceBins] = g.V * ((g.D + kThreads - 1) / kThreads) * it.batch;
-    d.nitems[kGatherQuads] =
-        ((g.W + kQuadTile - 1) / kQuadTile) * ((g.H + kQuadTile - 1) / kQuadTile) * tiles;
-    d.nitems[kLayoutSino] = g.V * tiles;
-    if (d.rows > 0) {
-      const int wt = ((g.W + kWalkW - 1) / kWalkW) * ((g.H + 4 * d.rows - 1) / (4 * d.rows));
-      d.nitems[kGatherPixels] = (wt + 3) / 4 * d.chunks * tiles;
-    } else {
-      d.nitems[kGatherPixels] = ((g.W + kTile - 1) / kTile) * ((g.H + kTile - 1) / kTile) * tiles;
-    }
     d.nitems[kSumPixels] = d.chunks > 1 ? static_cast<int>((img + kThreads - 1) / kThreads) : 0;
     d.nitems[kLayoutPrefix] = (g.H + g.W) * tiles;
     for (int ph = 0; ph < kPhases; ++ph) {
@@ -744,43 +759,54 @@ dd_status dd2d_batch_run(const dd2d_batch* b, int op, const float* input, float*
                          st, inst, n, rtot, output);
     }
   } else {
-    if (b->prefix && op != DD_BPROJ_W) {
-      // running sums of every view, then one merge walk per 4-pixel run
-      ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
-      const int lt = b->total[kLayoutSino], qt = b->total[kGatherQuads];
+    // The running sums (prefix) take only the instances whose bins are too
+    // fine for the staged walk.  64 slices of 256^2 to 512^2, about one bin per
+    // pixel: running sums 7.1 ms, walk 5.6 ms; 16 of 512^2 2.05 and 2.01 ms, 32
+    // of 64^2 0.24 and 0.03 ms.  At 2 to 6 bins per pixel from 256^2 on, where
+    // a tile's bins no longer fit the staging: 1.16 to 3.5 and, per pixel, 1.74
+    // to 3.6 ms (32 of 256^2, 180 views).
+    const bool prefix = b->prefix && op != DD_BPROJ_W;
+    const int lt = b->total[kLayoutSino], kt = b->total[kLayoutKnots];
+    const int wt = b->total[kGatherPixels], ht = b->total[kGatherShort];
+    const int ft = b->total[kGatherFine], qt = b->total[kGatherQuads];
+    const int stot = b->total[kSumPixels];
+    if (!prefix || wt + ht > 0) {
       if (op == DD_PROJ_T)
-        hipLaunchKernelGGL(k_batch_prefix_sino<true>, dim3(grid_for(b, lt)), dim3(kThreads), 0,
-                           st, inst, n, lt, input);
+        hipLaunchKernelGGL((k_batch_layout<true>), dim3(grid_for(b, lt)), dim3(kThreads), 0, st,
+                           inst, n, static_cast<int>(kLayoutSino), lt, input);
       else
-        hipLaunchKernelGGL(k_batch_prefix_sino<false>, dim3(grid_for(b, lt)), dim3(kThreads), 0,
-                           st, inst, n, lt, input);
-      if (op == DD_PROJ_T)
-        hipLaunchKernelGGL((k_batch_quads_prefix<W_FP>), dim3(grid_for(b, qt)),
-                           dim3(kQuadThreads), 0, st, inst, n, qt, output);
-      else
-        hipLaunchKernelGGL((k_batch_quads_prefix<W_BP>), dim3(grid_for(b, qt)),
-                           dim3(kQuadThreads), 0, st, inst, n, qt, output);
-      return hipGetLastError() == hipSuccess ? DD_OK : DD_LAUNCH_FAIL;
+        hipLaunchKernelGGL((k_batch_layout<false>), dim3(grid_for(b, lt)), dim3(kThreads), 0, st,
+                           inst, n, static_cast<int>(kLayoutSino), lt, input);
     }
-    if (op == DD_PROJ_T)
-      hipLaunchKernelGGL((k_batch_layout<true>), dim3(grid_for(b, b->total[kLayoutSino])),
-                         dim3(kThreads), 0, st, inst, n, static_cast<int>(kLayoutSino),
-                         b->total[kLayoutSino], input);
-    else
-      hipLaunchKernelGGL((k_batch_layout<false>), dim3(grid_for(b, b->total[kLayoutSino])),
-                         dim3(kThreads), 0, st, inst, n, static_cast<int>(kLayoutSino),
-                         b->total[kLayoutSino], input);
     ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
-    const int tot = b->total[kGatherPixels], stot = b->total[kSumPixels];
+    auto run = [&](auto wm) {
+      constexpr int WM = decltype(wm)::value;
+      if (wt > 0)
+        hipLaunchKernelGGL((k_batch_walk<WM, 4>), dim3(grid_for(b, wt)), dim3(kThreads), 0, st,
+                           inst, n, wt, output);
+      if (ht > 0)
+        hipLaunchKernelGGL((k_batch_walk<WM, 2>), dim3(grid_for(b, ht)), dim3(kThreads), 0, st,
+                           inst, n, ht, output);
+      if (ft == 0) return;
+      if constexpr (WM != W_BPW) {
+        if (prefix) {
+          // running sums of every view, then one merge walk per 4-pixel run
+          hipLaunchKernelGGL((k_batch_prefix_sino<WM == W_FP>), dim3(grid_for(b, kt)),
+                             dim3(kThreads), 0, st, inst, n, kt, input);
+          hipLaunchKernelGGL((k_batch_quads_prefix<WM>), dim3(grid_for(b, qt)),
+                             dim3(kQuadThreads), 0, st, inst, n, qt, output);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((k_batch_pixels<WM>), dim3(grid_for(b, ft)), dim3(kThreads), 0, st,
+                         inst, n, ft, output);
+    };
     if (op == DD_PROJ_T)
-      hipLaunchKernelGGL((k_batch_walk<W_FP>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
-                         inst, n, tot, output);
+      run(std::integral_constant<int, W_FP>{});
     else if (op == DD_BPROJ)
-      hipLaunchKernelGGL((k_batch_walk<W_BP>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
-                         inst, n, tot, output);
+      run(std::integral_constant<int, W_BP>{});
     else
-      hipLaunchKernelGGL((k_batch_walk<W_BPW>), dim3(grid_for(b, tot)), dim3(kThreads), 0, st,
-                         inst, n, tot, output);
+      run(std::integral_constant<int, W_BPW>{});
     if (stot > 0)
       hipLaunchKernelGGL(k_batch_sum, dim3(grid_for(b, stot)), dim3(kThreads), 0, st, inst, n,
                          stot, output);

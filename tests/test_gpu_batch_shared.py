@@ -93,3 +93,33 @@ def test_slices_of_an_instance_equal_their_own_calls(lib, scan):
             torch.cuda.synchronize()
     finally:
         lib.dd2d_batch_destroy(b)
+
+
+@pytest.mark.parametrize("scan", [0, 1, 2])
+def test_running_sum_variant_keeps_the_walk_where_bins_are_staged(lib, scan):
+    """DD_ADJ_BLOCK_PREFIX: the staged instances' pixels are the walk's bit for
+    bit; with finer bins (2 a pixel: staged in parallel beam only) they are
+    running sums, within 1e-6 relative L2 of the walk (knots in FP64, one
+    rounding to FP32 a view)."""
+    b, items, images, sinos, keep, stream = _batch(lib, scan)
+    gen = torch.Generator(device="cuda").manual_seed(15 + scan)
+    y = torch.rand(sinos, device="cuda", generator=gen)
+    try:
+        for op in (1, 2):
+            got = []
+            for variant in (0, 5):
+                lib.dd2d_batch_set_variant(b, variant)
+                out = torch.full((images,), float("nan"), device="cuda")
+                assert lib.dd2d_batch_run(b, op, y.data_ptr(), out.data_ptr(), stream) == DD_OK
+                got.append(out)
+            for it, (w, h, _, fine, _, k) in zip(items, SHAPES):
+                walk, sums = (o[it.image_offset:][:k * w * h] for o in got)
+                print(f"scan {scan} op {op} {w}x{h}: {float((walk - sums).norm() / walk.norm()):.2e}",
+                      flush=True)
+                if fine < 2.0:
+                    assert torch.equal(walk, sums)
+                else:
+                    assert (walk - sums).norm() <= 1e-6 * walk.norm()
+            torch.cuda.synchronize()
+    finally:
+        lib.dd2d_batch_destroy(b)
