@@ -123,11 +123,22 @@ bool make_shape(const dd_shape* in, Shape* out) {
 // ---------------------------------------------------------------------------
 // one-call kernels: thin grids over the shared bodies
 // ---------------------------------------------------------------------------
+// ranges: the staged walk's edge range of every 16 x 8 pixels of the view,
+// ranges[v * tiles + t] (null: not needed), from the tables that the workgroup
+// has just written.  A launch of its own with a thread per range took 5 us at
+// 256 x 256 x 180 views and 18 us at 512 x 512 x 720, of which the loop here
+// saves 3 us of the step and none.
 __global__ __launch_bounds__(kThreads) void k_setup2d(
     Geo2 g, const float* __restrict__ angles, ViewGeo* __restrict__ views,
     double* __restrict__ edges, float* __restrict__ wfp,
-    LineGeo* __restrict__ lines, float* __restrict__ pint) {
-  setup2d_view(g, angles, views, edges, wfp, lines, pint, blockIdx.x);
+    LineGeo* __restrict__ lines, float* __restrict__ pint, unsigned* __restrict__ ranges) {
+  const int v = blockIdx.x;
+  setup2d_view(g, angles, views, edges, wfp, lines, pint, v);
+  if (!ranges) return;
+  __syncthreads();
+  walk_ranges_view(g, views[v], edges + static_cast<size_t>(v) * (g.D + 1),
+                   lines + static_cast<size_t>(v) * g.Lmax,
+                   ranges + static_cast<size_t>(v) * walk_range_tiles(g));
 }
 
 // x [B][H][W] -> the row copy and the column copy, by 16 x 16 pixel tiles.
@@ -277,22 +288,6 @@ __global__ __launch_bounds__(kThreads) void k_pixels(
   const int r = blockIdx.y * TH + ty;
   if (c >= g.W || r >= g.H) return;
   pixels_body<BT, WM>(g, views, edges, lines, pint, sino, out, r, c, blockIdx.z * BT, ep);
-}
-
-// Edge range of every (view, 16 x 8 pixels): ranges[v * tiles + t].
-__global__ __launch_bounds__(kThreads) void k_walk_ranges(
-    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
-    const LineGeo* __restrict__ lines, unsigned* __restrict__ ranges) {
-  const int tx = (g.W + kWalkW - 1) / kWalkW;
-  const int tiles = walk_range_tiles(g);
-  const long long idx = 1LL * blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= 1LL * tiles * g.V) return;
-  const int v = static_cast<int>(idx / tiles), t = static_cast<int>(idx % tiles);
-  const int c0 = (t % tx) * kWalkW, r0 = (t / tx) * kWalkRangeH;
-  ranges[idx] = pack_range(knot_range(
-      g, views[v], edges + static_cast<size_t>(v) * (g.D + 1),
-      lines + static_cast<size_t>(v) * g.Lmax, r0, min(r0 + kWalkRangeH, g.H), c0,
-      min(c0 + kWalkW, g.W)));
 }
 
 // sinogram -> image by the staged walk: one wavefront per pixel tile.  SPLIT:
@@ -774,14 +769,9 @@ void launch_setup(const Geo2& g, const float* angles, void* geo,
                      reinterpret_cast<double*>(b + L.edges),
                      reinterpret_cast<float*>(b + L.wfp),
                      reinterpret_cast<LineGeo*>(b + L.lines),
-                     reinterpret_cast<float*>(b + L.pint));
-  if (!ranges || !L.has_ranges) return;
-  const long long n = 1LL * g.V * walk_range_tiles(g);
-  hipLaunchKernelGGL(k_walk_ranges, dim3(static_cast<unsigned>((n + kThreads - 1) / kThreads)),
-                     dim3(kThreads), 0, st, g, reinterpret_cast<const ViewGeo*>(b + L.views),
-                     reinterpret_cast<const double*>(b + L.edges),
-                     reinterpret_cast<const LineGeo*>(b + L.lines),
-                     reinterpret_cast<unsigned*>(b + L.wranges));
+                     reinterpret_cast<float*>(b + L.pint),
+                     ranges && L.has_ranges ? reinterpret_cast<unsigned*>(b + L.wranges)
+                                            : nullptr);
 }
 
 // Staged walk of the sinogram -> image ops.
@@ -1194,7 +1184,7 @@ bool sys_setup(int scan, const dd_geom2d* g, const float* angles, int views,
                      reinterpret_cast<double*>(w + L->edges),
                      reinterpret_cast<float*>(w + L->wfp),
                      reinterpret_cast<LineGeo*>(w + L->lines),
-                     reinterpret_cast<float*>(w + L->pint));
+                     reinterpret_cast<float*>(w + L->pint), static_cast<unsigned*>(nullptr));
   return true;
 }
 }  // namespace

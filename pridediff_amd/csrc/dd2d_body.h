@@ -969,6 +969,19 @@ __device__ __forceinline__ unsigned pack_range(int2 r) {
          static_cast<unsigned>(n > kWalkSlots || r.x >= (1 << 24) ? 255 : n);
 }
 
+// The range table of one view, by one workgroup.
+__device__ __forceinline__ void walk_ranges_view(const Geo2& g, const ViewGeo& vg,
+                                                 const double* __restrict__ ev,
+                                                 const LineGeo* __restrict__ lv,
+                                                 unsigned* __restrict__ out) {
+  const int tx = (g.W + kWalkW - 1) / kWalkW, tiles = walk_range_tiles(g);
+  for (int t = threadIdx.x; t < tiles; t += blockDim.x) {
+    const int c0 = (t % tx) * kWalkW, r0 = (t / tx) * kWalkRangeH;
+    out[t] = pack_range(
+        knot_range(g, vg, ev, lv, r0, min(r0 + kWalkRangeH, g.H), c0, min(c0 + kWalkW, g.W)));
+  }
+}
+
 // Rows per lane of the staged walk (tiles of 16 x 4 rows pixels), or 0 where
 // the per-pixel kernel takes the op.  A taller tile shares each staged view
 // over more pixels, but its edges have to fit the slots: a tile's diagonal
@@ -1131,7 +1144,7 @@ __device__ __forceinline__ void walk_window(
 // per-pixel walk it replaces searched and placed three to five edges per
 // pixel in FP64 from global memory, one after the other, at about 200
 // instructions.  ProjTrans of 512 x 512 x 720 views x 736 bins: one slice
-// 1087 -> 372 us, 16 slices 1573 -> 760 us; 256 x 256 x 180 views parallel
+// 1087 -> 350 us, 16 slices 1573 -> 939 us; 256 x 256 x 180 views parallel
 // 206 -> 43 us.
 // AXES: a window of its own for each direction of the lines.  Uneven batches
 // gain 2.5 % by it (64 slices of 256^2 to 512^2: 5.73 -> 5.58 ms); a single

@@ -183,13 +183,8 @@ __global__ __launch_bounds__(kThreads) void k_batch_ranges(char* __restrict__ me
     const double* __restrict__ ev = d.edges + static_cast<size_t>(v) * (d.g.D + 1);
     const LineGeo* __restrict__ lv = d.lines + static_cast<size_t>(v) * d.g.Lmax;
     if (d.rows > 0) {
-      const int tx = (d.g.W + kWalkW - 1) / kWalkW, tiles = walk_range_tiles(d.g);
-      for (int t = threadIdx.x; t < tiles; t += blockDim.x) {
-        const int c0 = (t % tx) * kWalkW, r0 = (t / tx) * kWalkRangeH;
-        d.wrange[static_cast<size_t>(v) * tiles + t] =
-            pack_range(knot_range(d.g, vg, ev, lv, r0, min(r0 + kWalkRangeH, d.g.H), c0,
-                                  min(c0 + kWalkW, d.g.W)));
-      }
+      walk_ranges_view(d.g, vg, ev, lv,
+                       d.wrange + static_cast<size_t>(v) * walk_range_tiles(d.g));
     } else {
       const int tx = (d.g.W + kQuadTile - 1) / kQuadTile;
       const int tiles = tx * ((d.g.H + kQuadTile - 1) / kQuadTile);
