@@ -151,27 +151,22 @@ def roofline_for(key, kernel, ms, b_alg, step_ms=None, n_ops=2):
 # Counter groups per workload: key -> kernels whose dispatches make up one
 # HIP-event-timed launch of that key (a forward is gather + chunk reduction).
 COUNTER_KEYS = {
-    "fanarc": {"fanarc_b16:k_pixels<16,0>": ["k_pixels<16, 0, "],
-               "fanarc_b16:k_pixels_walk<16,0>": ["k_pixels_walk<16, 0, "],
+    "fanarc": {"fanarc_b16:k_pixels_walk<16,0>": ["k_pixels_walk<16, 0, "],
                "fanarc_b16:k_bins_split<16,0>": ["k_bins_split<16, 0>", "k_bins_reduce<0>"],
-               "fanarc_plain:k_pixels<1,0>": ["k_pixels<1, 0, "],
                "fanarc_plain:k_pixels_walk<1,0>": ["k_pixels_walk<1, 0, "],
                "fanarc_plain:k_bins_split<1,0>": ["k_bins_split<1, 0>", "k_bins_reduce<0>"],
                "fanarc_plain:k_pixels_prefix<0>": ["k_prefix_sino<true>", "k_prefix_ranges",
                                                    "k_pixels_prefix<0>", "k_sum_chunks"],
                "fanarc_plain:k_bins_prefix<0>": ["k_prefix_lines", "k_bins_prefix<0>",
                                                  "k_bins_reduce<0>"]},
-    "uneven": {"uneven64:k_batch_quads_window": ["k_batch_quads<0, 8>"],
-               "uneven64:k_batch_quads": ["k_batch_quads<0, 0>"],
-               "uneven64:k_batch_quads_prefix": ["k_batch_prefix_sino<true>",
-                                                 "k_batch_quads_prefix<0>"],
+    "uneven": {"uneven64:k_batch_walk": ["k_batch_walk<0, 4>"],
                "uneven64:k_batch_bins": ["k_batch_bins<0, false>", "k_batch_reduce<0>"],
                "uneven64:k_batch_bins_prefix": ["k_batch_prefix", "k_batch_bins<0, true>",
                                                 "k_batch_reduce<0>"]},
-    "cone_flat": {"cone_flat:k_voxels3d": ["k_voxel_ranges", "k_voxels3d<2, 0, true, true>"],
-                  "cone_flat:k_bins3d": ["k_bins3d<2, 0, false>"]},
-    "helical": {"helical:k_voxels3d": ["k_voxels3d<4, 0, false, false>"],
-                "helical:k_bins3d": ["k_bins3d<4, 0, true>"]},
+    "cone_flat": {"cone_flat:k_voxel_rows": ["k_row_ranges<2>", "k_voxel_rows<2, 0>"],
+                  "cone_flat:k_bins3d": ["k_bins3d<2, 0, 16, false>"]},
+    "helical": {"helical:k_voxel_rows": ["k_row_ranges<4>", "k_voxel_rows<4, 0>"],
+                "helical:k_bins3d": ["k_bins3d<4, 0, 8, true>"]},
 }
 
 
@@ -388,8 +383,7 @@ def uneven_c2(torch, dev, steps, warmup, check, tune_grid=True, cpu=False, varia
            "forward_ms": fp_ms / max(fp_n, 1), "adjoint_ms": bp_ms / max(bp_n, 1)}
     var = tune.get("variant", rt.ADJ_QUAD)
     out["forward_kernel"] = "running sums" if var & rt.FWD_PREFIX else "pixel walk"
-    adj_name = ("k_batch_quads_prefix" if var & ~rt.FWD_PREFIX == rt.ADJ_BLOCK_PREFIX
-                else "k_batch_walk")
+    adj_name = "k_batch_walk"  # every instance here can be staged, whatever the variant
     fwd_name = "k_batch_bins_prefix" if var & rt.FWD_PREFIX else "k_batch_bins"
     dom = ((fwd_name, out["forward_ms"]) if out["forward_ms"] >= out["adjoint_ms"]
            else (adj_name, out["adjoint_ms"]))
@@ -521,7 +515,7 @@ def bench3d(torch, kind, steps, warmup, check, dc_loop=True):
         sl = np.count_nonzero((z_edges[1:] > lo) & (z_edges[:-1] < hi))
         in_cone += sl * W * H
     b_alg = 4.0 * (in_cone + V * R * C) * Bn  # bytes per operator launch
-    dom_ms, dom = (fp_ms, "k_bins3d") if fp_ms >= bp_ms else (bp_ms, "k_voxels3d")
+    dom_ms, dom = (fp_ms, "k_bins3d") if fp_ms >= bp_ms else (bp_ms, "k_voxel_rows")
     samples = Bn * V * R * C
     out = {
         "metric": "FP+BP detector samples/s & %HBM roofline (3D)",
@@ -534,8 +528,8 @@ def bench3d(torch, kind, steps, warmup, check, dc_loop=True):
         "roofline": dict(roofline_for(f"{kind}:{dom}", dom, dom_ms, b_alg, t * 1e3),
                          in_cone_voxel_views=in_cone),
         "kernels": {"k_bins3d (A, volume->sino)": {"ms": fp_ms, "effective_GBps": b_alg / fp_ms / 1e6},
-                    "k_voxels3d (A^T, sino->volume)": {"ms": bp_ms,
-                                                       "effective_GBps": b_alg / bp_ms / 1e6}},
+                    "k_voxel_rows (A^T, sino->volume)": {"ms": bp_ms,
+                                                         "effective_GBps": b_alg / bp_ms / 1e6}},
         "cpu_baseline": None,
     }
     if loop_out is not None:
@@ -567,10 +561,11 @@ def bench3d(torch, kind, steps, warmup, check, dc_loop=True):
                         a_sub, g, s_sub)
         acc = {"views_checked": sel.tolist(),
                "fp_rel_l2_vs_fp64": O.rel_l2(got, want), "fp_max_abs_vs_fp64": O.max_abs(got, want)}
-        # the adjoint with compensated running sums (the default) and with
-        # running sums rounded to FP32, accuracy and kernel time of each
-        for comp in (True, False):
-            rt.set_compensated3d(1 if comp else 0)
+        # the adjoint by detector rows (the default), with compensated running
+        # sums and with running sums rounded to FP32, accuracy and kernel time
+        # of each
+        for mode, tag in ((2, "rows"), (1, "compensated"), (0, "rounded")):
+            rt.set_compensated3d(mode)
             with torch.no_grad():
                 got_t = P.projection_t(ysp, ang, *sp_args)[:1, 0].cpu().numpy()
                 rt.profile_enable(True)
@@ -580,15 +575,11 @@ def bench3d(torch, kind, steps, warmup, check, dc_loop=True):
                 torch.cuda.synchronize()
                 ms, n = rt.profile_read(1)
                 rt.profile_enable(False)
-            tag = "compensated" if comp else "rounded"
             acc[f"adjoint_{tag}"] = {"rel_l2_vs_fp64": O.rel_l2(got_t, want_t),
                                      "max_abs_vs_fp64": O.max_abs(got_t, want_t),
-                                     "k_voxels3d_ms": ms / max(n, 1)}
+                                     "kernel_ms": ms / max(n, 1)}
         rt.set_compensated3d(2)
-        acc["default_mode"] = ("compensated" if Bn <= 2 else "rounded") + \
-            " (automatic: compensated at instance tiles 1-2)"
-        acc["lds_staging"] = ("on" if Bn <= 2 else "on for compensated sums only") + \
-            " (automatic: compensated sums or instance tiles 1-2; same bits either way)"
+        acc["default_mode"] = "rows"
         out["accuracy"] = acc
     return out
 

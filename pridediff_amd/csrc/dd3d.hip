@@ -15,13 +15,18 @@
 //   k_interleave_volume  volume -> [tile][line][slice][pixel][b] copies (rows
 //                        and bottom-up columns) for image -> sinogram ops;
 //   k_bins3d             image -> sinogram: one thread per detector column and
-//                        chunk of rows, gathering over the lines its ray band
-//                        meets in z;
-//   k_prefix_sino3d      sinogram -> per-column running sums over detector
-//                        rows, [view][row][col][b] (x FP weight);
-//   k_voxels3d           sinogram -> image: one thread per pixel and chunk of
-//                        slices, gathering over views; the row/slice overlap
-//                        sums come from differences of the running sums.
+//                        chunk of rows, gathering row by row over the lines
+//                        its ray band meets in z (k_bins3d_slices: slice by
+//                        slice, rows thicker than two slices);
+//   k_interleave_sino3d  sinogram -> [view][row][col][b] (x FP weight);
+//   k_row_ranges         per view and pixel tile: the columns to be staged;
+//   k_voxel_rows         sinogram -> image: one thread per pixel and chunk of
+//                        slices, gathering over views the one to three rows
+//                        that each slice overlaps, staged in LDS;
+//                        k_sum_volumes adds the parts of split views.
+// Thick slices, and the two running-sum modes, instead of the last three:
+//   k_prefix_sino3d      per-column running sums over detector rows;
+//   k_voxels3d           the row/slice overlap sums as differences of them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
