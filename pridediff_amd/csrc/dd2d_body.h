@@ -824,8 +824,8 @@ __device__ __forceinline__ void pixel_run_view_prefix(
 }
 
 // One view's contribution to the Q x Q pixel block at (r0, c0) (nr x nc of
-// it inside the image) through the view's knots (pixel_run_view_prefix);
-// the block's lines as in blocks_body.  WM is W_FP or W_BP.
+// it inside the image) through the view's knots (pixel_run_view_prefix).
+// WM is W_FP or W_BP.
 template <int WM, int Q, typename KP>
 __device__ __forceinline__ void block_view_prefix(
     const Geo2& g, const ViewGeo& vg, const LineGeo* __restrict__ lv,
