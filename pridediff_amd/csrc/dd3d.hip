@@ -602,12 +602,20 @@ constexpr int line_batch3() {
   return BT >= 4 ? 4 : BT == 2 ? 0 : S == 8 ? 2 : 3;
 }
 
+// The row gathers below step from edge u_j to edge u_{j+1} = u_j + d, both
+// rounded to FP32, and read the K cells from floor(u_j) to floor(u_{j+1}): at
+// d = K - 1 exactly, rounding could carry the second edge past one more cell,
+// and the rest of the weight with it, to a cell that the row does not meet.
+// Edges lie below 64 (at most 16 steps of at most 3 from below 1), so each
+// is off by at most 2^-19: K cells hold d <= K - 1 - kEdgeSlack3.
+constexpr float kEdgeSlack3 = 0x1p-17f;
+
 // One line's share of a detector column's S rows, by rows: n <= NX pixels from
 // px on (weights wx), summed over x slice by slice as the rows meet them.  Row
 // edge j lies at slice coordinate t_j = dt + j d relative to slice `base`,
 // so row j holds d slices from t_j on: min(d, 1 - fraction) of slice
 // floor(t_j), then whole slices, then the rest, K slices in all
-// (d <= K - 1); the last of them is the first of the next row, so it is read
+// (d <= K - 1 - kEdgeSlack3); the last of them is the first of the next row, so it is read
 // once.  K = 0: any d, every slice of a row read for itself (a source that
 // comes nearer than the geometry's own radius, which the host does not see).
 // Slices outside the volume are its zero slices.
@@ -785,9 +793,9 @@ __attribute__((amdgpu_waves_per_eu(line_waves3<BT, S>()))) void k_bins3d(
         }
       }
     };
-    if (__all(d <= 1.0f))
+    if (__all(d <= 1.0f - kEdgeSlack3))
       rows(std::integral_constant<int, 2>{});
-    else if (__all(d <= 2.0f))
+    else if (__all(d <= 2.0f - kEdgeSlack3))
       rows(std::integral_constant<int, 3>{});
     else
       rows(std::integral_constant<int, 0>{});
@@ -1451,8 +1459,8 @@ __global__ __launch_bounds__(kThreads3) void k_row_ranges(
 // Adds one detector column's rows to S consecutive slices.  Slice edge j lies
 // at row coordinate u_j = du + j d (relative to a base row), so slice j holds
 // d rows from u_j on: w_0 = min(d, 1 - fraction) of row floor(u_j), then
-// whole rows, then the rest, K rows in all (d <= K - 1); each weight times
-// its row, times wx.  The last of them is row floor(u_{j+1}), the first of
+// whole rows, then the rest, K rows in all (d <= K - 1 - kEdgeSlack3); each
+// weight times its row, times wx.  The last of them is row floor(u_{j+1}), the first of
 // the next slice, so it is read once: one row per slice at K = 2, two at 3.
 // row(fl, m, x) gives row fl + m.
 template <int BT, int S, int K, typename Row>
@@ -1544,11 +1552,11 @@ __device__ __forceinline__ void gather_rows(const Geo3& g, const ViewGeo3& vg,
     const float d = static_cast<float>(lg.pz * z.x);
     const float wx = (p2 - p1) * gw * static_cast<float>(z.y * lg.inv_pz);
     const auto row_at = rows(k, rbase);
-    if (__all(d <= 1.0f))
+    if (__all(d <= 1.0f - kEdgeSlack3))
       column_slices<BT, S, 2>(du, d, wx, row_at, acc);
-    else if (__all(d <= 2.0f))
+    else if (__all(d <= 2.0f - kEdgeSlack3))
       column_slices<BT, S, 3>(du, d, wx, row_at, acc);
-    else if (__all(d <= 3.0f))
+    else if (__all(d <= 3.0f - kEdgeSlack3))
       column_slices<BT, S, 4>(du, d, wx, row_at, acc);
     else
       column_slices_any<BT, S>(du, d, wx, row_at, acc);
