@@ -616,9 +616,10 @@ constexpr float kEdgeSlack3 = 0x1p-17f;
 // so row j holds d slices from t_j on: min(d, 1 - fraction) of slice
 // floor(t_j), then whole slices, then the rest, K slices in all
 // (d <= K - 1 - kEdgeSlack3); the last of them is the first of the next row, so it is read
-// once.  K = 0: any d, every slice of a row read for itself (a source that
-// comes nearer than the geometry's own radius, which the host does not see).
-// Slices outside the volume are its zero slices.
+// once.  K = 0: any d, every slice of a row read for itself (a source distance
+// that differs from the geometry's own, which the host does not see), between
+// the row's edges held to the volume: no d makes more steps than there are
+// slices.  Slices outside the volume are its zero slices.
 template <int BT, int S, int K, int NX>
 __device__ __forceinline__ void line_rows(const float* __restrict__ px, int sstride, int base,
                                           int Dz, float dt, float d, const float (&wx)[NX],
@@ -650,18 +651,19 @@ __device__ __forceinline__ void line_rows(const float* __restrict__ px, int sstr
   };
   float fl = floorf(dt), f = dt - fl;
   if constexpr (K == 0) {
+    const float first = static_cast<float>(-base);
+    float e = __builtin_amdgcn_fmed3f(dt, first, hi);
 #pragma unroll
     for (int j = 0; j < S; ++j) {
-      const float t = fmaf(static_cast<float>(j), d, dt);
-      fl = floorf(t);
-      float w = fminf(d, 1.0f - (t - fl)), rest = d;
-      for (float s = fl; rest > 0.0f; s += 1.0f) {
+      const float a = e;
+      e = __builtin_amdgcn_fmed3f(fmaf(static_cast<float>(j + 1), d, dt), first, hi);
+      for (int s = static_cast<int>(floorf(a)); static_cast<float>(s) < e; ++s) {
+        const float sf = static_cast<float>(s);
+        const float w = fminf(e, sf + 1.0f) - fmaxf(a, sf);
         float x[BT];
-        slice(s, x);
+        slice(sf, x);
 #pragma unroll
         for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(w, x[b], acc[j][b]);
-        rest -= w;
-        w = fminf(rest, 1.0f);
       }
     }
     return;
@@ -1323,26 +1325,29 @@ __attribute__((amdgpu_waves_per_eu(adj_waves3<BT>()))) void k_voxels3d(
 // ---------------------------------------------------------------------------
 // sinogram -> image by detector rows: slices no thicker than a few rows
 // ---------------------------------------------------------------------------
-// The same for any d (a source that comes nearer than the geometry's own
-// radius, which the host does not see): every row of a slice read for itself.
+// The same for any d (a source distance that differs from the geometry's own,
+// which the host does not see): every row of a slice read for itself, between
+// the slice's edges held to rows [lo, hi), so that no d makes more steps than
+// there are rows.
 template <int BT, int S, typename Row>
-__device__ __forceinline__ void column_slices_any(float du, float d, float wx, Row row,
-                                                  float (&acc)[S][BT]) {
+__device__ __forceinline__ void column_slices_any(float du, float d, float wx, float lo,
+                                                  float hi, Row row, float (&acc)[S][BT]) {
   asm volatile("; any rows" : "+v"(du));
+  float e = __builtin_amdgcn_fmed3f(du, lo, hi);
 #pragma unroll
   for (int j = 0; j < S; ++j) {
-    const float u = fmaf(static_cast<float>(j), d, du);
-    const float fl = floorf(u);
-    float t[BT], w = fminf(d, 1.0f - (u - fl)), rest = d;
+    const float a = e;
+    e = __builtin_amdgcn_fmed3f(fmaf(static_cast<float>(j + 1), d, du), lo, hi);
+    float t[BT];
 #pragma unroll
     for (int b = 0; b < BT; ++b) t[b] = 0.0f;
-    for (int m = 0; rest > 0.0f; ++m) {
+    for (int r = static_cast<int>(floorf(a)); static_cast<float>(r) < e; ++r) {
+      const float rf = static_cast<float>(r);
+      const float w = fminf(e, rf + 1.0f) - fmaxf(a, rf);
       float x[BT];
-      row(fl, m, x);
+      row(rf, 0, x);
 #pragma unroll
       for (int b = 0; b < BT; ++b) t[b] = fmaf(w, x[b], t[b]);
-      rest -= w;
-      w = fminf(rest, 1.0f);
     }
 #pragma unroll
     for (int b = 0; b < BT; ++b) acc[j][b] = fmaf(wx, t[b], acc[j][b]);
@@ -1510,12 +1515,13 @@ __device__ __forceinline__ void column_slices(float du, float d, float wx, Row r
 
 // One view's rows into the pixel (row, col)'s slices s0 .. s0 + S - 1,
 // columns [kmin, kend) (column k of the detector being k + koff), through the
-// given accessors: edge k, z law of column k, and one column's rows.
+// given accessors: edge k, z law of column k, and one column's rows (rows
+// outside [rlo, rhi) are zero).
 template <int BT, int WM, int S, typename Edge, typename ZLaw, typename Rows>
 __device__ __forceinline__ void gather_rows(const Geo3& g, const ViewGeo3& vg,
                                             const LineGeo3& lg, int row, int col, int s0,
                                             int kmin, int kend, Edge edge, ZLaw zlaw, Rows rows,
-                                            float (&acc)[S][BT], int koff) {
+                                            int rlo, int rhi, float (&acc)[S][BT], int koff) {
   const int i = vg.xaxis ? col : g.H - 1 - row;
   const PixelFrame fr(lg.a0, lg.inv_p, i);
   // first column: the last whose lower edge lies before pixel i (or kmin);
@@ -1559,7 +1565,8 @@ __device__ __forceinline__ void gather_rows(const Geo3& g, const ViewGeo3& vg,
     else if (__all(d <= 3.0f - kEdgeSlack3))
       column_slices<BT, S, 4>(du, d, wx, row_at, acc);
     else
-      column_slices_any<BT, S>(du, d, wx, row_at, acc);
+      column_slices_any<BT, S>(du, d, wx, static_cast<float>(rlo - rbase),
+                               static_cast<float>(rhi - rbase), row_at, acc);
     if (++k >= kend) break;
     u1 = u2;
     p1 = p2;
@@ -1702,7 +1709,7 @@ __attribute__((amdgpu_waves_per_eu(row_waves3<BT>()))) void k_voxel_rows(
             load_tile<BT>(reinterpret_cast<const float*>(lq + at) + m * (kStep / 4), x);
           };
         },
-        acc, skb);
+        srb, srb + nrow, acc, skb);
   }
   const int col = tc + tx, row = tr + ty;
   if (col >= g.W || row >= g.H) return;
@@ -1767,7 +1774,7 @@ __global__ __launch_bounds__(kThreads3) void k_voxel_rows_global(
               for (int b = 0; b < BT; ++b) x[b] = in ? x[b] : 0.0f;
             };
           },
-          acc, 0);
+          0, g.R, acc, 0);
     }
     if (!any) continue;
     if (ranges)
