@@ -620,6 +620,7 @@ constexpr float kEdgeSlack3 = 0x1p-17f;
 // that differs from the geometry's own, which the host does not see), between
 // the row's edges held to the volume: no d makes more steps than there are
 // slices.  Slices outside the volume are its zero slices.
+// Offsets of a line's slices are 32-bit (use_line_rows3).
 template <int BT, int S, int K, int NX>
 __device__ __forceinline__ void line_rows(const float* __restrict__ px, int sstride, int base,
                                           int Dz, float dt, float d, const float (&wx)[NX],
@@ -2030,8 +2031,12 @@ bool use_cols_first(const Geo3& g, int bt) {
 }
 
 // Whether the volume -> sinogram ops go row by row: rows at most two slices
-// thick at the volume's far corner.  Thicker rows go slice by slice.
+// thick at the volume's far corner, and lines whose slices line_rows can
+// address (24-bit factors, one line's slices within 2 GiB).  Others go slice
+// by slice.
 bool use_line_rows3(const Geo3& g) {
+  const long long slice = 4LL * std::max(g.W, g.H) * g.BT;  // bytes of one line's slice
+  if (g.Dz >= 1 << 22 || slice >= 1LL << 23 || slice * (g.Dz + 1) >= 1LL << 31) return false;
   const double half = 0.5 * std::hypot(g.W * g.dx, g.H * g.dy) + std::hypot(g.shx, g.shy);
   return g.row > 0.0f && g.dz > 0.0f && g.sdd > 0.0f &&
          g.row / g.sdd * (g.sid + half) / g.dz <= 2.0;
