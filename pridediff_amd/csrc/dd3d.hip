@@ -1622,9 +1622,11 @@ constexpr int row_waves3() {  // per SIMD: what the LDS block allows
 // prologue, helical 512 x 512 x 64 x 1152 views x 4 56.1 -> 40.3 ms; a
 // 96 x 81 x 50 volume x 100 views 0.51 -> 0.11 ms with its views split.
 //
-// Workgroup z takes instance tile z / nsplit and the views' part z % nsplit
-// (nsplit > 1: partial volumes, added by k_sum_volumes).
-template <int BT, int WM>
+// The views are added in nsplit parts.  Workgroup z takes instance tile
+// z / nsplit and part z % nsplit (nsplit > 1: partial volumes, added by
+// k_sum_volumes); SERIAL: instance tile z and the parts one after the other,
+// added to the output in the same order.
+template <int BT, int WM, bool SERIAL>
 __global__ __launch_bounds__(kThreads3)
 __attribute__((amdgpu_waves_per_eu(row_waves3<BT>()))) void k_voxel_rows(
     Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
@@ -1640,82 +1642,90 @@ __attribute__((amdgpu_waves_per_eu(row_waves3<BT>()))) void k_voxel_rows(
   int ty = static_cast<int>(threadIdx.x) / kTile3;
   const int tc = (tile % ntx) * kTile3, tr = (tile / ntx) * kTile3;
   const int s0 = blockIdx.y * S;
-  const int b0 = (blockIdx.z / nsplit) * BT, part = blockIdx.z % nsplit;
-  const int v0 = static_cast<int>(1LL * g.V * part / nsplit);
-  const int v1 = static_cast<int>(1LL * g.V * (part + 1) / nsplit);
+  const int b0 = (SERIAL ? blockIdx.z : blockIdx.z / nsplit) * BT;
+  int part = SERIAL ? 0 : blockIdx.z % nsplit;
   float acc[S][BT];
-#pragma unroll
-  for (int j = 0; j < S; ++j)
-#pragma unroll
-    for (int b = 0; b < BT; ++b) acc[j][b] = 0.0f;
   // world z extent of this thread's slices (block-uniform)
   const float z0w = -g.Dz * 0.5f * g.dz + (g.scan == DD_SPIRAL ? 0.0f : g.shz);
   const float zc_lo = z0w + s0 * g.dz, zc_hi = z0w + min(s0 + S, g.Dz) * g.dz;
-  for (int v = v0; v < v1; ++v) {
-    const ViewGeo3 vg = views[v];
-    if (zc_hi < vg.zlo || zc_lo > vg.zhi) continue;  // the view's cone misses the chunk
-    const RowRange vr = ranges[static_cast<size_t>(v) * tiles + tile];
-    float first, count;
-    vr.block(static_cast<float>(s0), static_cast<float>(s0 + S), static_cast<float>(vg.row0),
-             &first, &count);
-    // past the detector, or too large
-    if (first + count < 0.0f || first > static_cast<float>(g.R) || vr.ke == vr.kb) continue;
-    const int srb = __builtin_amdgcn_readfirstlane(static_cast<int>(first));
-    const int nrow = __builtin_amdgcn_readfirstlane(static_cast<int>(count));
-    const int skb = vr.kb, ncols = vr.ke - vr.kb;
-    // what follows from the lane alone is cheaper formed again than kept in
-    // registers over the views
-    asm volatile("" : "+v"(tx), "+v"(ty));
-    __syncthreads();  // the previous view's walks are done with the block
-    {
-      const char* __restrict__ sv = reinterpret_cast<const char*>(
-          sino + static_cast<size_t>(v) * g.R * g.C * g.Bp + b0);
-      // 16 columns x 16 rows of threads per step
-      for (int c = tx; c < ncols; c += kTile3)
-        for (int r = ty; r < nrow; r += kTile3) {
-          const int rr = srb + r;
-          float x[BT];
+  do {
+    const int v0 = static_cast<int>(1LL * g.V * part / nsplit);
+    const int v1 = static_cast<int>(1LL * g.V * (part + 1) / nsplit);
 #pragma unroll
-          for (int b = 0; b < BT; ++b) x[b] = 0.0f;
-          if (static_cast<unsigned>(rr) < static_cast<unsigned>(g.R))
-            load_tile<BT>(reinterpret_cast<const float*>(
-                              sv + 4u * static_cast<unsigned>((rr * g.C + skb + c) * g.Bp)),
-                          x);
-          store_tile<BT>(lds.q + (r * kRowPitch + c) * BT, x);
-        }
-      const int t = static_cast<int>(threadIdx.x);
-      if (t <= ncols) lds.edge[t] = cedge[static_cast<size_t>(v) * (g.C + 1) + skb + t];
-      if (t < ncols) lds.colz[t] = colz[static_cast<size_t>(v) * g.C + skb + t];
-      // the tile's lines, dword by dword
-      constexpr int kWords = sizeof(LineGeo3) / 4;
-      const int l0 = vg.xaxis ? tr : tc, nl = min(kTile3, (vg.xaxis ? g.H : g.W) - l0);
-      if (t < nl * kWords)
-        reinterpret_cast<int*>(lds.line)[t] =
-            reinterpret_cast<const int*>(lines + static_cast<size_t>(v) * g.Lmax + l0)[t];
+    for (int j = 0; j < S; ++j)
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc[j][b] = 0.0f;
+    for (int v = v0; v < v1; ++v) {
+      const ViewGeo3 vg = views[v];
+      if (zc_hi < vg.zlo || zc_lo > vg.zhi) continue;  // the view's cone misses the chunk
+      const RowRange vr = ranges[static_cast<size_t>(v) * tiles + tile];
+      float first, count;
+      vr.block(static_cast<float>(s0), static_cast<float>(s0 + S), static_cast<float>(vg.row0),
+               &first, &count);
+      // past the detector, or too large
+      if (first + count < 0.0f || first > static_cast<float>(g.R) || vr.ke == vr.kb) continue;
+      const int srb = __builtin_amdgcn_readfirstlane(static_cast<int>(first));
+      const int nrow = __builtin_amdgcn_readfirstlane(static_cast<int>(count));
+      const int skb = vr.kb, ncols = vr.ke - vr.kb;
+      // what follows from the lane alone is cheaper formed again than kept in
+      // registers over the views
+      asm volatile("" : "+v"(tx), "+v"(ty));
+      __syncthreads();  // the previous view's walks are done with the block
+      {
+        const char* __restrict__ sv = reinterpret_cast<const char*>(
+            sino + static_cast<size_t>(v) * g.R * g.C * g.Bp + b0);
+        // 16 columns x 16 rows of threads per step
+        for (int c = tx; c < ncols; c += kTile3)
+          for (int r = ty; r < nrow; r += kTile3) {
+            const int rr = srb + r;
+            float x[BT];
+#pragma unroll
+            for (int b = 0; b < BT; ++b) x[b] = 0.0f;
+            if (static_cast<unsigned>(rr) < static_cast<unsigned>(g.R))
+              load_tile<BT>(reinterpret_cast<const float*>(
+                                sv + 4u * static_cast<unsigned>((rr * g.C + skb + c) * g.Bp)),
+                            x);
+            store_tile<BT>(lds.q + (r * kRowPitch + c) * BT, x);
+          }
+        const int t = static_cast<int>(threadIdx.x);
+        if (t <= ncols) lds.edge[t] = cedge[static_cast<size_t>(v) * (g.C + 1) + skb + t];
+        if (t < ncols) lds.colz[t] = colz[static_cast<size_t>(v) * g.C + skb + t];
+        // the tile's lines, dword by dword
+        constexpr int kWords = sizeof(LineGeo3) / 4;
+        const int l0 = vg.xaxis ? tr : tc, nl = min(kTile3, (vg.xaxis ? g.H : g.W) - l0);
+        if (t < nl * kWords)
+          reinterpret_cast<int*>(lds.line)[t] =
+              reinterpret_cast<const int*>(lines + static_cast<size_t>(v) * g.Lmax + l0)[t];
+      }
+      __syncthreads();
+      const int col = tc + tx, row = tr + ty;
+      if (col >= g.W || row >= g.H) continue;
+      gather_rows<BT, WM, S>(
+          g, vg, lds.line[vg.xaxis ? ty : tx], row, col, s0, 0, ncols,
+          [&](int k) { return lds.edge[k]; }, [&](int k) { return lds.colz[k]; },
+          [&](int k, int rbase) {
+            // row rbase + fl + m of column k at byte lb + (fl + m) kStep of the
+            // block, formed in float (below 2^24: exact)
+            constexpr int kStep = kRowPitch * BT * 4;
+            const float lb = static_cast<float>((rbase - srb) * kStep + k * BT * 4);
+            const char* lq = reinterpret_cast<const char*>(lds.q);
+            return [=](float fl, int m, float(&x)[BT]) {
+              const int at = static_cast<int>(fmaf(fl, static_cast<float>(kStep), lb));
+              load_tile<BT>(reinterpret_cast<const float*>(lq + at) + m * (kStep / 4), x);
+            };
+          },
+          srb, srb + nrow, acc, skb);
     }
-    __syncthreads();
     const int col = tc + tx, row = tr + ty;
-    if (col >= g.W || row >= g.H) continue;
-    gather_rows<BT, WM, S>(
-        g, vg, lds.line[vg.xaxis ? ty : tx], row, col, s0, 0, ncols,
-        [&](int k) { return lds.edge[k]; }, [&](int k) { return lds.colz[k]; },
-        [&](int k, int rbase) {
-          // row rbase + fl + m of column k at byte lb + (fl + m) kStep of the
-          // block, formed in float (below 2^24: exact)
-          constexpr int kStep = kRowPitch * BT * 4;
-          const float lb = static_cast<float>((rbase - srb) * kStep + k * BT * 4);
-          const char* lq = reinterpret_cast<const char*>(lds.q);
-          return [=](float fl, int m, float(&x)[BT]) {
-            const int at = static_cast<int>(fmaf(fl, static_cast<float>(kStep), lb));
-            load_tile<BT>(reinterpret_cast<const float*>(lq + at) + m * (kStep / 4), x);
-          };
-        },
-        srb, srb + nrow, acc, skb);
-  }
-  const int col = tc + tx, row = tr + ty;
-  if (col >= g.W || row >= g.H) return;
-  if (nsplit > 1) out += static_cast<size_t>(part) * g.B * g.Dz * g.H * g.W;
-  store_slices<BT, S, false>(g, out, row, col, s0, b0, acc);
+    if (col < g.W && row < g.H) {
+      if (SERIAL && part > 0) {
+        store_slices<BT, S, true>(g, out, row, col, s0, b0, acc);
+      } else {
+        if (!SERIAL && nsplit > 1) out += static_cast<size_t>(part) * g.B * g.Dz * g.H * g.W;
+        store_slices<BT, S, false>(g, out, row, col, s0, b0, acc);
+      }
+    }
+  } while (SERIAL && ++part < nsplit);
 }
 
 // The same from global memory: all views (ranges null), or, added to the
@@ -1806,7 +1816,14 @@ struct Layout3 {
   size_t buf0, buf1, ranges, parts, data_total;
   bool rows;    // sinogram -> volume by detector rows (k_voxel_rows)
   int nsplit;   // its view parts
+  bool split;   // each part by its own workgroups, to partial volumes
 };
+
+// Largest partial volumes that the views are split for: what the Infinity
+// Cache can hand to their sum.  One volume's parts are at most 2048 x 4096
+// voxels (view_split3), 34 MB, so a batch with more fills the chip without the
+// split; its workgroups take the parts one after the other (same bits).
+constexpr size_t kPartBytes3 = size_t{256} << 20;
 
 // Whether the sinogram -> volume ops add detector rows directly: where a
 // slice meets at most 4 rows (is at most 3 rows thick at the volume's corner
@@ -1872,8 +1889,9 @@ Layout3 make_layout3(const Geo3& g, int op) {
     L.ranges = take(sizeof(RowRange) * g.V * ((g.W + kTile3 - 1) / kTile3) *
                     ((g.H + kTile3 - 1) / kTile3));
     L.nsplit = view_split3(g);
-    if (L.nsplit > 1)
-      L.parts = take(sizeof(float) * L.nsplit * static_cast<size_t>(g.B) * g.Dz * g.H * g.W);
+    const size_t parts = sizeof(float) * L.nsplit * static_cast<size_t>(g.B) * g.Dz * g.H * g.W;
+    L.split = L.nsplit > 1 && parts <= kPartBytes3;
+    if (L.split) L.parts = take(parts);
   } else {
     const size_t q = sizeof(float) * static_cast<size_t>(g.V) * (g.R + 2) * g.C * g.Bp;
     L.buf0 = take(q);
@@ -1999,11 +2017,17 @@ void launch_rows3(const Geo3& g, int op, const float* input, float* output,
     hipLaunchKernelGGL((k_row_ranges<BT>),
                        dim3(static_cast<unsigned>((n + kThreads3 - 1) / kThreads3)),
                        dim3(kThreads3), 0, st, g, views, cedge, colz, lines, ranges, misfits);
-    auto* dst = L.nsplit > 1 ? reinterpret_cast<float*>(ws + L.parts) : output;
-    hipLaunchKernelGGL((k_voxel_rows<BT, WM>), dim3(ntx * nty, chunks, g.Bp / BT * L.nsplit),
+    auto* dst = L.split ? reinterpret_cast<float*>(ws + L.parts) : output;
+    auto kernel = k_voxel_rows<BT, WM, false>;
+    bool serial = false;
+    if constexpr (BT == 4) {  // below, the parts of a batch fit kPartBytes3
+      serial = L.nsplit > 1 && !L.split;
+      if (serial) kernel = k_voxel_rows<BT, WM, true>;
+    }
+    hipLaunchKernelGGL(kernel, dim3(ntx * nty, chunks, g.Bp / BT * (serial ? 1 : L.nsplit)),
                        dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, dst, ranges,
                        L.nsplit);
-    if (L.nsplit > 1) {
+    if (L.split) {
       const size_t m = static_cast<size_t>(g.B) * g.Dz * g.H * g.W;
       hipLaunchKernelGGL(k_sum_volumes,
                          dim3(static_cast<unsigned>((m + kThreads3 - 1) / kThreads3)),

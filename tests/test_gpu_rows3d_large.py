@@ -47,9 +47,9 @@ def test_lines_of_more_than_two_gib(rt):
 @pytest.mark.parametrize("batch", [1, 2])
 def test_slices_of_more_than_eight_mib_a_line(rt, batch):
     """2.2 million pixels on a line: relative L2 against 64 bits <= 5e-6 (sums
-    of a few hundred pixels in FP32)."""
-    w, n, rows, cols = 2_200_000 // batch, 4, 5, 4000
-    g = O.Geom3D(w, 1, n, cols, rows, 1e-4, 1e-4, 1.0, 0.1 / batch, 2.0, 500.0, 1000.0)
+    of 2500 pixels in FP32)."""
+    w, n, rows, cols = 2_200_000 // batch, 2, 5, 40
+    g = O.Geom3D(w, 1, n, cols, rows, 1e-4, 1e-4, 1.0, 0.5, 1.0, 500.0, 1000.0)
     ang = np.array([0.0], dtype=np.float32)
     x = np.random.default_rng(2).random((batch, n, 1, w), dtype=np.float32)
     got = rt.ProjConeFlatDis3d(torch.from_numpy(x)[:, None].cuda(), torch.tensor(g.options()),
