@@ -17,7 +17,8 @@
 //   k_bins3d             image -> sinogram: one thread per detector column and
 //                        chunk of rows, gathering row by row over the lines
 //                        its ray band meets in z (k_bins3d_slices: slice by
-//                        slice, rows thicker than two slices);
+//                        slice, where that is the faster: few, thick or thin
+//                        rows, coarse columns);
 //   k_interleave_sino3d  sinogram -> [view][row][col][b] (x FP weight);
 //   k_row_ranges         per view and pixel tile: the columns to be staged;
 //   k_voxel_rows         sinogram -> image: one thread per pixel and chunk of
@@ -819,8 +820,8 @@ __attribute__((amdgpu_waves_per_eu(line_waves3<BT, S>()))) void k_bins3d(
   }
 }
 
-// The same for rows thicker than two slices, slice by slice: per
-// line the column's x footprint and the z law are evaluated once and shared
+// The same slice by slice, where the rows' form does not hold or is the slower
+// (use_line_rows3): per line the column's x footprint and the z law are evaluated once and shared
 // by the S rows; the slices the chunk reaches are then visited once each,
 // every slice's voxels loaded once and spread over the S rows by their z
 // overlaps (slice-major: a row-by-row walk reloads each slice for every
@@ -2054,16 +2055,41 @@ bool use_cols_first(const Geo3& g, int bt) {
   return tile_bytes > 192.0 * (1 << 20);
 }
 
-// Whether the volume -> sinogram ops go row by row: rows at most two slices
-// thick at the volume's far corner, and lines whose slices line_rows can
-// address (24-bit factors, one line's slices within 2 GiB).  Others go slice
-// by slice.
+// Whether the volume -> sinogram ops go row by row (line_rows) or slice by
+// slice.  By rows only what it holds: rows at most two slices thick at the
+// volume's far corner, lines whose slices its offsets address (24-bit factors,
+// one line's slices within 2 GiB).  And only where it is the faster (ms by
+// rows / by slices, 120 views):
+//  * enough rows: a chunk of 8 or 16 is walked whole.  128 x 128 x 64 volume,
+//    180 columns: one instance 1 row 0.29 / 0.13, 4 0.30 / 0.25, 6 0.30 / 0.32,
+//    8 0.30 / 0.39; two 1 row 0.17 / 0.16, 4 0.17 / 0.34; four 1 row 0.24 / 0.15,
+//    3 0.24 / 0.25, 6 0.25 / 0.32.  256 x 256, as many slices as rows: one
+//    instance 6 rows 0.57 / 0.56; four 3 rows 0.45 / 0.40, 4 0.46 / 0.51;
+//    400 x 400 x 300 views, two instances: 2 rows 0.80 / 0.56, 3 0.80 / 0.76,
+//    4 0.81 / 0.98.
+//  * columns that mostly meet three pixels of a line at most; past that a
+//    row's pixels are taken in pairs, each with the row's whole walk.  128 x
+//    128 x 64, 80 rows, 90 views, 1, 2 and 4 instances: 1.33 pixels a column
+//    0.74 / 0.56, 0.89 / 0.75, 1.12 / 0.57; 1.25 0.50 / 0.55, 0.51 / 0.75,
+//    0.67 / 0.57; 1.18 0.45 / 0.56, 0.31 / 0.76, 0.45 / 0.57; 2 1.02 / 0.67,
+//    1.28 / 1.08, 1.66 / 0.75.
+//  * rows not much thinner than a slice, which by slices is loaded once for
+//    all the chunk's rows.  96 x 96 x 24, 100 views and 192 x 192 x 48, 200
+//    views: one instance 1/4 slice a row 0.18 / 0.21 and 1.49 / 1.54, 1/8 0.28 /
+//    0.25 and 2.53 / 2.34; two 1/4 0.22 / 0.25 and 2.04 / 1.94, 1/8 0.36 / 0.28
+//    and 3.70 / 2.74; four 1/3 0.25 / 0.26, 1/4 0.29 / 0.26 and 3.06 / 2.79.
 bool use_line_rows3(const Geo3& g) {
   const long long slice = 4LL * std::max(g.W, g.H) * g.BT;  // bytes of one line's slice
   if (g.Dz >= 1 << 22 || slice >= 1LL << 23 || slice * (g.Dz + 1) >= 1LL << 31) return false;
+  if (g.R < (g.BT == 1 ? 7 : g.BT == 2 ? 3 : 4)) return false;
+  if (!(g.row > 0.0f && g.dz > 0.0f && g.sdd > 0.0f)) return false;
+  // column width and row height at the isocentre
+  const double col = g.scan == DD_CONE_FLAT ? g.col / g.sdd * g.sid : g.col * g.sid;
+  const double row = g.row / g.sdd * g.sid / g.dz;
+  if (col > 1.27 * std::min(g.dx, g.dy)) return false;
+  if (row < (g.BT == 1 ? 0.22 : g.BT == 2 ? 0.28 : 0.33)) return false;
   const double half = 0.5 * std::hypot(g.W * g.dx, g.H * g.dy) + std::hypot(g.shx, g.shy);
-  return g.row > 0.0f && g.dz > 0.0f && g.sdd > 0.0f &&
-         g.row / g.sdd * (g.sid + half) / g.dz <= 2.0;
+  return g.row / g.sdd * (g.sid + half) / g.dz <= 2.0;
 }
 
 template <int BT, bool COLS_FIRST>

@@ -27,8 +27,8 @@ def test_rows_of_millions_of_slices(rt, batch):
     takes the upper half of the volume (2.2e7 slices from its middle on), the
     others nothing.  Sums of 8 slices of 16 pixels in FP32: relative L2 <= 5e-6."""
     sid, sdd, step = 100.0, 16.0 - 2.0 ** -10, 2.0 ** -20  # step: one ulp below 16
-    g = O.Geom3D(16, 16, 16, 4, 6, 1.0, 1.0, 1.0, 0.02 * step / sdd, 0.25, sid, sdd, 0.0, 0.0,
-                 0.0, 0.0, 0.75)
+    g = O.Geom3D(16, 16, 16, 4, 8, 1.0, 1.0, 1.0, 0.02 * step / sdd, 0.25, sid, sdd, 0.0, 0.0,
+                 0.0, 0.0, 1.0)
     ang = np.array([0.0, 1.5, 2.9], dtype=np.float32)
     spos = np.zeros((4, 3), dtype=np.float32)
     spos[1] = step - sdd
