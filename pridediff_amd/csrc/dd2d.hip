@@ -674,7 +674,7 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone, int walk = kWa
   L.wfp = take(sizeof(float) * g.V * g.D);
   L.lines = take(sizeof(LineGeo) * g.V * g.Lmax);
   L.pint = take(sizeof(float) * g.V * g.Lmax);
-  L.has_ranges = walk != kWalkNoTables;
+  L.has_ranges = walk != kWalkNoTables && walk_stages(g);
   if (L.has_ranges) L.wranges = take(sizeof(unsigned) * g.V * walk_range_tiles(g));
   L.geo_total = off;
   off = 0;
@@ -690,7 +690,8 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone, int walk = kWa
     L.buf0 = take(sizeof(float) * static_cast<size_t>(g.V) * g.D * g.Bp);
     L.buf1 = L.buf0;
     const size_t part = sizeof(float) * static_cast<size_t>(walk_chunks(g.V)) * g.B * g.H * g.W;
-    L.split = walk == kWalkFull && walk_chunks(g.V) > 1 && part <= kWalkPartBytes;
+    L.split = walk == kWalkFull && walk_rows(g) > 0 && walk_chunks(g.V) > 1 &&
+              part <= kWalkPartBytes;
     if (L.split) L.wpart = take(part);
     if (prefix & kPrefAdjoint) {
       L.psino = take(16 * static_cast<size_t>(g.B) * g.V * (g.D + 1));
@@ -704,7 +705,8 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone, int walk = kWa
 
 // Walk memory of a one-call op: none where the staged walk does not run.
 int run_walk_mem(const Geo2& g, int op, int variant) {
-  return to_sino(op) || prefix_path(g, op, variant) ? kWalkNoTables : kWalkFull;
+  return to_sino(op) || prefix_path(g, op, variant) || walk_rows(g) == 0 ? kWalkNoTables
+                                                                         : kWalkFull;
 }
 
 // Planned workspaces hold the running-sum buffers whenever they can be used

@@ -1006,6 +1006,13 @@ inline int walk_rows(const Geo2& g) {
   return 0;
 }
 
+// Whether the walk takes the geometry at some instance tile (a plan's tables
+// serve them all; the tiles of 8 and more stage the lower pixel tiles).
+inline bool walk_stages(Geo2 g) {
+  g.BT = 8;
+  return walk_rows(g) > 0;
+}
+
 template <int BT>
 struct WalkLds {
   double e[kWalkSlots];                    // bin edges from the tile's first on
