@@ -143,9 +143,10 @@ size_t dd2d_geometry_size(int scan, const dd_geom2d* g, int views);
 dd_status dd2d_geometry(int scan, const dd_geom2d* g, const float* angles,
                         int views, void* geo, size_t geo_bytes, void* stream);
 /* Kernel variants of the sinogram -> image gathers.  The first five name the
- * walk over each pixel's bins; they are one kernel (a wavefront stages each
- * view's bins for its pixel tile in LDS; one thread per pixel where the bins
- * are too fine for that) and give equal results, in every batch size. */
+ * walk over each pixel's bins; they are one choice (a wavefront stages each
+ * view's bins for its pixel tile in LDS; one thread per pixel or per 2 x 2
+ * pixels where the bins are too fine for that) and give equal results, in
+ * every batch size. */
 #define DD_ADJ_PER_PIXEL 0
 #define DD_ADJ_TILE16 1
 #define DD_ADJ_TILE8 2
@@ -205,9 +206,10 @@ typedef struct {
  *   fwd_waves : image -> sinogram: 63-bin wavefronts per workgroup (1, 2, 4);
  *   fwd_views : image -> sinogram: views per workgroup, one after the other
  *               (1 - 8); the lines are one of the 8 per-XCD line chunks;
- *   pix_width : per-pixel sinogram -> image gather (bins too fine for the
- *               staged walk): pixels per workgroup row (16, 32 or 64; 256
- *               threads, so 16, 8 or 4 rows).
+ *   pix_width : sinogram -> image gather of bins too fine for the staged
+ *               walk: one pixel a thread, workgroups of 16, 32 or 64 pixels
+ *               a row (256 threads, so 16, 8 or 4 rows); built-in: 16, and 2 x
+ *               2 pixels a thread for large images.
  * The shape never changes a result bit; it is what the autotuner sweeps. */
 typedef struct {
   int fwd_waves;

@@ -290,6 +290,19 @@ __global__ __launch_bounds__(kThreads) void k_pixels(
   pixels_body<BT, WM>(g, views, edges, lines, pint, sino, out, r, c, blockIdx.z * BT, ep);
 }
 
+// The same, one thread per 2 x 2 pixels (32 x 32 a workgroup): large images
+// (use_quads).
+template <int BT, int WM>
+__global__ __launch_bounds__(kThreads) void k_pixels_quad(
+    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
+    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
+    const float* __restrict__ sino, float* __restrict__ out, Epi ep) {
+  const int c0 = blockIdx.x * (2 * kTile) + 2 * (threadIdx.x % kTile);
+  const int r0 = blockIdx.y * (2 * kTile) + 2 * (threadIdx.x / kTile);
+  if (c0 >= g.W || r0 >= g.H) return;
+  quads_body<BT, WM>(g, views, edges, lines, pint, sino, out, r0, c0, blockIdx.z * BT, ep);
+}
+
 // sinogram -> image by the staged walk: one wavefront per pixel tile.  SPLIT:
 // workgroup row y takes view chunk y and writes its partial image to out
 // (k_sum_chunks adds them); otherwise a wavefront takes the chunks one after
@@ -799,10 +812,32 @@ void launch_walk(const Geo2& g, const GeoPtrs& G, const float* buf0, float* outp
   }
 }
 
-// Per-pixel gather, workgroups of TW x 256 / TW pixels.
+// Whether the gather of fine bins takes 2 x 2 pixels a thread: one search and
+// one load of each bin for two pixels of a line.  From 1024 workgroups on (four
+// a compute unit) and for one or two instances.  90 views, two bins a pixel, us
+// by quads / per pixel: 1024 x 1024 one instance 393 / 438, two 423 / 467;
+// 2048 x 2048 1324 / 1540 and 1409 / 1684; 3000 x 3000 2827 / 3550 and 3046 /
+// 3780; below 1024 workgroups, and with four instances (registers), per pixel
+// is as fast or faster (900 x 900 344 us, quads 369).
+bool use_quads(const Geo2& g) {
+  return g.BT <= 2 && 1LL * ((g.W + 31) / 32) * ((g.H + 31) / 32) * (g.Bp / g.BT) >= 1024;
+}
+
+// Gather of fine bins: 2 x 2 pixels a thread, or one, in workgroups of
+// TW x 256 / TW pixels (a width given chooses the latter).
 template <int BT, int WM>
 void launch_pixels(const Geo2& g, const GeoPtrs& G, const float* buf0, float* output,
                    hipStream_t st, const Epi& ep, int width) {
+  if constexpr (BT <= 2) {
+    if (width == 0 && use_quads(g)) {
+      hipLaunchKernelGGL((k_pixels_quad<BT, WM>),
+                         dim3((g.W + 2 * kTile - 1) / (2 * kTile),
+                              (g.H + 2 * kTile - 1) / (2 * kTile), g.Bp / BT),
+                         dim3(kThreads), 0, st, g, G.views, G.edges, G.lines, G.pint, buf0, output,
+                         ep);
+      return;
+    }
+  }
   const int tw = width > 0 ? width : pix_tile_w<BT>();
   const int th = kThreads / tw;
   const dim3 grid((g.W + tw - 1) / tw, (g.H + th - 1) / th, g.Bp / BT);

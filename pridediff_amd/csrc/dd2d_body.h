@@ -948,6 +948,133 @@ __device__ __forceinline__ void pixels_body(
     }
 }
 
+// Adds view v to the two consecutive pixels i0, i0 + 1 of one line (i0 + 1 only
+// when has1): one first-bin search, for i0, and one walk over the bins that
+// reach either pixel, each loaded once.  A pixel's bins are those whose upper
+// edge does not lie before it nor the lower past it, in its own frame: the set
+// and order that pixel_one_view walks, so each sum is the same bit for bit.
+template <int BT>
+__device__ __forceinline__ void pixel_pair_view(
+    const Geo2& g, const ViewGeo& vg, const double* __restrict__ ev, const LineGeo& lg, float pl,
+    const float* __restrict__ sv, int i0, bool has1, float gw0, float gw1, float (&acc0)[BT],
+    float (&acc1)[BT]) {
+  const PixelFrame f0(lg.a0, lg.inv_p, i0), f1(lg.a0, lg.inv_p, i0 + 1);
+  int k = min(max(guess_bin_fast(g, vg, lg.a0 + (i0 + 0.5) * static_cast<double>(pl)), 0),
+              g.D - 1);
+  double e1 = ev[k];
+  while (k > 0 && f0.at(e1) >= 0.0) e1 = ev[--k];
+  double e2 = ev[k + 1];
+  while (f0.at(e2) < 0.0) {
+    if (++k >= g.D) return;
+    e1 = e2;
+    e2 = ev[k + 1];
+  }
+  double u0 = f0.at(e1), u1 = f1.at(e1);
+  while ((has1 ? u1 : u0) < 1.0) {
+    const double v0 = f0.at(e2), v1 = f1.at(e2);
+    float q[BT];
+    load_sino<BT>(g, sv, k, q);
+    if (u0 < 1.0) {
+      const float w = (pixel_fraction(v0) - pixel_fraction(u0)) * gw0;
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc0[b] = fmaf(w, q[b], acc0[b]);
+    }
+    if (has1 && v1 >= 0.0) {
+      const float w = (pixel_fraction(v1) - pixel_fraction(u1)) * gw1;
+#pragma unroll
+      for (int b = 0; b < BT; ++b) acc1[b] = fmaf(w, q[b], acc1[b]);
+    }
+    if (++k >= g.D) break;
+    u0 = v0;
+    u1 = v1;
+    if ((has1 ? u1 : u0) >= 1.0) break;
+    e2 = ev[k + 1];
+  }
+}
+
+// sinogram -> image for the 2 x 2 pixels at (r0, c0), all views: per view two
+// lines of two consecutive pixels, image rows r0, r0 + 1 or columns c0, c0 + 1
+// (read bottom-up).  Equal bit for bit to pixels_body on each pixel.
+template <int BT, int WM>
+__device__ __forceinline__ void quads_body(
+    const Geo2& g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
+    const LineGeo* __restrict__ lines, const float* __restrict__ pint,
+    const float* __restrict__ sino, float* __restrict__ out, int r0, int c0, int b0,
+    const Epi& ep = Epi{}) {
+  const bool hr = r0 + 1 < g.H, hc = c0 + 1 < g.W;
+  float xc[2][2] = {}, yc[2][2] = {};  // [row][column]
+  if constexpr (WM == W_BPW) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) pixel_centre(g, 1, r0 + r, c0 + c, &xc[r][c], &yc[r][c]);
+  }
+  float acc[2][2][BT], sum[2][2][BT];
+  const int nc = walk_chunks(g.V);
+  for (int ch = 0, v = 0; ch < nc; ++ch) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int b = 0; b < BT; ++b) acc[r][c][b] = 0.0f;
+    for (const int v1 = walk_chunk_begin(g.V, ch + 1); v < v1; ++v) {
+      const ViewGeo vg = const_load(views + v);
+      const double* __restrict__ ev = edges + static_cast<size_t>(v) * (g.D + 1);
+      const LineGeo* __restrict__ lv = lines + static_cast<size_t>(v) * g.Lmax;
+      const float* __restrict__ pv = pint + static_cast<size_t>(v) * g.Lmax;
+      const float* __restrict__ sv = sino_view<BT>(g, sino, v, b0);
+      const float kbp = bp_const(g);
+      auto weight = [&](float pl, int r, int c) {
+        float w = (WM == W_FP) ? pl : kbp;
+        if constexpr (WM == W_BPW) w *= fbp_weight(g, vg, xc[r][c], yc[r][c]);
+        return w;
+      };
+      if (vg.xaxis) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          if (r == 1 && !hr) break;
+          const float pl = pv[r0 + r];
+          pixel_pair_view<BT>(g, vg, ev, lv[r0 + r], pl, sv, c0, hc, weight(pl, r, 0),
+                              weight(pl, r, 1), acc[r][0], acc[r][1]);
+        }
+      } else {
+        // pixel H - 1 - r: the pair is rows r0 + 1, r0, or the last row alone
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          if (c == 1 && !hc) break;
+          const float pl = pv[c0 + c];
+          const LineGeo lg = lv[c0 + c];
+          if (hr)
+            pixel_pair_view<BT>(g, vg, ev, lg, pl, sv, g.H - 2 - r0, true, weight(pl, 1, c),
+                                weight(pl, 0, c), acc[1][c], acc[0][c]);
+          else
+            pixel_pair_view<BT>(g, vg, ev, lg, pl, sv, g.H - 1 - r0, false, weight(pl, 0, c), 0.0f,
+                                acc[0][c], acc[1][c]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int b = 0; b < BT; ++b)
+          sum[r][c][b] = ch == 0 ? acc[r][c][b] : sum[r][c][b] + acc[r][c][b];
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      if ((r == 0 || hr) && (c == 0 || hc))
+#pragma unroll
+        for (int b = 0; b < BT; ++b)
+          if (b0 + b < g.B) {
+            const size_t at = (static_cast<size_t>(b0 + b) * g.H + r0 + r) * g.W + c0 + c;
+            out[at] = epi_value(ep, sum[r][c][b], at);
+          }
+}
+
 // ---------------------------------------------------------------------------
 // 3c. sinogram -> image: the staged walk, one wavefront per pixel tile
 // ---------------------------------------------------------------------------
