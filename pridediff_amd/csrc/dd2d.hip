@@ -124,10 +124,8 @@ bool make_shape(const dd_shape* in, Shape* out) {
 // one-call kernels: thin grids over the shared bodies
 // ---------------------------------------------------------------------------
 // ranges: the staged walk's edge range of every 16 x 8 pixels of the view,
-// ranges[v * tiles + t] (null: not needed), from the tables that the workgroup
-// has just written.  A launch of its own with a thread per range took 5 us at
-// 256 x 256 x 180 views and 18 us at 512 x 512 x 720, of which the loop here
-// saves 3 us of the step and none.
+// ranges[v * tiles + t] (null: not needed here), from the tables that the
+// workgroup has just written.
 __global__ __launch_bounds__(kThreads) void k_setup2d(
     Geo2 g, const float* __restrict__ angles, ViewGeo* __restrict__ views,
     double* __restrict__ edges, float* __restrict__ wfp,
@@ -137,7 +135,20 @@ __global__ __launch_bounds__(kThreads) void k_setup2d(
   if (!ranges) return;
   __syncthreads();
   walk_ranges_view(g, views[v], edges + static_cast<size_t>(v) * (g.D + 1),
+                   lines + static_cast<size_t>(v) * g.Lmax, threadIdx.x, blockDim.x,
+                   ranges + static_cast<size_t>(v) * walk_range_tiles(g));
+}
+
+// The range table by a launch of its own, a thread per entry: grid (entries of
+// a view / 256, views).
+__global__ __launch_bounds__(kThreads) void k_walk_ranges(
+    Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
+    const LineGeo* __restrict__ lines, unsigned* __restrict__ ranges) {
+  const int v = blockIdx.y;
+  walk_ranges_view(g, views[v], edges + static_cast<size_t>(v) * (g.D + 1),
                    lines + static_cast<size_t>(v) * g.Lmax,
+                   static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x),
+                   static_cast<int>(gridDim.x * blockDim.x),
                    ranges + static_cast<size_t>(v) * walk_range_tiles(g));
 }
 
@@ -274,7 +285,7 @@ __global__ __launch_bounds__(kThreads) void k_bins_reduce(
 
 // sinogram -> image: one thread per pixel, BT instances, all views; every
 // pixel finds its bins on its own.  For detectors so fine that the staged
-// walk's tiles overflow their slots (walk_rows).
+// walk's tiles overflow their slots (walk_rows), and for few views (few_views).
 template <int BT, int WM, int TW>
 __global__ __launch_bounds__(kThreads) void k_pixels(
     Geo2 g, const ViewGeo* __restrict__ views, const double* __restrict__ edges,
@@ -664,6 +675,24 @@ bool to_sino(int op) {
 // (16 bytes each), knot ranges [V][tiles] and partial images
 // [chunks][B][H][W]; or the running-sum forward's line tables, rows
 // [B][H][W+1] and columns [B][W][H+1] of 16-byte entries.
+// Whether an op with few views takes the gather of one or 2 x 2 pixels a thread
+// instead of the staged walk (same bits).  Below 16 views the walk has one
+// chunk, so a small image is a few wavefronts, and a call that forms its own
+// tables pays for the range table; a tile of 16 instances also pays about 8 us
+// for its long code.  ProjTrans, walk against gather, us (T: plus a table a
+// call): 256 x 256 one instance 8 views 15.3 / 13.8, T 24.5 / 18.9; 512 x 512
+// one 8 views 15.6 / 17.3, T 27.3 / 23.2, four weighted T 31.9 / 24.7; sixteen 4
+// views 33 / 20, 16 views 47 / 42, 32 views 74 / 72, 48 views 99 / 102, of 256 x
+// 256 16 views 28 / 31; 1024 x 1024 one 1 view T 20.0 / 16.9, 4 views T 27 / 28.
+bool few_views(const Geo2& g, int op, bool planned) {
+  const long long px = 1LL * g.W * g.H;
+  if (g.BT == 16 && g.V < 48 && px >= 400 * 400) return true;
+  if (g.V >= 16) return false;
+  if (g.BT == 16) return true;
+  if (!planned) return px < 600 * 600 || px * g.V < 2200000;
+  return g.BT < 8 && px <= (op == DD_BPROJ_W && g.BT > 1 ? 512 * 512 : 300 * 300);
+}
+
 // Memory of the staged walk a layout holds: range table and partial images,
 // the table alone (a wavefront then takes all view chunks), or neither (the
 // per-pixel kernel).  The bits are the same.
@@ -703,8 +732,8 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone, int walk = kWa
     L.buf0 = take(sizeof(float) * static_cast<size_t>(g.V) * g.D * g.Bp);
     L.buf1 = L.buf0;
     const size_t part = sizeof(float) * static_cast<size_t>(walk_chunks(g.V)) * g.B * g.H * g.W;
-    L.split = walk == kWalkFull && walk_rows(g) > 0 && walk_chunks(g.V) > 1 &&
-              part <= kWalkPartBytes;
+    L.split = walk == kWalkFull && walk_rows(g) > 0 && !few_views(g, op, true) &&
+              walk_chunks(g.V) > 1 && part <= kWalkPartBytes;
     if (L.split) L.wpart = take(part);
     if (prefix & kPrefAdjoint) {
       L.psino = take(16 * static_cast<size_t>(g.B) * g.V * (g.D + 1));
@@ -718,8 +747,10 @@ Layout make_layout(const Geo2& g, int op, int prefix = kPrefNone, int walk = kWa
 
 // Walk memory of a one-call op: none where the staged walk does not run.
 int run_walk_mem(const Geo2& g, int op, int variant) {
-  return to_sino(op) || prefix_path(g, op, variant) || walk_rows(g) == 0 ? kWalkNoTables
-                                                                         : kWalkFull;
+  return to_sino(op) || prefix_path(g, op, variant) || walk_rows(g) == 0 ||
+                 few_views(g, op, false)
+             ? kWalkNoTables
+             : kWalkFull;
 }
 
 // Planned workspaces hold the running-sum buffers whenever they can be used
@@ -779,14 +810,24 @@ GeoPtrs geo_ptrs(const void* geo, const Layout& L) {
 void launch_setup(const Geo2& g, const float* angles, void* geo,
                   const Layout& L, hipStream_t st, bool ranges) {
   char* b = static_cast<char*>(geo);
-  hipLaunchKernelGGL(k_setup2d, dim3(g.V), dim3(kThreads), 0, st, g, angles,
-                     reinterpret_cast<ViewGeo*>(b + L.views),
-                     reinterpret_cast<double*>(b + L.edges),
-                     reinterpret_cast<float*>(b + L.wfp),
-                     reinterpret_cast<LineGeo*>(b + L.lines),
-                     reinterpret_cast<float*>(b + L.pint),
-                     ranges && L.has_ranges ? reinterpret_cast<unsigned*>(b + L.wranges)
-                                            : nullptr);
+  auto* views = reinterpret_cast<ViewGeo*>(b + L.views);
+  auto* edges = reinterpret_cast<double*>(b + L.edges);
+  auto* lines = reinterpret_cast<LineGeo*>(b + L.lines);
+  auto* table = ranges && L.has_ranges ? reinterpret_cast<unsigned*>(b + L.wranges) : nullptr;
+  const int tiles = walk_range_tiles(g);
+  // By k_setup2d, one launch less (256 x 256 x 180 views 109 -> 104.6 us a step),
+  // unless its one workgroup a view would walk a large image's ranges while the
+  // chip idles: ProjTrans of 1024 x 1024, with and without a launch of its own,
+  // 4 views 27 and 69 us, 64 views 132 and 182, 2048 x 2048 x 180 views 1.18 and
+  // 1.32 ms.  From about 512 views on the ranges fill it either way (512 x 512 x
+  // 720 views: the same time).
+  const bool apart = table && tiles > 4 * kThreads && g.V < 512;
+  hipLaunchKernelGGL(k_setup2d, dim3(g.V), dim3(kThreads), 0, st, g, angles, views, edges,
+                     reinterpret_cast<float*>(b + L.wfp), lines,
+                     reinterpret_cast<float*>(b + L.pint), apart ? nullptr : table);
+  if (apart)
+    hipLaunchKernelGGL(k_walk_ranges, dim3((tiles + kThreads - 1) / kThreads, g.V), dim3(kThreads),
+                       0, st, g, views, edges, lines, table);
 }
 
 // Staged walk of the sinogram -> image ops.
@@ -812,7 +853,7 @@ void launch_walk(const Geo2& g, const GeoPtrs& G, const float* buf0, float* outp
   }
 }
 
-// Whether the gather of fine bins takes 2 x 2 pixels a thread: one search and
+// Whether the gather per pixel takes 2 x 2 pixels a thread: one search and
 // one load of each bin for two pixels of a line.  From 1024 workgroups on (four
 // a compute unit) and for one or two instances.  90 views, two bins a pixel, us
 // by quads / per pixel: 1024 x 1024 one instance 393 / 438, two 423 / 467;
@@ -823,8 +864,8 @@ bool use_quads(const Geo2& g) {
   return g.BT <= 2 && 1LL * ((g.W + 31) / 32) * ((g.H + 31) / 32) * (g.Bp / g.BT) >= 1024;
 }
 
-// Gather of fine bins: 2 x 2 pixels a thread, or one, in workgroups of
-// TW x 256 / TW pixels (a width given chooses the latter).
+// Gather per pixel: 2 x 2 pixels a thread, or one, in workgroups of TW x
+// 256 / TW pixels (a width given chooses the latter).
 template <int BT, int WM>
 void launch_pixels(const Geo2& g, const GeoPtrs& G, const float* buf0, float* output,
                    hipStream_t st, const Epi& ep, int width) {
@@ -941,7 +982,7 @@ dd_status launch_tile(const Geo2& g, int op, int variant, const float* input,
                          0, st, g, G.views, G.wfp, input, buf0);
     ProfileScope prof(DD_KERNEL_SINO_TO_IMAGE, st);
     constexpr int kMost = BT >= 8 ? 2 : 4;
-    const int rows = L.has_ranges ? walk_rows(g) : 0;
+    const int rows = L.has_ranges && !few_views(g, op, true) ? walk_rows(g) : 0;
     auto run = [&](auto wm) {
       constexpr int WM = decltype(wm)::value;
       if (rows == kMost)

@@ -1096,13 +1096,13 @@ __device__ __forceinline__ unsigned pack_range(int2 r) {
          static_cast<unsigned>(n > kWalkSlots || r.x >= (1 << 24) ? 255 : n);
 }
 
-// The range table of one view, by one workgroup.
+// Entries [t0, ...) of one view's range table, every `step`th.
 __device__ __forceinline__ void walk_ranges_view(const Geo2& g, const ViewGeo& vg,
                                                  const double* __restrict__ ev,
-                                                 const LineGeo* __restrict__ lv,
+                                                 const LineGeo* __restrict__ lv, int t0, int step,
                                                  unsigned* __restrict__ out) {
   const int tx = (g.W + kWalkW - 1) / kWalkW, tiles = walk_range_tiles(g);
-  for (int t = threadIdx.x; t < tiles; t += blockDim.x) {
+  for (int t = t0; t < tiles; t += step) {
     const int c0 = (t % tx) * kWalkW, r0 = (t / tx) * kWalkRangeH;
     out[t] = pack_range(
         knot_range(g, vg, ev, lv, r0, min(r0 + kWalkRangeH, g.H), c0, min(c0 + kWalkW, g.W)));

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kThreads) void k_batch_ranges(char* __restrict__ me
     const double* __restrict__ ev = d.edges + static_cast<size_t>(v) * (d.g.D + 1);
     const LineGeo* __restrict__ lv = d.lines + static_cast<size_t>(v) * d.g.Lmax;
     if (d.rows > 0) {
-      walk_ranges_view(d.g, vg, ev, lv,
+      walk_ranges_view(d.g, vg, ev, lv, threadIdx.x, blockDim.x,
                        d.wrange + static_cast<size_t>(v) * walk_range_tiles(d.g));
     } else {
       const int tx = (d.g.W + kQuadTile - 1) / kQuadTile;
