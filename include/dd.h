@@ -228,6 +228,13 @@ dd_status dd2d_run_planned_ep(int scan, int op, const dd_geom2d* g,
                               const dd_shape* shape, const dd_epilogue* ep, void* ws,
                               size_t ws_bytes, void* stream);
 
+/* Whether a planned sinogram -> image op at this instance tile takes the
+ * gather of one or 2 x 2 pixels a thread, the one that dd_shape's pix_width
+ * shapes, rather than the staged walk (1, 0; 0 for other ops and invalid
+ * geometries).  Host only. */
+int dd2d_planned_pixel_gather(int scan, int op, const dd_geom2d* g, int batch,
+                              int views, int tile);
+
 /* Batched projection of many instances of uneven geometry.
  *
  * Each item describes one instance (or `batch` instances sharing a

@@ -5,8 +5,8 @@ run — the instance tile (how many instances share one geometry evaluation,
 1-16), the sinogram -> image kernel variant (the walk or, at tile 1, the
 running sums) and the workgroup tiles of the gathers (forward: 63-bin waves x
 views per workgroup over one per-XCD line chunk; per-pixel adjoint, where the
-bins are too fine for the staged walk: 16x16, 32x8 or 64x4 pixels) of a
-uniform batch; the grid size and kernel variant of an uneven batch —
+bins are too fine for the staged walk or the views few: 16x16, 32x8 or 64x4
+pixels) of a uniform batch; the grid size and kernel variant of an uneven batch —
 times one forward projection plus one adjoint per candidate with HIP events,
 keeps the fastest, and remembers it in a JSON cache keyed by the device and
 the geometry, so later runs skip the sweep.
@@ -29,7 +29,7 @@ CACHE = os.environ.get("PRIDEDIFF_AMD_TUNE_CACHE",
                        os.path.join(os.path.expanduser("~"), ".cache", "pridediff_amd", "autotune.json"))
 
 
-SWEEP_VERSION = 10  # bumped when the set of swept parameters changes
+SWEEP_VERSION = 11  # bumped when the set of swept parameters changes
 
 _LIB_DIGEST = None
 
@@ -98,8 +98,8 @@ def tune_uniform(projector, angles: torch.Tensor, batch: int, tiles=(1, 2, 4, 8,
     """Fastest ``BatchedProjector2d`` for this projector, angle set and batch:
     first the instance tile x adjoint kernel variant, then, for the winner,
     the workgroup tile of each gather — forward (63-bin waves x views per
-    workgroup; its lines are one of the 8 per-XCD chunks) and per-pixel
-    adjoint (pixels per workgroup row).  The walks give the same bits at
+    workgroup; its lines are one of the 8 per-XCD chunks) and, where the
+    adjoint is gathered per pixel, its pixels per workgroup row.  The walks give the same bits at
     every tile; ``running_sums`` also sweeps, at tile 1, the running-sum
     adjoint alone and both directions, which round differently (within 1e-6
     of the walks)."""
@@ -148,7 +148,9 @@ def tune_uniform(projector, angles: torch.Tensor, batch: int, tiles=(1, 2, 4, 8,
             swept[f"tile{best[0]}/var{best[1]}/fwd{wv[0]}x{wv[1]}"] = fwd[wv]
         wv = min(fwd, key=fwd.get)
         pix = {0: fwd[wv]}
-        if best[1] == rt.ADJ_PER_PIXEL:
+        # a width reaches a kernel only where the adjoint is gathered per pixel
+        probe = BatchedProjector2d(projector, angles, batch, tile=best[0], variant=best[1])
+        if best[1] == rt.ADJ_PER_PIXEL and probe.plan.pixel_gather(rt.PROJ_T):
             for pw in PIX_WIDTHS:
                 pix[pw] = timed_shape((wv[0], wv[1], pw))
                 swept[f"tile{best[0]}/var{best[1]}/fwd{wv[0]}x{wv[1]}/pix{pw}"] = pix[pw]

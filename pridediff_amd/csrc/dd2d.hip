@@ -1205,6 +1205,14 @@ size_t dd2d_planned_workspace_size(int scan, int op, const dd_geom2d* g,
   return make_layout(q, op, planned_prefix(q, op)).data_total;
 }
 
+int dd2d_planned_pixel_gather(int scan, int op, const dd_geom2d* g, int batch, int views,
+                              int tile) {
+  Geo2 q;
+  if (check_op(scan, op) != DD_OK || to_sino(op)) return 0;
+  if (!fill_geo(&q, scan, g, batch, views, valid_tile(tile, batch))) return 0;
+  return walk_rows(q) == 0 || few_views(q, op, true);
+}
+
 dd_status dd2d_run_planned(int scan, int op, const dd_geom2d* g,
                            const void* geo, const float* input, float* output,
                            int batch, int views, int tile, int variant, void* ws,

@@ -432,6 +432,12 @@ class Plan2d {
   const dd_shape& shape() const { return shape_; }
   int64_t variant() const { return variant_; }
   int64_t views() const { return views_; }
+  // whether a sinogram -> image op of the plan takes the gather that
+  // pix_width shapes
+  bool pixel_gather(int64_t op) const {
+    return dd2d_planned_pixel_gather(scan_, static_cast<int>(op), &g_, static_cast<int>(batch_),
+                                     static_cast<int>(views_), tile_) != 0;
+  }
 
  private:
   int scan_;
@@ -640,6 +646,7 @@ PYBIND11_MODULE(radontorch, m) {
            pybind11::arg("fwd_waves") = 0, pybind11::arg("fwd_views") = 0,
            pybind11::arg("pix_width") = 0)
       .def("run", &Plan2d::run)
+      .def("pixel_gather", &Plan2d::pixel_gather, pybind11::arg("op"))
       .def("run_ep", &Plan2d::run_ep, pybind11::arg("op"), pybind11::arg("input"),
            pybind11::arg("c") = pybind11::none(), pybind11::arg("scale") = pybind11::none(),
            pybind11::arg("alpha") = 1.0, pybind11::arg("beta") = 0.0)
