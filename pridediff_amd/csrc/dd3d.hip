@@ -1730,24 +1730,27 @@ __attribute__((amdgpu_waves_per_eu(row_waves3<BT>()))) void k_voxel_rows(
 }
 
 // The same from global memory: all views (ranges null), or, added to the
-// result, those whose block does not fit the LDS buffer (nothing to do
-// unless *misfits).
+// result (nsplit > 1: to the partial volumes), those whose block does not fit
+// the LDS buffer (nothing to do unless *misfits).  In the staged kernel's parts,
+// as a small volume's few workgroups would walk all the views: 33 x 33 x 120 x
+// 60 views x 4, most of them too large, 700 -> 252 us.
 template <int BT, int WM>
 __global__ __launch_bounds__(kThreads3) void k_voxel_rows_global(
     Geo3 g, const ViewGeo3* __restrict__ views, const double* __restrict__ cedge,
     const double2* __restrict__ colz, const LineGeo3* __restrict__ lines,
     const float* __restrict__ sino, float* __restrict__ out,
-    const RowRange* __restrict__ ranges, const int* __restrict__ misfits) {
+    const RowRange* __restrict__ ranges, const int* __restrict__ misfits, int nsplit) {
   constexpr int S = row_slices3<BT>();
   if (ranges && *misfits == 0) return;
   const int ntx = (g.W + kTile3 - 1) / kTile3;
   const int tiles = ntx * ((g.H + kTile3 - 1) / kTile3);
   const int chunks = (g.Dz + S - 1) / S;
-  const long long items = 1LL * tiles * chunks * (g.Bp / BT);
+  const long long items = 1LL * tiles * chunks * nsplit * (g.Bp / BT);
   for (long long item = blockIdx.x; item < items; item += gridDim.x) {
     const int tile = static_cast<int>(item % tiles);
     const int s0 = static_cast<int>(item / tiles % chunks) * S;
-    const int b0 = static_cast<int>(item / tiles / chunks) * BT;
+    const int part = static_cast<int>(item / tiles / chunks % nsplit);
+    const int b0 = static_cast<int>(item / tiles / chunks / nsplit) * BT;
     const int col = (tile % ntx) * kTile3 + static_cast<int>(threadIdx.x) % kTile3;
     const int row = (tile / ntx) * kTile3 + static_cast<int>(threadIdx.x) / kTile3;
     if (col >= g.W || row >= g.H) continue;
@@ -1759,7 +1762,9 @@ __global__ __launch_bounds__(kThreads3) void k_voxel_rows_global(
     const float z0w = -g.Dz * 0.5f * g.dz + (g.scan == DD_SPIRAL ? 0.0f : g.shz);
     const float zc_lo = z0w + s0 * g.dz, zc_hi = z0w + min(s0 + S, g.Dz) * g.dz;
     bool any = !ranges;
-    for (int v = 0; v < g.V; ++v) {
+    const int v0 = static_cast<int>(1LL * g.V * part / nsplit);
+    const int v1 = static_cast<int>(1LL * g.V * (part + 1) / nsplit);
+    for (int v = v0; v < v1; ++v) {
       if (ranges) {
         const RowRange& vr = ranges[static_cast<size_t>(v) * tiles + tile];
         if (vr.ke > vr.kb) continue;
@@ -1790,7 +1795,8 @@ __global__ __launch_bounds__(kThreads3) void k_voxel_rows_global(
     }
     if (!any) continue;
     if (ranges)
-      store_slices<BT, S, true>(g, out, row, col, s0, b0, acc);
+      store_slices<BT, S, true>(g, out + static_cast<size_t>(part) * g.B * g.Dz * g.H * g.W, row,
+                                col, s0, b0, acc);
     else
       store_slices<BT, S, false>(g, out, row, col, s0, b0, acc);
   }
@@ -2011,7 +2017,7 @@ void launch_rows3(const Geo3& g, int op, const float* input, float* output,
     if (g_stage3.load() == 0) {
       hipLaunchKernelGGL((k_voxel_rows_global<BT, WM>), dim3(static_cast<unsigned>(items)),
                          dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, output,
-                         static_cast<const RowRange*>(nullptr), misfits);
+                         static_cast<const RowRange*>(nullptr), misfits, 1);
       return;
     }
     const long long n = 1LL * ntx * nty * g.V;
@@ -2028,16 +2034,17 @@ void launch_rows3(const Geo3& g, int op, const float* input, float* output,
     hipLaunchKernelGGL(kernel, dim3(ntx * nty, chunks, g.Bp / BT * (serial ? 1 : L.nsplit)),
                        dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, dst, ranges,
                        L.nsplit);
+    const int parts = L.split ? L.nsplit : 1;
+    hipLaunchKernelGGL((k_voxel_rows_global<BT, WM>),
+                       dim3(static_cast<unsigned>(std::min<long long>(items * parts, 1024))),
+                       dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, dst, ranges,
+                       misfits, parts);
     if (L.split) {
       const size_t m = static_cast<size_t>(g.B) * g.Dz * g.H * g.W;
       hipLaunchKernelGGL(k_sum_volumes,
                          dim3(static_cast<unsigned>((m + kThreads3 - 1) / kThreads3)),
                          dim3(kThreads3), 0, st, dst, m, L.nsplit, output);
     }
-    hipLaunchKernelGGL((k_voxel_rows_global<BT, WM>),
-                       dim3(static_cast<unsigned>(std::min<long long>(items, 1024))),
-                       dim3(kThreads3), 0, st, g, views, cedge, colz, lines, q, output, ranges,
-                       misfits);
   };
   if (op == DD_PROJ_T)
     run(std::integral_constant<int, W3_FP>{});
