@@ -819,9 +819,10 @@ void launch_setup(const Geo2& g, const float* angles, void* geo,
   // unless its one workgroup a view would walk a large image's ranges while the
   // chip idles: ProjTrans of 1024 x 1024, with and without a launch of its own,
   // 4 views 27 and 69 us, 64 views 132 and 182, 2048 x 2048 x 180 views 1.18 and
-  // 1.32 ms.  From about 512 views on the ranges fill it either way (512 x 512 x
-  // 720 views: the same time).
-  const bool apart = table && tiles > 4 * kThreads && g.V < 512;
+  // 1.32 ms.  From about 512 views on the ranges of images up to 1024 x 512 fill
+  // it either way (512 x 512 x 720 views: the same time; 1024 x 1024 x 720 views
+  // 1.14 and 1.16 ms).
+  const bool apart = table && tiles > 4 * kThreads && (g.V < 512 || tiles > 16 * kThreads);
   hipLaunchKernelGGL(k_setup2d, dim3(g.V), dim3(kThreads), 0, st, g, angles, views, edges,
                      reinterpret_cast<float*>(b + L.wfp), lines,
                      reinterpret_cast<float*>(b + L.pint), apart ? nullptr : table);
