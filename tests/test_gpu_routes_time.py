@@ -109,3 +109,24 @@ def test_adjoint3d_of_blocks_beyond_the_buffer(rt):
         t.append(best_us(lambda: rt.ProjTransConeFlatDis3d(y, opt, ang)))
     print(f"four {t[0]:.0f} us, one {t[1]:.0f} us", flush=True)
     assert t[0] <= 2.3 * t[1]
+
+
+def test_setup_of_uneven_batches(rt):
+    """Plans of one instance, 16 views: 2048 x 2048 against 256 x 256, 4 times
+    the time where one workgroup forms a view's ranges, 1.3 where several do."""
+    import time
+    ang = torch.arange(16, device="cuda", dtype=torch.float32) * 0.3
+    t = {}
+    for n in (2048, 256):
+        opt = torch.tensor([n, n, int(1.44 * n), 358.4 / n, 358.4 / n, 358.4 / n / 595.0, 595.0,
+                            1085.6, 0.0, 0.0, 0.0])
+        t[n] = 1e9
+        for _ in range(12):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            plan = rt.PlanBatch2d(rt.SCAN["arc"], [opt], [ang], 0)
+            torch.cuda.synchronize()
+            t[n] = min(t[n], (time.perf_counter() - t0) * 1e6)
+            del plan
+    print(f"2048: {t[2048]:.0f} us, 256: {t[256]:.0f} us", flush=True)
+    assert t[2048] <= 2.5 * t[256]
