@@ -163,9 +163,9 @@ COUNTER_KEYS = {
                "uneven64:k_batch_bins": ["k_batch_bins<0, false>", "k_batch_reduce<0>"],
                "uneven64:k_batch_bins_prefix": ["k_batch_prefix", "k_batch_bins<0, true>",
                                                 "k_batch_reduce<0>"]},
-    "cone_flat": {"cone_flat:k_voxel_rows": ["k_row_ranges<2>", "k_voxel_rows<2, 0>"],
+    "cone_flat": {"cone_flat:k_voxel_rows": ["k_row_ranges<2>", "k_voxel_rows<2, 0, false>"],
                   "cone_flat:k_bins3d": ["k_bins3d<2, 0, 16, false>"]},
-    "helical": {"helical:k_voxel_rows": ["k_row_ranges<4>", "k_voxel_rows<4, 0>"],
+    "helical": {"helical:k_voxel_rows": ["k_row_ranges<4>", "k_voxel_rows<4, 0, false>"],
                 "helical:k_bins3d": ["k_bins3d<4, 0, 8, true>"]},
 }
 
