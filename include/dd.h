@@ -97,8 +97,8 @@ dd_status dd2d_run(int scan, int op, const dd_geom2d* g, const float* input,
  * not hold the partial images or range table that dd2d_workspace_size()
  * includes, the op runs without them (slower, the same bits); a problem that
  * does not fit even so is rejected with DD_TOO_LARGE (a 512x512 fan-arc slice
- * with 720 views and 736 bins needs 27 MB at batch 1).  Results equal dd2d_run's bit for bit.  Every call on
- * one device shares that device's buffer: calls that overlap on one device
+ * with 720 views and 736 bins needs 30 to 33 MB at batch 1).  Results equal
+ * dd2d_run's bit for bit.  Every call on one device shares that device's buffer: calls that overlap on one device
  * (two streams, two host threads) race and must be ordered by the caller. */
 #define DD_NOALLOC_SCRATCH_BYTES (64u << 20)
 dd_status dd2d_run_noalloc(int scan, int op, const dd_geom2d* g, const float* input,
@@ -243,9 +243,8 @@ int dd2d_planned_pixel_gather(int scan, int op, const dd_geom2d* g, int batch,
  * [batch, H, W], sinogram [batch, views, D]).  dd2d_batch_create is host
  * only; dd2d_batch_setup builds every instance's geometry in the device
  * memory it is given (dd2d_batch_device_bytes) and waits for it once;
- * dd2d_batch_run then runs one op for all instances as two launches
- * (layout, gather; plus the chunk reduction for image -> sinogram ops),
- * capturable into a HIP graph.  The result for
+ * dd2d_batch_run then runs one op for all instances as a few launches
+ * (layout, gather, the sum of chunks), capturable into a HIP graph.  The result for
  * each instance equals dd2d_run on that instance bit for bit.  No
  * counterpart in the reference, which launches once per instance and op
  * (deeprecon/cuda/dis2d/FanArcDisCUDA2d.cu:758-1016). */
@@ -267,8 +266,8 @@ size_t dd2d_batch_device_bytes(const dd2d_batch* b);
  * workgroup per work item). */
 void dd2d_batch_set_grid(dd2d_batch* b, int workgroups);
 /* Sinogram -> image kernel of the batch: a walk variant (the default) or
- * DD_ADJ_BLOCK_PREFIX (instances of fine bins), optionally OR-ed with DD_FWD_PREFIX for the image ->
- * sinogram ops. */
+ * DD_ADJ_BLOCK_PREFIX (instances of fine bins), optionally OR-ed with
+ * DD_FWD_PREFIX for the image -> sinogram ops. */
 void dd2d_batch_set_variant(dd2d_batch* b, int variant);
 dd_status dd2d_batch_setup(dd2d_batch* b, void* device_mem, size_t bytes,
                            void* stream);

@@ -44,7 +44,10 @@ typedef struct {
  * whose per-view detector block (rows + 2) * cols * padded batch reaches
  * 2^29 floats are rejected (0 here, DD_BAD_ARG from dd3d_run): the
  * sinogram -> volume gather addresses a view's block with 32-bit offsets.
- * The size depends on dd3d_set_compensated() at the time of the query. */
+ * The size depends on dd3d_set_compensated() at the time of the query.  For
+ * sinogram -> volume ops by rows it holds, besides the sinogram's copy, the
+ * partial volumes of small volumes' split views: up to 16 a volume, 256 MB in
+ * all (a larger batch takes the parts one after the other). */
 size_t dd3d_workspace_size(int scan, int op, const dd_geom3d* g, int batch,
                            int views);
 
@@ -82,15 +85,15 @@ void dd3d_set_compensated(int mode);
  * batches of 1-2 (at batches of 3+ 94 ms unstaged, 105 ms staged, helical
  * 512x512x64 x 4 x 3456 views).  The same values either way; a view whose
  * block exceeds the LDS buffer is read from global memory (with rows: after
- * the others, so such a sum is rounded in another order).  No counterpart in
+ * the others of its part, so such a sum is rounded in another order).  No counterpart in
  * the reference. */
 void dd3d_set_adjoint_staging(int mode);
 /* Dispatch order of the volume -> sinogram gather: 0 views first (two
  * detector-row chunks per workgroup), 1 detector columns first (one chunk),
  * 2 (default) automatic: columns first when one instance tile's volume copy
- * exceeds 192 MB (helical 512x512x64 x 4, 268 MB: forward 75.4 -> 65.7 ms),
- * views first otherwise (cone-flat 256^3 x 2, 134 MB: 17.7 ms views first,
- * 19.5 ms columns first).  The same bits either way.  No
+ * exceeds 192 MB (helical 512x512x64 x 4, 268 MB), views first otherwise
+ * (cone-flat 256^3 x 2, 134 MB); measured slice by slice: 75.4 -> 65.7 ms, and
+ * 17.7 ms views first, 19.5 ms columns first.  The same bits either way.  No
  * counterpart in the reference. */
 void dd3d_set_forward_order(int mode);
 

@@ -16,7 +16,9 @@
 //      k_pixels_walk    sinogram -> image ops: one wavefront per 16-wide pixel
 //                       tile and chunk of views gathers over its views, each
 //                       staged in LDS (no atomics); k_sum_chunks adds the
-//                       chunks in order.
+//                       chunks in order.  k_pixels, k_pixels_quad: a thread per
+//                       pixel or 2 x 2 pixels where bins are too fine to be
+//                       staged or the views few.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -706,8 +706,8 @@ __device__ __forceinline__ void line_rows(const float* __restrict__ px, int sstr
 // Bound by the vector-memory path's latency and return rate; the slice-major
 // form it replaces spread each slice over all the chunk's rows, two thirds of
 // them with weight zero, at twice the VALU instructions (saturated).  Forward
-// of cone-flat 256^3 x 360 views x 512 x 384 x 2 17.7 -> 12.2 ms, helical
-// 512 x 512 x 64 x 1152 views x 4 49.7 -> 43 ms.
+// of cone-flat 256^3 x 360 views x 512 x 384 x 2 17.7 -> 11.2 ms, helical
+// 512 x 512 x 64 x 1152 views x 4 49.7 -> 42.7 ms.
 template <int BT, int WM, int S, bool COLS_FIRST>
 __global__ __launch_bounds__(kFwdThreads)
 __attribute__((amdgpu_waves_per_eu(line_waves3<BT, S>()))) void k_bins3d(
@@ -1619,8 +1619,8 @@ constexpr int row_waves3() {  // per SIMD: what the LDS block allows
 // pair of instances.  It replaces differences of running row sums, which need
 // a serial scan over the rows, three LDS reads of sums and values per slice
 // edge where this reads one or two rows, and 23 instructions.  ProjTrans of
-// cone-flat 256^3 x 360 views x 512 x 384 x 2 16.4 -> 11.0 ms with its
-// prologue, helical 512 x 512 x 64 x 1152 views x 4 56.1 -> 40.3 ms; a
+// cone-flat 256^3 x 360 views x 512 x 384 x 2 16.4 -> 11.4 ms with its
+// prologue (0.44), helical 512 x 512 x 64 x 1152 views x 4 56.1 -> 41.0 ms; a
 // 96 x 81 x 50 volume x 100 views 0.51 -> 0.11 ms with its views split.
 //
 // The views are added in nsplit parts.  Workgroup z takes instance tile
